@@ -402,11 +402,10 @@ RTG_HD V3 render_sample(const SceneView &S, int max_level, const TraceRay &prima
 // by position.w > 1e-6 and attenuation x + y sqrt(d) + z d; RTshd: lights
 // with shadow rays.  RTmtl and RTshd add the environment ambient after the
 // lights (RTfrac adds it first).
-template <class Stack>
-RTG_HD V3 debug_sample(const SceneView &S, int mode, const TraceRay &q, Stack &st, RayCounts &rc, PrimaryOut &po) {
-    rc.primary++;
-    const Hit h = trace_closest(S, q, st);
-    po = PrimaryOut{h.obj, id_prim(S, h), h.t};
+// debug_color is the colour of primary hit h; `blocked(li, lt, matters, hr)`
+// answers the shadow test of light li (RTshd only), as in shade_local.
+template <class Blocked>
+RTG_HD V3 debug_color(const SceneView &S, int mode, const TraceRay &q, const Hit &h, Blocked &&blocked) {
     const float zNear = S.cam.zNear, zFar = S.cam.zFar;
     if (mode == 0x2) {  // MY_MODEL_DEPTHTEST
         const float d = h.t;
@@ -448,23 +447,32 @@ RTG_HD V3 debug_sample(const SceneView &S, int mode, const TraceRay &q, Stack &s
         }
         va = va + mixmul(m.ka, lt.la);
         const LightDots ld = light_dots(hr.N, q.r.d, lt);
-        if (mode == 0x6) {  // MY_MODEL_SHADOWTEST
-            rc.shadow++;
-            if (!ld.matters()) continue;
-            TraceRay sr;
-            sr.r.o = hr.P;
-            sr.r.d = lt.p2l;
-            sr.type = RAY_SHADOW;
-            sr.inside = 0;
-            sr.src = hr.id;
-            sr.self_test = self_testable(S, sr.r, hr.id, lt.dis);
-            if (trace_any(S, sr, lt.dis, st)) continue;
-        }
+        // MY_MODEL_SHADOWTEST
+        if (mode == 0x6 && (blocked(li, lt, ld.matters(), hr) || !ld.matters())) continue;
         if (ld.n_l > 0) vd = vd + mixmul(m.kd, lt.ld) * ld.n_l;
         if (ld.n_h > 0) vs = vs + mixmul(m.ks, lt.ls) * powf(ld.n_h, m.shiness);
     }
     va = va + mixmul(m.ka, S.env);
     return mixmul(vc, vd + va) + vs;
+}
+
+template <class Stack>
+RTG_HD V3 debug_sample(const SceneView &S, int mode, const TraceRay &q, Stack &st, RayCounts &rc, PrimaryOut &po) {
+    rc.primary++;
+    const Hit h = trace_closest(S, q, st);
+    po = PrimaryOut{h.obj, id_prim(S, h), h.t};
+    return debug_color(S, mode, q, h, [&](int, const LightTerm &lt, bool matters, const HitRec &hr) -> bool {
+        rc.shadow++;
+        if (!matters) return false;
+        TraceRay sr;
+        sr.r.o = hr.P;
+        sr.r.d = lt.p2l;
+        sr.type = RAY_SHADOW;
+        sr.inside = 0;
+        sr.src = hr.id;
+        sr.self_test = self_testable(S, sr.r, hr.id, lt.dis);
+        return trace_any(S, sr, lt.dis, st);
+    });
 }
 
 }  // namespace rtg

@@ -98,13 +98,6 @@ int resolve_size(const SceneRes &S, const rtg_params *p, int &W, int &H) {
     return RTG_OK;
 }
 
-__global__ void k_fill_u8(uint8_t *p, size_t n, uint8_t v) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
-}
-__global__ void k_zero_u64(unsigned long long *p, int n) {
-    if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
-}
-
 int DevBuf::alloc(size_t n) {
     release();
     if (n == 0) n = 16;
@@ -222,33 +215,29 @@ void ktime_end(Arena &A, hipStream_t s, int rec, const unsigned *dev_items) {
 // the job's cancel flag (asynchronous jobs), else null.
 static int render_device(SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
                          Arena &A, const Cancel *cancel) {
-    const size_t npix = (size_t)W * H;
     A.ktimes = (p.flags & RTG_FLAG_KERNEL_TIMES) != 0;
     if (A.ktimes && A.kitems_host == nullptr)
         RTG_HIP(hipHostMalloc(reinterpret_cast<void **>(&A.kitems_host), Arena::kItemSlots * sizeof(unsigned),
                               hipHostMallocDefault));
-    k_fill_u8<<<1024, 256, 0, stream>>>(o.rgb, npix * 3, 127);
-    if (o.ids) k_fill_u8<<<1024, 256, 0, stream>>>(reinterpret_cast<uint8_t *>(o.ids), npix * 8, 0xff);
-    k_zero_u64<<<1, 64, 0, stream>>>(o.counts, 4);
-    if (o.retests) k_zero_u64<<<1, 64, 0, stream>>>(o.retests, 1);
     if (!(p.mode == 0 || (p.mode >= RTG_MODE_CHECK && p.mode <= RTG_MODE_REFRACTTEST) || p.mode == RTG_MODE_RAYTRACE))
         return fail(RTG_E_INVALID, "unknown render mode");
     // AUTO: the wavefront engine.  The megakernel is slower on every large or
     // deep frame (its per-thread ray trees diverge); it only wins on small,
     // shallow frames that take well under a millisecond either way.  The
-    // primary-only debug modes (checker, depth, normal, texture, material,
-    // shadow) run in the megakernel: one closest hit per sample, no tree.
+    // primary-only modes (depth, normal, texture, material, shadow) are one
+    // level of the wavefront, unless the megakernel is asked for; the checker,
+    // which traces nothing, runs in the megakernel.
     int engine = p.engine == RTG_ENGINE_AUTO ? RTG_ENGINE_WAVEFRONT : p.engine;
-    if (p.mode >= RTG_MODE_CHECK && p.mode <= RTG_MODE_SHADOWTEST) {
-        if (p.flags & RTG_FLAG_FP64_RETEST) return fail(RTG_E_INVALID, "the FP64 re-test applies to ray-traced modes");
-        engine = RTG_ENGINE_MEGAKERNEL;
-    }
+    if (p.mode >= RTG_MODE_CHECK && p.mode <= RTG_MODE_SHADOWTEST && (p.flags & RTG_FLAG_FP64_RETEST))
+        return fail(RTG_E_INVALID, "the FP64 re-test applies to ray-traced modes");
+    if (p.mode == RTG_MODE_CHECK) engine = RTG_ENGINE_MEGAKERNEL;
     if (engine == RTG_ENGINE_MEGAKERNEL && (p.flags & RTG_FLAG_FP64_RETEST))
         return fail(RTG_E_INVALID, "the FP64 near-tie re-test needs the wavefront engine");
     int st = A.ws.order_before(stream);
     if (st != RTG_OK) return st;
-    st = engine == RTG_ENGINE_WAVEFRONT ? launch_wavefront(S, p, W, H, o, stream, A.ws, A, cancel)
-                                        : launch_megakernel(S, p, W, H, o, stream, A, cancel);
+    st = engine == RTG_ENGINE_WAVEFRONT
+             ? launch_wavefront(S, p, W, H, o, stream, A.ws, A, cancel, init_of(o, W, H))
+             : launch_megakernel(S, p, W, H, o, stream, A, cancel);
     const int st2 = A.ws.mark_done(stream);
     return st != RTG_OK ? st : st2;
 }
@@ -703,9 +692,10 @@ int rtg_render_batch(const rtg_request *reqs, int n, rtg_stats *stats) {
     }
     hipStream_t s = A.stream;
     unsigned long long *counts = A.counters.as<unsigned long long>();
-    k_fill_u8<<<1024, 256, 0, s>>>(A.out_rgb.as<uint8_t>(), rgb_bytes, 127);
-    if (ids_bytes) k_fill_u8<<<1024, 256, 0, s>>>(A.out_ids.as<uint8_t>(), ids_bytes, 0xff);
-    k_zero_u64<<<1, 64, 0, s>>>(counts, 5);
+    int st = launch_init(FrameInit{A.out_rgb.as<uint8_t>(), rgb_bytes, ids_bytes ? A.out_ids.as<int32_t>() : nullptr,
+                                   ids_bytes, counts, counts + 4},
+                         nullptr, 0, s);
+    if (st != RTG_OK) return st;
     RTG_HIP(hipEventRecord(A.ev0, s));
     // One wavefront level holds at most level_ray_cap rays: a request list
     // with more level-0 samples runs as consecutive batches, and a request
@@ -718,12 +708,13 @@ int rtg_render_batch(const rtg_request *reqs, int n, rtg_stats *stats) {
     }
     const size_t cap = level_ray_cap(n_on);
     int replayed = 0;
-    int st = A.ws.order_before(s);
+    st = A.ws.order_before(s);
     for (int b = 0; st == RTG_OK && b < n;) {
         const int e = batch_group_end(samples.data(), n, b, cap);
         if (e == b + 1 && batch_bucket(samples[b]) > cap) {
             const RenderOut o{items[b].rgb, items[b].ids, nullptr, counts, counts + 4};
-            st = launch_wavefront(*items[b].scene, items[b].params, items[b].W, items[b].H, o, s, A.ws, A, nullptr);
+            st = launch_wavefront(*items[b].scene, items[b].params, items[b].W, items[b].H, o, s, A.ws, A, nullptr,
+                                  FrameInit{});
         } else {
             int rep = 0;
             st = launch_batch(items.data() + b, e - b, counts, counts + 4, s, A.ws, A, eager ? 0 : 1, &rep);
@@ -834,13 +825,14 @@ int rtg_autotune(const rtg_request *reqs, int n, int reps, rtg_tuning *best, rtg
     hipStream_t s = A.stream;
     unsigned long long *counts = A.counters.as<unsigned long long>();
     auto run = [&]() -> int {
-        k_zero_u64<<<1, 64, 0, s>>>(counts, 5);
+        const FrameInit zero{nullptr, 0, nullptr, 0, counts, counts + 4};
         int st = A.ws.order_before(s);
         if (st != RTG_OK) return st;
         if (n == 1) {
             const RenderOut o{items[0].rgb, nullptr, nullptr, counts, counts + 4};
-            st = launch_wavefront(*items[0].scene, items[0].params, items[0].W, items[0].H, o, s, A.ws, A, nullptr);
-        } else {
+            st = launch_wavefront(*items[0].scene, items[0].params, items[0].W, items[0].H, o, s, A.ws, A, nullptr,
+                                  zero);
+        } else if ((st = launch_init(zero, nullptr, 0, s)) == RTG_OK) {
             st = launch_batch(items.data(), n, counts, counts + 4, s, A.ws, A, 0, nullptr);
         }
         const int st2 = A.ws.mark_done(s);

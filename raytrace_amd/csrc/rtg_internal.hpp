@@ -193,6 +193,8 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
 int scene_update_shading(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream);
 // Frame size of a render (params or the scene camera's) and parameter checks.
 int resolve_size(const SceneRes &S, const rtg_params *p, int &W, int &H);
+// The modes that trace primary (and, for the shadow test, shadow) rays only.
+inline bool primary_only(int mode) { return mode >= RTG_MODE_DEPTHTEST && mode <= RTG_MODE_SHADOWTEST; }
 
 
 struct RenderOut {
@@ -202,6 +204,25 @@ struct RenderOut {
     unsigned long long *counts;  // device, 4 counters (accumulated)
     unsigned long long *retests = nullptr;  // device, 1 counter: FP64 re-tests (optional)
 };
+
+// What the first kernel of a frame or batch clears: RGB to 127 (the reference
+// clears its output to it, RayTracer.cpp:620), ids to -1, the ray counts (and
+// the FP64 re-test count) to 0.  Null pointers are left out.
+struct FrameInit {
+    uint8_t *rgb = nullptr;
+    size_t rgb_bytes = 0;
+    int32_t *ids = nullptr;
+    size_t ids_bytes = 0;
+    unsigned long long *counts = nullptr;   // 4
+    unsigned long long *retests = nullptr;  // 1
+};
+inline FrameInit init_of(const RenderOut &o, int W, int H) {
+    const size_t npix = (size_t)W * H;
+    return FrameInit{o.rgb, npix * 3, o.ids, o.ids ? npix * 8 : 0, o.counts, o.retests};
+}
+// Enqueue that kernel; it also zeroes the `n_words` words at `words` (a pass's
+// queue counters), if any.
+int launch_init(const FrameInit &f, unsigned *words, int n_words, hipStream_t stream);
 
 // Cooperative cancel of a frame (rtg_cancel of an asynchronous job).  `host`
 // and `dev` are the host and device addresses of one mapped flag.  Kernels
@@ -229,8 +250,8 @@ struct MegaScratch {
     int blocks;
     double dp;
 };
-// Enqueue the megakernel with the given scratch (tables already written);
-// allocates nothing.
+// Enqueue the megakernel with the given scratch (tables already written) and
+// the launch that clears its outputs and counters; allocates nothing.
 int enqueue_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
                        Arena &A, const Cancel *cancel, const MegaScratch &ms);
 // Enqueue the ray-generation tables (float)((x - W/2) dp), (float)((y - H/2) dp)
@@ -257,8 +278,11 @@ int reserve_frame(Workspace &ws, int W, int H, int spp, int max_level, int fanou
 // reserves before it launches.
 int reserve_batch(Workspace &ws, size_t samples, int n_reqs, int n_scenes, size_t table_floats, int max_level,
                   int fanout, int n_on, hipStream_t stream, Arena &A);
+// `init`: what its first kernel clears (a frame inside a batch clears nothing).
+// The primary-only modes (depth, normal, texture, material, shadow test) take
+// the same path: level 0's rays, and k_view in place of the shading kernels.
 int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                     Workspace &ws, Arena &A, const Cancel *cancel);
+                     Workspace &ws, Arena &A, const Cancel *cancel, const FrameInit &init);
 
 // One request of a batch (rtg_render_batch): a frame of `scene` into device
 // outputs.

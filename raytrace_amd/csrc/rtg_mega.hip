@@ -156,6 +156,8 @@ int enqueue_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, con
     a.counts = o.counts;
     a.cancel = cancel ? cancel->dev : nullptr;
     a.spill = ms.spill;
+    const int st = launch_init(init_of(o, W, H), nullptr, 0, stream);
+    if (st != RTG_OK) return st;
     const int kt = ktime_begin(A, stream, KT_MEGA, (uint64_t)W * H * a.spp);
     k_megakernel<<<ms.blocks, kBlockThreads, 0, stream>>>(S.view, a);
     ktime_end(A, stream, kt);

@@ -33,13 +33,6 @@ constexpr int kMaxDevices = 64;
 std::mutex g_lock;
 unsigned char *g_ptr[kMaxDevices] = {};  // the device address of `scratch` on each device
 
-__global__ void k_fill_bytes(uint8_t *p, size_t n, uint8_t v) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
-}
-__global__ void k_zero_counts(unsigned long long *p) {
-    if (threadIdx.x < 4) p[threadIdx.x] = 0;
-}
-
 }  // namespace
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -91,11 +84,6 @@ extern "C" int rtg_render_device_noalloc(rtg_scene_t scene, const rtg_params *pa
     ms.dp = tan((double)scene->res.camera.fovy * 3.1415926535897932384 / 360) / (H / 2);
     unsigned long long *counts = stats_dev ? reinterpret_cast<unsigned long long *>(stats_dev)
                                            : reinterpret_cast<unsigned long long *>(base);
-    const size_t npix = (size_t)W * H;
-    k_fill_bytes<<<1024, 256, 0, s>>>(rgb_dev, npix * 3, 127);
-    if (ids_dev) k_fill_bytes<<<1024, 256, 0, s>>>(reinterpret_cast<uint8_t *>(ids_dev), npix * 8, 0xff);
-    k_zero_counts<<<1, 64, 0, s>>>(counts);
-    RTG_HIP(hipGetLastError());
     if ((st = write_raygen_tables(ms.tables, W, H, ms.dp, s)) != RTG_OK) return st;
     const bool kt = A.ktimes;
     A.ktimes = false;

@@ -30,13 +30,6 @@
 namespace rtg {
 namespace {
 
-__global__ void k_fill_bytes(uint8_t *p, size_t n, uint8_t v) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
-}
-__global__ void k_zero_counts(unsigned long long *p) {
-    if (threadIdx.x < 5) p[threadIdx.x] = 0;  // 4 ray counts + FP64 re-tests
-}
-
 using Clock = std::chrono::steady_clock;
 
 constexpr int kGraphMinBatch = 8;  // smallest batch the loop captures into a hipGraph
@@ -108,14 +101,13 @@ static int slot_launch(ServeSlot &s, rtg_serve_request *reqs, const std::vector<
     }
     int st = slot_reserve(s, bytes);
     if (st != RTG_OK) return st;
-    k_fill_bytes<<<1024, 256, 0, s.stream>>>(s.out.as<uint8_t>(), bytes, 127);
-    k_zero_counts<<<1, 64, 0, s.stream>>>(s.counts.as<unsigned long long>());
+    unsigned long long *counts = s.counts.as<unsigned long long>();  // 4 ray counts + FP64 re-tests
+    const FrameInit init{s.out.as<uint8_t>(), bytes, nullptr, 0, counts, counts + 4};
     if (plain || ids.size() == 1) {  // a batch of one takes the single-frame path (uniform kernel arguments)
         const rtg_serve_request &q = reqs[ids[0]];
-        const RenderOut o{s.out.as<uint8_t>(), nullptr, nullptr, s.counts.as<unsigned long long>(),
-                          s.counts.as<unsigned long long>() + 4};
+        const RenderOut o{s.out.as<uint8_t>(), nullptr, nullptr, counts, counts + 4};
         st = launch_wavefront(q.scene->res, stream_mode(q.params, side_stream), info[ids[0]].W, info[ids[0]].H, o, s.stream, s.ws, A,
-                              nullptr);
+                              nullptr, init);
     } else {
         std::vector<BatchItem> items(ids.size());
         for (size_t k = 0; k < ids.size(); ++k) {
@@ -127,8 +119,8 @@ static int slot_launch(ServeSlot &s, rtg_serve_request *reqs, const std::vector<
         // milliseconds inside some request's latency for little launch time saved.
         int replayed = 0;
         const int cap = (int)items.size() >= kGraphMinBatch ? capture_at : 0;
-        st = launch_batch(items.data(), (int)items.size(), s.counts.as<unsigned long long>(),
-                          s.counts.as<unsigned long long>() + 4, s.stream, s.ws, A, cap, &replayed);
+        if ((st = launch_init(init, nullptr, 0, s.stream)) == RTG_OK)
+            st = launch_batch(items.data(), (int)items.size(), counts, counts + 4, s.stream, s.ws, A, cap, &replayed);
     }
     if (st != RTG_OK) return st;
     RTG_HIP(hipMemcpyAsync(s.pinned, s.out.p, bytes, hipMemcpyDeviceToHost, s.stream));

@@ -367,6 +367,7 @@ __global__ __launch_bounds__(kBlockThreads, 4) void k_shade(SceneView S0, WaveAr
                                                          unsigned *masks, WRay *next, LevelCtr *ctr,
                                                          unsigned *shadow, float4 *slots) {
     const int n = k == 0 ? A.n_samples : (int)*n_ptr;
+    if (surplus_block(n)) return;
     if (wave_cancelled(A)) return;
     WaveQueue wq(ctr->sched[1], n, grab_lg_for(n, A.grab_lg));
     uint32_t c_shadow = 0;
@@ -672,9 +673,68 @@ __global__ void k_resolve(WaveArgs A, const float4 *samples) {
     }
 }
 
-__global__ void k_zero_u32(unsigned *p, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
+// The primary-only modes: the colour of every level-0 sample's closest hit
+// (debug_color, the megakernel's arithmetic), from the hits of k_extend and,
+// for the shadow test, the light masks of k_occlude.  One walk of k_extend,
+// 6 waves per SIMD, and this in place of the megakernel's walk at the
+// registers of a whole ray tree, 3 waves per SIMD (normal view of 200,000
+// triangles, 1280x720, to the host: 543 -> 465 us a call).
+__global__ __launch_bounds__(kBlockThreads) void k_view(SceneView S, WaveArgs A, int mode, const WHit *hits,
+                                                      const unsigned *masks, float4 *samples) {
+    if (A.cancel != nullptr && *(volatile unsigned *)A.abort != 0) return;
+    const WaveReq &R = A.r0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < A.n_samples; i += gridDim.x * blockDim.x) {
+        int px, py, si;
+        if (!sample_pixel(R, i, px, py, si)) continue;
+        const TraceRay q = primary_ray_w(S, R, px, py, si);
+        const WHit w = hits[i];
+        const Hit h{w.t, w.kind, w.obj, w.prim, w.w, w.u, w.v};
+        const size_t pix = (size_t)py * R.W + px;
+        if (si == 0 && R.ids) {
+            R.ids[2 * pix] = h.obj;
+            R.ids[2 * pix + 1] = id_prim(S, h);
+        }
+        if (si == 0 && R.tprim) R.tprim[pix] = h.t;
+        const V3 c = debug_color(S, mode, q, h, [&](int li, const LightTerm &, bool, const HitRec &) -> bool {
+            return (masks[i] >> li) & 1u;
+        });
+        if (R.spp != 1) {
+            samples[i] = make_float4(c.x, c.y, c.z, h.t);
+            continue;
+        }
+        uint8_t *p = R.rgb + 3 * pix;
+        p[0] = quantize(c.x), p[1] = quantize(c.y), p[2] = quantize(c.z);
+    }
+}
+
+// Fill n bytes with v: whole 16-byte words, and the bytes before and after them.
+__device__ inline void fill_bytes(uint8_t *p, size_t n, uint8_t v, size_t i, size_t step) {
+    const size_t head = min(n, (size_t)(-(intptr_t)p & 15)), words = (n - head) >> 4, tail = head + (words << 4);
+    const unsigned w = v * 0x01010101u;
+    uint4 *q = reinterpret_cast<uint4 *>(p + head);
+    for (size_t k = i; k < words; k += step) q[k] = make_uint4(w, w, w, w);
+    if (i < head) p[i] = v;
+    if (i < n - tail) p[tail + i] = v;
+}
+
+// Everything a frame clears, in one launch: the first k_extend waits for what
+// precedes it, which was a launch each for RGB, ids, two groups of counters
+// and the queue counters (64x64 frame 267 -> 261 us a call, 640x480 with ids
+// 639 -> 609 us, together with k_shade's surplus blocks leaving at once).
+__global__ void k_init(FrameInit f, unsigned *words, int n_words) {
+    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+    fill_bytes(f.rgb, f.rgb_bytes, 127, i, step);
+    fill_bytes(reinterpret_cast<uint8_t *>(f.ids), f.ids_bytes, 0xff, i, step);
+    for (size_t k = i; k < (size_t)n_words; k += step) words[k] = 0;
+    if (f.counts != nullptr && i < 4) f.counts[i] = 0;
+    if (f.retests != nullptr && i == 4) f.retests[0] = 0;
+}
+
+int launch_init(const FrameInit &f, unsigned *words, int n_words, hipStream_t stream) {
+    const size_t items = std::max({f.rgb_bytes / 16, f.ids_bytes / 16, (size_t)n_words, (size_t)16});
+    k_init<<<(int)std::min<size_t>(1024, (items + 255) / 256), 256, 0, stream>>>(f, words, n_words);
+    RTG_HIP(hipGetLastError());
+    return RTG_OK;
 }
 
 // Batch: request of every 64-sample chunk of level 0 (binary search over the
@@ -809,8 +869,11 @@ static int reserve_all(Workspace &ws, const WavePlan &pl, int cus) {
 // allocates or waits.
 template <bool B>
 static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &pl, hipStream_t stream,
-                        Workspace &ws, Arena &A, const Cancel *cancel, bool retest, bool overlap) {
+                        Workspace &ws, Arena &A, const Cancel *cancel, bool retest, bool overlap,
+                        const FrameInit &init, int mode) {
     const int *cancel_host = cancel ? cancel->host : nullptr;
+    const bool view = primary_only(mode);  // (one level) k_view shades the hits
+    const bool shadows = pl.n_on > 0 && (!view || mode == RTG_MODE_SHADOWTEST);
     const int cus = A.cus > 0 ? A.cus : 256;
     const Grids<B> g(cus, A.tune.grid_pct);
     if (!pl.no_sync) {
@@ -824,7 +887,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     // they run on the workspace's side stream, concurrently with the next
     // level, and join the render stream before k_combine (the last level's
     // stay on the render stream, see below).
-    const bool ov = overlap && pl.n_on > 0;
+    const bool ov = overlap && shadows;
     if (ov) {
         int st = ws.side_init();
         if (st != RTG_OK) return st;
@@ -855,12 +918,18 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         return RTG_OK;
     };
     LevelCtr *ctr = ws.w_qcount.as<LevelCtr>();
-    k_zero_u32<<<(kPassCtrWords + 255) / 256, 256, 0, stream>>>(ws.w_qcount.as<unsigned>(), kPassCtrWords);
-    const int lblocks = std::max(8, cus * 16);  // k_local, k_combine
+    {
+        const int st = launch_init(init, ws.w_qcount.as<unsigned>(), kPassCtrWords, stream);
+        if (st != RTG_OK) return st;
+    }
     const bool early_local = !B && pl.no_sync;
     auto grid = [](int gmax, size_t items) {
         return (int)std::max<size_t>(8, std::min<size_t>(gmax, (items + 127) / 128));
     };
+    // k_local, k_combine: at most 16 blocks per CU, no more than the level's
+    // bound needs (the blocks of an empty 4096-block grid take 4-5 us to
+    // dispatch); whole eighths (xcd_chunks)
+    auto lgrid = [&](size_t items) { return (std::min(cus * 16, grid(cus * 16, items)) + 7) & ~7; };
     WaveArgs args = a;
     args.spill = ws.spill.as<int>();
     args.cancel = cancel ? cancel->dev : nullptr;
@@ -869,6 +938,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     if (ov) oargs.spill = ws.spill2.as<int>();
     if (ov2) oargs2.spill = ws.spill3.as<int>();
     size_t n_k = (size_t)pl.n_samples;
+    size_t counted[Workspace::kLevels] = {};  // rays of each level, as far as the host knows
     int last = -1;
     const size_t cap = level_ray_cap(pl.n_on);
     for (int k = 0; k <= pl.max_level && n_k > 0; ++k) {
@@ -896,11 +966,14 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             k_extend<B, false><<<grid(g.extend, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         ktime_end(A, stream, kt, n_ptr);
-        kt = ktime_begin(A, stream, KT_SHADE, n_k);
-        k_shade<B><<<grid(g.shade, n_k), kBlockThreads, 0, stream>>>(
-            S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ws.w_nodes[k].as<WNode>(),
-            ws.w_masks[k].as<unsigned>(), next, ctr + k, ws.w_shadow[k].as<unsigned>(), ws.w_slots[k].as<float4>());
-        ktime_end(A, stream, kt, n_ptr);
+        if (!view || shadows) {
+            kt = ktime_begin(A, stream, KT_SHADE, n_k);
+            k_shade<B><<<grid(g.shade, n_k), kBlockThreads, 0, stream>>>(
+                S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ws.w_nodes[k].as<WNode>(),
+                ws.w_masks[k].as<unsigned>(), next, ctr + k, ws.w_shadow[k].as<unsigned>(),
+                ws.w_slots[k].as<float4>());
+            ktime_end(A, stream, kt, n_ptr);
+        }
         // The last level has no next level to overlap: its shadow rays stay
         // on the render stream (with that stream's spill area), where they
         // run beside the previous level's shadow rays on the side stream.
@@ -911,7 +984,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             RTG_HIP(hipStreamWaitEvent(sk, ws.ev_fork[k], 0));
             (second ? forked2 : forked) = true;
         }
-        if (pl.n_on > 0) {
+        if (shadows) {
             kt = ktime_begin(A, sk, KT_OCCLUDE, 0);
             k_occlude<B><<<grid(side_k ? g.occlude : g.occlude_alone, n_k * pl.n_on), kBlockThreads, 0, sk>>>(
                 S0, side_k ? (second ? oargs2 : oargs) : args, ws.w_nodes[k].as<WNode>(),
@@ -926,12 +999,13 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         // up on the frame's path (measured).
         if (early_local && k < pl.max_level) {
             kt = ktime_begin(A, sk, KT_LOCAL, 0);
-            k_local<B><<<lblocks, kBlockThreads, 0, sk>>>(S0, args, k, n_ptr, ws.w_nodes[k].as<WNode>(),
+            k_local<B><<<lgrid(n_k), kBlockThreads, 0, sk>>>(S0, args, k, n_ptr, ws.w_nodes[k].as<WNode>(),
                                                           ws.w_masks[k].as<unsigned>());
             ktime_end(A, sk, kt, n_ptr);
         }
         RTG_HIP(hipGetLastError());
         last = k;
+        counted[k] = n_k;
         if (k == pl.max_level) break;
         if (pl.no_sync) {
             n_k = pl.bound[k + 1];
@@ -948,12 +1022,17 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     if (cancel_host && *cancel_host) return RTG_OK;
     if (!pl.no_sync && ws.grow(ws.w_samples, (size_t)pl.n_samples * sizeof(float4)))
         return fail(RTG_E_NOMEM, "samples");
-    const int blocks = std::max(8, cus * 16);
-    for (int k = last; k >= 0; --k) {
+    if (view) {
+        const int kt = ktime_begin(A, stream, KT_COMBINE, (uint64_t)pl.n_samples);
+        k_view<<<lgrid((size_t)pl.n_samples), kBlockThreads, 0, stream>>>(
+            S0, args, mode, ws.w_hits[0].as<WHit>(), ws.w_masks[0].as<unsigned>(), ws.w_samples.as<float4>());
+        ktime_end(A, stream, kt);
+    }
+    for (int k = view ? -1 : last; k >= 0; --k) {
         const WRay *rays = k == 0 ? nullptr : ws.w_rays[k].as<WRay>();
         const unsigned *n_ptr = k == 0 ? nullptr : &ctr[k - 1].n_next.v;
         const int kt = ktime_begin(A, stream, KT_COMBINE, k == 0 ? (uint64_t)pl.n_samples : 0);
-        k_combine<B><<<blocks, kBlockThreads, 0, stream>>>(
+        k_combine<B><<<lgrid(counted[k]), kBlockThreads, 0, stream>>>(
             S0, args, k, rays, n_ptr, ws.w_nodes[k].as<WNode>(), ws.w_masks[k].as<unsigned>(),
             ws.w_slots[k].as<float4>(), k > 0 ? ws.w_slots[k - 1].as<float4>() : nullptr,
             ws.w_samples.as<float4>(), early_local && k < pl.max_level ? 1 : 0);
@@ -989,7 +1068,7 @@ int reserve_frame(Workspace &ws, int W, int H, int spp, int max_level, int fanou
 }
 
 int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                     Workspace &ws, Arena &A, const Cancel *cancel) {
+                     Workspace &ws, Arena &A, const Cancel *cancel, const FrameInit &init) {
     const int *cancel_host = cancel ? cancel->host : nullptr;
     double dp;
     int st = upload_raygen_tables(S, W, H, stream, ws, dp);
@@ -997,7 +1076,10 @@ int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const
     if ((st = host_buffers(ws)) != RTG_OK) return st;
     WaveArgs a{};
     WaveReq &r = a.r0;
-    r.W = W, r.H = H, r.spp = p.spp > 0 ? p.spp : 1, r.max_level = p.max_level, r.tile_compat = p.tile_compat;
+    const bool view = primary_only(p.mode);
+    const int fanout = view ? 0 : S.max_fanout;
+    r.W = W, r.H = H, r.spp = p.spp > 0 ? p.spp : 1, r.tile_compat = p.tile_compat;
+    r.max_level = view ? 0 : p.max_level;
     const int lg = A.tune.tile_lg, tw = 1 << lg, th = 64 >> lg;
     r.tile_lg = lg;
     r.bw = (W + tw - 1) / tw;
@@ -1018,21 +1100,22 @@ int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const
     // samples each, so that the queues of all levels stay a few GB.
     const int rows = (H + th - 1) / th, per_row = r.bw * 64 * r.spp;
     const int n_on = __builtin_popcount(S.lights_on);
-    int rows_per_pass = frame_rows_per_pass(rows, (size_t)per_row, S.max_fanout, n_on, kPassSamples);
+    int rows_per_pass = frame_rows_per_pass(rows, (size_t)per_row, fanout, n_on, kPassSamples);
+    if (view) rows_per_pass = std::min(rows_per_pass, std::max(1, kNoSyncMaxSamples / per_row));
     if (cancel && cancel->pass_samples > 0)
         rows_per_pass = std::min(rows_per_pass, std::max(1, (int)(cancel->pass_samples / (size_t)per_row)));
     for (int row0 = 0; row0 < rows; row0 += rows_per_pass) {
         r.row0 = row0;
         r.n_samples = std::min(rows_per_pass, rows - row0) * per_row;
         a.n_samples = r.n_samples;
-        WavePlan pl = make_plan(r.n_samples, p.max_level, S.max_fanout, n_on, 1, A.no_sync_budget);
+        WavePlan pl = make_plan(r.n_samples, r.max_level, fanout, n_on, 1, A.no_sync_budget);
         // A very large frame keeps the GPU busy at every level; there the
         // host round trip per level costs little, and sizing each level from
         // the previous level's count saves the worst-case queue memory.
         if (r.n_samples > kNoSyncMaxSamples) pl.no_sync = false;
         if (pl.no_sync && (st = reserve_all(ws, pl, A.cus > 0 ? A.cus : 256)) != RTG_OK) return st;
         st = enqueue_wave<false>(S.view, a, pl, stream, ws, A, cancel, r.retest != 0,
-                                 (p.flags & RTG_FLAG_ONE_STREAM) == 0);
+                                 (p.flags & RTG_FLAG_ONE_STREAM) == 0, row0 == 0 ? init : FrameInit{}, p.mode);
         if (st != RTG_OK || (cancel_host && *cancel_host)) return st;
     }
     return RTG_OK;
@@ -1188,7 +1271,8 @@ int launch_batch(const BatchItem *items, int n, unsigned long long *counts, unsi
     auto enqueue = [&](bool overlap) -> int {
         k_chunk_req<<<(int)((n_chunks + 255) / 256), 256, 0, stream>>>(a.reqs, n_pad, ws.b_chunks.as<int>(),
                                                                       (int)n_chunks);
-        return enqueue_wave<true>(SceneView{}, a, pl, stream, ws, A, nullptr, any_retest, overlap && !one_stream);
+        return enqueue_wave<true>(SceneView{}, a, pl, stream, ws, A, nullptr, any_retest, overlap && !one_stream,
+                                  FrameInit{}, RTG_MODE_RAYTRACE);
     };
     if (use_graph && capture_at > 1 && !(ws.graph != nullptr && ws.graph_key == key)) {
         int slot = -1;
