@@ -117,25 +117,27 @@ struct alignas(256) LineCtr {
     unsigned pad[63];
 };
 
-// Per-wave dynamic work split: a wave grabs chunks of 64 << grab_lg items,
+// Per-wave dynamic work split: a wave grabs chunks of kStep << grab_lg items,
 // first from its XCD's contiguous eighth of the range (one counter per XCD, so
 // neighbouring chunks share an L2), then from the other XCDs' eighths once its
-// own is exhausted, and hands a grabbed chunk out 64 items per next() call.
+// own is exhausted, and hands a grabbed chunk out kStep items per next() call.
 // `ctr` points to 8 counters that are zero at launch.  Every lane of the wave
-// must call next(); it returns the first item of the next 64, or -1 when every
-// chunk is taken.  A region whose counter was seen past its end is never tried
-// again by the wave, so a wave makes at most 8 failed grabs.
-struct WaveQueue {
+// must call next(); it returns the first item of the next kStep, or -1 when
+// every chunk is taken.  A region whose counter was seen past its end is never
+// tried again by the wave, so a wave makes at most 8 failed grabs.
+template <int kStepLg = 6>
+struct WaveQueueT {
+    static constexpr int kStep = 1 << kStepLg;
     LineCtr *ctr;
     int n, glg, nchunks, region, x;
     int cur, end;   // the grabbed chunk: next item handed out, end (wave-uniform)
     uint32_t dead;  // regions this wave has seen exhausted
-    __device__ WaveQueue(LineCtr *c, int n_items, int grab_lg = 0)
-        : ctr(c), n(n_items), glg(grab_lg), nchunks((n_items + (64 << grab_lg) - 1) >> (6 + grab_lg)),
+    __device__ WaveQueueT(LineCtr *c, int n_items, int grab_lg = 0)
+        : ctr(c), n(n_items), glg(grab_lg), nchunks((n_items + (kStep << grab_lg) - 1) >> (kStepLg + grab_lg)),
           region((nchunks + 7) >> 3), x(blockIdx.x & 7), cur(0), end(0), dead(0) {}
     __device__ int region_len(int r) const { return max(0, min(region, nchunks - r * region)); }
     __device__ int next() {
-        if (cur + 64 < end) return cur += 64;
+        if (cur + kStep < end) return cur += kStep;
         if (nchunks == 0) return -1;
         const int lane = __lane_id();
         for (;;) {
@@ -143,8 +145,8 @@ struct WaveQueue {
             if (lane == 0) c = (int)atomicAdd(&ctr[x].v, 1u);
             c = __builtin_amdgcn_readfirstlane(c);  // wave-uniform: an SGPR
             if (c < region_len(x)) {
-                cur = (x * region + c) << (6 + glg);
-                end = min(n, cur + (64 << glg));
+                cur = (x * region + c) << (kStepLg + glg);
+                end = min(n, cur + (kStep << glg));
                 return cur;
             }
             dead |= 1u << x;
@@ -160,6 +162,7 @@ struct WaveQueue {
         }
     }
 };
+using WaveQueue = WaveQueueT<>;
 
 __device__ inline uint32_t wave_sum_u32(uint32_t v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

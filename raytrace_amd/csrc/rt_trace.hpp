@@ -447,6 +447,39 @@ RTG_HD PrimRec load_prim(const SceneView &S, int pi) {
     return r;
 }
 
+// Closest-hit test of one primitive: objects with index < `before` only.
+RTG_HD bool closest_prim(const TraceRay &q, const PrimRec &R, int before, Hit &h) {
+    const int tag = as_int(R.a.w);
+    const V3 p = V3{R.a.x, R.a.y, R.a.z};
+    if (tag >= 0) {  // triangle, tag = global index
+        const int obj = as_int(R.b.w);
+        if (obj >= before || (tag == q.src.prim && obj == q.src.obj && !q.self_test)) return false;
+        float w, u, v;
+        const float t = tri_test(q.r, V3{R.b.x, R.b.y, R.b.z}, V3{R.c.x, R.c.y, R.c.z}, p, w, u, v);
+        h = Hit{t, HIT_TRI, obj, tag, w, u, v};
+        return t < kMiss;
+    }
+    const int obj = ~tag;  // sphere, tag = ~object
+    if (obj >= before || (q.src.obj == obj && !q.inside)) return false;
+    const float t = q.src.obj == obj ? sphere_exit_t(q.r, p, R.b.x) : sphere_enter_t(q.r, p, R.b.x);
+    h = Hit{t, HIT_SPHERE, obj, -1, 0, 0, 0};
+    return t > 1e-6f && t < kMiss;
+}
+
+// Any-hit test of one primitive: it blocks the segment of length `dis`.
+RTG_HD bool any_prim(const TraceRay &q, const PrimRec &R, float dis) {
+    const int tag = as_int(R.a.w);
+    const V3 p = V3{R.a.x, R.a.y, R.a.z};
+    if (tag >= 0) {
+        if (tag == q.src.prim && as_int(R.b.w) == q.src.obj && !q.self_test) return false;
+        float w, u, v;
+        return tri_test(q.r, V3{R.b.x, R.b.y, R.b.z}, V3{R.c.x, R.c.y, R.c.z}, p, w, u, v) < dis;
+    }
+    if (q.src.obj == ~tag) return q.inside && R.b.y < dis;  // HitRes(radius) (Basic3DObject.cpp:143-144)
+    const float t = sphere_enter_t(q.r, p, R.b.x);
+    return t > 1e-6f && t < dis;
+}
+
 // Closest hit (RayTracer.cpp:455-465).  kRetest: FP64 near-tie re-test (see
 // above); *retested counts the queries that were re-tested.  kBefore: only
 // objects with index < `before` take part (see child_src).
@@ -473,41 +506,40 @@ RTG_HD Hit trace_closest(const SceneView &S, const TraceRay &q, Stack &st, int *
     };
     bvh_walk<!kRetest>(S, q.r, tmax, st, [&](int pi, float &tm) -> bool {
         const PrimRec R = load_prim(S, pi);
+        if constexpr (!kRetest) {
+            Hit h;
+            if (closest_prim(q, R, kBefore ? before : 0x7fffffff, h))
+                take(h.t, hit_key(h.obj, h.prim), pi, h, tm);
+            return false;
+        }
         const float4 A = R.a;
         const int tag = as_int(A.w);
         const V3 p = V3{A.x, A.y, A.z};
         if (tag >= 0) {  // triangle, tag = global index
             const float4 B = R.b, C = R.c;
             const int obj = as_int(B.w);
-            if (kBefore && obj >= before) return false;
             if (tag == q.src.prim && obj == q.src.obj && !q.self_test) return false;
             const V3 e1 = V3{B.x, B.y, B.z}, e2 = V3{C.x, C.y, C.z};
-            float w, u, v, t;
-            if constexpr (kRetest) {
-                // tri_test's values without its early exits (same operations)
-                const V3 tmp1 = cross(q.r.d, e2), t2r = q.r.o - p;
-                const float f = 1.0f / dot(e1, tmp1);
-                u = dot(t2r, tmp1) * f;
-                const V3 tmp2 = cross(t2r, e1);
-                v = dot(q.r.d, tmp2) * f;
-                w = 1.0f - u - v;
-                const float tt = dot(e2, tmp2) * f;
-                if (tt == tt && tt > 0.0f) {
-                    const float eps = 1e-6f;
-                    const bool marginal = fabsf(u) <= eps || fabsf(u - 1.0f) <= eps || fabsf(v) <= eps ||
-                                          fabsf(w) <= eps || fabsf(tt - 1e-5f) <= eps;
-                    const bool inside = u >= -eps && u <= 1.0f + eps && v >= -eps && w >= -eps;
-                    if (marginal && inside) band.add(pi, tt);
-                }
-                const bool ok = !(u < 0.0f || u > 1.0f) && !(v < 0.0f || w < 0.0f) && tt > 1e-5f;
-                t = ok ? tt : kMiss;
-            } else {
-                t = tri_test(q.r, e1, e2, p, w, u, v);
+            // tri_test's values without its early exits (same operations)
+            const V3 tmp1 = cross(q.r.d, e2), t2r = q.r.o - p;
+            const float f = 1.0f / dot(e1, tmp1);
+            const float u = dot(t2r, tmp1) * f;
+            const V3 tmp2 = cross(t2r, e1);
+            const float v = dot(q.r.d, tmp2) * f;
+            const float w = 1.0f - u - v;
+            const float tt = dot(e2, tmp2) * f;
+            if (tt == tt && tt > 0.0f) {
+                const float eps = 1e-6f;
+                const bool marginal = fabsf(u) <= eps || fabsf(u - 1.0f) <= eps || fabsf(v) <= eps ||
+                                      fabsf(w) <= eps || fabsf(tt - 1e-5f) <= eps;
+                const bool inside = u >= -eps && u <= 1.0f + eps && v >= -eps && w >= -eps;
+                if (marginal && inside) band.add(pi, tt);
             }
+            const bool ok = !(u < 0.0f || u > 1.0f) && !(v < 0.0f || w < 0.0f) && tt > 1e-5f;
+            const float t = ok ? tt : kMiss;
             if (t < kMiss) take(t, hit_key(obj, tag), pi, Hit{t, HIT_TRI, obj, tag, w, u, v}, tm);
         } else {  // sphere, tag = ~object
             const int obj = ~tag;
-            if (kBefore && obj >= before) return false;
             const float4 B = R.b;
             float t;
             if (q.src.obj == obj) {
@@ -516,12 +548,10 @@ RTG_HD Hit trace_closest(const SceneView &S, const TraceRay &q, Stack &st, int *
             } else {
                 t = sphere_enter_t(q.r, p, B.x);
             }
-            if constexpr (kRetest) {
-                const V3 s2r = q.r.o - p;
-                const float b = dot(q.r.d, s2r);
-                const float dis = b * b - dot(s2r, s2r) + B.x;
-                if (fabsf(dis) <= 1e-5f * (B.x + b * b)) band.add(pi, -b);
-            }
+            const V3 s2r = q.r.o - p;
+            const float b = dot(q.r.d, s2r);
+            const float dis = b * b - dot(s2r, s2r) + B.x;
+            if (fabsf(dis) <= 1e-5f * (B.x + b * b)) band.add(pi, -b);
             if (t > 1e-6f && t < kMiss) take(t, hit_key(obj, -1), pi, Hit{t, HIT_SPHERE, obj, -1, 0, 0, 0}, tm);
         }
         return false;
@@ -587,29 +617,7 @@ RTG_HD bool trace_any(const SceneView &S, const TraceRay &q, float dis, Stack &s
     bool blocked = false;
     float tmax = dis;
     bvh_walk<true, false>(S, q.r, tmax, st, [&](int pi, float &) -> bool {
-        const PrimRec R = load_prim(S, pi);
-        const float4 A = R.a;
-        const int tag = as_int(A.w);
-        const V3 p = V3{A.x, A.y, A.z};
-        float t;
-        if (tag >= 0) {
-            const float4 B = R.b, C = R.c;
-            const int obj = as_int(B.w);
-            if (tag == q.src.prim && obj == q.src.obj && !q.self_test) return false;
-            float w, u, v;
-            t = tri_test(q.r, V3{B.x, B.y, B.z}, V3{C.x, C.y, C.z}, p, w, u, v);
-        } else {
-            const int obj = ~tag;
-            const float4 B = R.b;
-            if (q.src.obj == obj) {
-                if (!q.inside) return false;
-                blocked = B.y < dis;  // HitRes(radius) (Basic3DObject.cpp:143-144)
-                return blocked;
-            }
-            t = sphere_enter_t(q.r, p, B.x);
-            if (!(t > 1e-6f)) return false;
-        }
-        blocked = t < dis;
+        blocked = any_prim(q, load_prim(S, pi), dis);
         return blocked;
     });
     return blocked;

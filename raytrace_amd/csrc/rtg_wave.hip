@@ -29,6 +29,7 @@
 
 #include "rt_devstack.hpp"
 #include "rt_prep.hpp"
+#include "rt_quad.hpp"
 #include "rtg_internal.hpp"
 
 namespace rtg {
@@ -93,6 +94,7 @@ struct WaveArgs {
     const int *chunk_req;     // B = true: request of each 64-sample chunk of level 0 (-1: padding)
     int n_samples;            // level-0 queue length
     int grab_lg;              // WaveQueue grabs of 64 << grab_lg items
+    int quad_max;  // longest queue walked with four lanes per ray (rt_quad.hpp)
     unsigned long long *counts;
     unsigned long long *retests;  // closest-hit queries re-tested in FP64
     int *spill;
@@ -219,8 +221,9 @@ __device__ inline int sample_req(const WaveArgs &A, int i) {
 // last 64-item chunk finds no work, and leaves before copying the top nodes
 // into LDS (block-uniform, so ahead of the barrier there).  The blocks that
 // stay take every chunk: waves keep grabbing until the queue is empty.
+template <int kStepLg = 6>
 __device__ inline bool surplus_block(int n) {
-    return (int)blockIdx.x * (kBlockThreads / 64) >= ((n + 63) >> 6);
+    return (int)blockIdx.x * (kBlockThreads / 64) >= ((n + (1 << kStepLg) - 1) >> kStepLg);
 }
 
 // Grab size (64 << lg items) for n items: the tuning's, doubled up to eight
@@ -234,26 +237,17 @@ __device__ inline int grab_lg_for(int n, int lg) {
     return lg;
 }
 
-// R: some request asks for the FP64 near-tie re-test (a separate kernel, so
-// the plain closest-hit walk keeps its registers).
-template <bool B, bool R>
-__global__ __launch_bounds__(kBlockThreads, 6) void k_extend(SceneView S0, WaveArgs A, int k, const WRay *rays,
-                                                             const unsigned *n_ptr, WHit *hits, int4 *cs,
-                                                             LineCtr *sched) {
-    const int n = k == 0 ? A.n_samples : (int)*n_ptr;
-    if (surplus_block(n)) return;
-    __shared__ int lds[kLdsStack * kBlockThreads];
-    DevStack st = make_stack(lds, A.spill);
-    if constexpr (!B) {  // one scene: its top nodes in LDS
-        __shared__ Bvh4Node top_nodes[kTopNodes];
-        stack_top_nodes(st, top_nodes, S0);
-    }
-    if (wave_cancelled(A)) return;
-    WaveQueue wq(sched, n, A.grab_lg);
+// Closest hits of the queue's rays: one lane per ray, or with Q four
+// (rt_quad.hpp; lane 0 of the quad writes).
+template <bool B, bool R, bool Q, class Stack>
+__device__ inline void extend_rays(const SceneView &S0, const WaveArgs &A, int k, const WRay *rays, int n, WHit *hits,
+                                   int4 *cs, LineCtr *sched, Stack &st) {
+    WaveQueueT<Q ? 4 : 6> wq(sched, n, Q ? 0 : A.grab_lg);
     uint32_t c_prim = 0, c_refl = 0, c_refr = 0;
     int n_retest = 0;
+    const bool writer = !Q || (threadIdx.x & (kQuadLanes - 1)) == 0;
     for (int base = wq.next(); base >= 0; base = wq.next()) {
-        const int i = base + __lane_id();
+        const int i = base + (Q ? __lane_id() / kQuadLanes : __lane_id());
         if (i >= n) continue;
         int r = 0;
         WRay w{};
@@ -286,15 +280,17 @@ __global__ __launch_bounds__(kBlockThreads, 6) void k_extend(SceneView S0, WaveA
             if (valid) {
                 if constexpr (R)
                     h = Rq.retest ? trace_closest<true>(S, q, st, &n_retest) : trace_closest<false>(S, q, st);
+                else if constexpr (Q)
+                    h = quad_closest(S, q, st, before);
                 else
                     h = trace_closest<false, true>(S, q, st, nullptr, before);
             }
             if (before != 0x7fffffff) {
                 const SrcId c = child_src_of(S, q, h);
-                cs[i] = int4{c.obj, c.prim, c.bin, 0};
+                if (writer) cs[i] = int4{c.obj, c.prim, c.bin, 0};
                 break;
             }
-            if (valid) {
+            if (valid && writer) {
                 if (k == 0)
                     ++c_prim;
                 else if (q.type == RAY_REFLECT)
@@ -303,7 +299,7 @@ __global__ __launch_bounds__(kBlockThreads, 6) void k_extend(SceneView S0, WaveA
                     ++c_refr;
             }
             const bool self = valid && h.kind != HIT_NONE && is_self_rehit(q, h);
-            hits[i] = WHit{h.t, h.w, h.u, h.v, h.kind, h.obj, h.prim, self ? 1 : 0};
+            if (writer) hits[i] = WHit{h.t, h.w, h.u, h.v, h.kind, h.obj, h.prim, self ? 1 : 0};
             if (!self) break;
             if constexpr (R) {
                 const SrcId c = child_src(S, q, h, st);
@@ -318,6 +314,31 @@ __global__ __launch_bounds__(kBlockThreads, 6) void k_extend(SceneView S0, WaveA
         const uint32_t nr = wave_sum_u32((uint32_t)n_retest);
         if (__lane_id() == 0 && nr) atomicAdd(A.retests, (unsigned long long)nr);
     }
+}
+
+// R: some request asks for the FP64 near-tie re-test (a separate kernel, so
+// the plain closest-hit walk keeps its registers).
+template <bool B, bool R>
+__global__ __launch_bounds__(kBlockThreads, 6) void k_extend(SceneView S0, WaveArgs A, int k, const WRay *rays,
+                                                             const unsigned *n_ptr, WHit *hits, int4 *cs,
+                                                             LineCtr *sched) {
+    const int n = k == 0 ? A.n_samples : (int)*n_ptr;
+    const bool quads = !R && n <= A.quad_max;
+    if (quads ? surplus_block<4>(n) : surplus_block(n)) return;
+    __shared__ int lds[kLdsStack * kBlockThreads];
+    DevStack st = make_stack(lds, A.spill);
+    if constexpr (!B) {  // one scene: its top nodes in LDS
+        __shared__ Bvh4Node top_nodes[kTopNodes];
+        stack_top_nodes(st, top_nodes, S0);
+    }
+    if (wave_cancelled(A)) return;
+    if constexpr (!R)
+        if (quads) {
+            QuadStack qs(st, lds);
+            extend_rays<B, R, true>(S0, A, k, rays, n, hits, cs, sched, qs);
+            return;
+        }
+    extend_rays<B, R, false>(S0, A, k, rays, n, hits, cs, sched, st);
 }
 
 // k_shade's appends are staged per wave in LDS and reach their queue a buffer
@@ -529,21 +550,13 @@ __global__ __launch_bounds__(kBlockThreads, 4) void k_shade(SceneView S0, WaveAr
     add_counts(A.counts, 0, c_shadow, 0, 0);
 }
 
-template <bool B>
-__global__ __launch_bounds__(kBlockThreads, 8) void k_occlude(SceneView S0, WaveArgs A, const WNode *nodes,
-                                                           const unsigned *shadow, LevelCtr *ctr, unsigned *masks) {
-    const int n = (int)ctr->n_shadow.v;
-    if (surplus_block(n)) return;
-    __shared__ int lds[kLdsStack * kBlockThreads];
-    DevStack st = make_stack(lds, A.spill);
-    if constexpr (!B) {  // one scene: its top nodes in LDS
-        __shared__ Bvh4Node top_nodes[kTopNodes];
-        stack_top_nodes(st, top_nodes, S0);
-    }
-    if (wave_cancelled(A)) return;
-    WaveQueue wq(ctr->sched[2], n, A.grab_lg);
+// Shadow tests of the queue's entries: one lane per entry, or with Q four.
+template <bool B, bool Q, class Stack>
+__device__ inline void occlude_entries(const SceneView &S0, const WaveArgs &A, const WNode *nodes,
+                                       const unsigned *shadow, int n, LineCtr *sched, unsigned *masks, Stack &st) {
+    WaveQueueT<Q ? 4 : 6> wq(sched, n, Q ? 0 : A.grab_lg);
     for (int base = wq.next(); base >= 0; base = wq.next()) {
-        const int j = base + __lane_id();
+        const int j = base + (Q ? __lane_id() / kQuadLanes : __lane_id());
         if (j >= n) continue;
         const unsigned e = shadow[j];
         const int i = (int)(e >> 5), li = (int)(e & 31);
@@ -558,7 +571,32 @@ __global__ __launch_bounds__(kBlockThreads, 8) void k_occlude(SceneView S0, Wave
         sr.inside = 0;
         sr.src = node_id(nd);
         sr.self_test = self_testable(S, sr.r, sr.src, lt.dis);
-        if (trace_any(S, sr, lt.dis, st)) atomicOr(&masks[i], 1u << li);
+        if constexpr (Q) {
+            if (quad_any(S, sr, lt.dis, st) && (threadIdx.x & (kQuadLanes - 1)) == 0) atomicOr(&masks[i], 1u << li);
+        } else {
+            if (trace_any(S, sr, lt.dis, st)) atomicOr(&masks[i], 1u << li);
+        }
+    }
+}
+
+template <bool B>
+__global__ __launch_bounds__(kBlockThreads, 8) void k_occlude(SceneView S0, WaveArgs A, const WNode *nodes,
+                                                           const unsigned *shadow, LevelCtr *ctr, unsigned *masks) {
+    const int n = (int)ctr->n_shadow.v;
+    const bool quads = n <= A.quad_max;
+    if (quads ? surplus_block<4>(n) : surplus_block(n)) return;
+    __shared__ int lds[kLdsStack * kBlockThreads];
+    DevStack st = make_stack(lds, A.spill);
+    if constexpr (!B) {  // one scene: its top nodes in LDS
+        __shared__ Bvh4Node top_nodes[kTopNodes];
+        stack_top_nodes(st, top_nodes, S0);
+    }
+    if (wave_cancelled(A)) return;
+    if (quads) {
+        QuadStack qs(st, lds);
+        occlude_entries<B, true>(S0, A, nodes, shadow, n, ctr->sched[2], masks, qs);
+    } else {
+        occlude_entries<B, false>(S0, A, nodes, shadow, n, ctr->sched[2], masks, st);
     }
 }
 
@@ -932,6 +970,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     auto lgrid = [&](size_t items) { return (std::min(cus * 16, grid(cus * 16, items)) + 7) & ~7; };
     WaveArgs args = a;
     args.spill = ws.spill.as<int>();
+    args.quad_max = cus * kQuadRaysPerCu;
     args.cancel = cancel ? cancel->dev : nullptr;
     args.abort = ws.w_qcount.as<unsigned>() + Workspace::kLevels * kCtrWords;
     WaveArgs oargs = args, oargs2 = args;
@@ -963,7 +1002,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             k_extend<B, true><<<grid(g.extend, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         else
-            k_extend<B, false><<<grid(g.extend, n_k), kBlockThreads, 0, stream>>>(
+            k_extend<B, false><<<grid(g.extend, kQuadLanes * n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         ktime_end(A, stream, kt, n_ptr);
         if (!view || shadows) {
@@ -986,7 +1025,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         }
         if (shadows) {
             kt = ktime_begin(A, sk, KT_OCCLUDE, 0);
-            k_occlude<B><<<grid(side_k ? g.occlude : g.occlude_alone, n_k * pl.n_on), kBlockThreads, 0, sk>>>(
+            k_occlude<B><<<grid(side_k ? g.occlude : g.occlude_alone, kQuadLanes * n_k * pl.n_on), kBlockThreads, 0, sk>>>(
                 S0, side_k ? (second ? oargs2 : oargs) : args, ws.w_nodes[k].as<WNode>(),
                 ws.w_shadow[k].as<unsigned>(), ctr + k, ws.w_masks[k].as<unsigned>());
             ktime_end(A, sk, kt, &ctr[k].n_shadow.v);
