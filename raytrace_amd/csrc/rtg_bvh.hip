@@ -57,15 +57,22 @@ __global__ void k_bounds_partial(const Box6 *boxes, int n, float *partial) {
     if (threadIdx.x < 6) partial[6 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ void k_bounds_final(const float *partial, int nb, float *cb) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float r[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int b = 0; b < nb; ++b)
-        for (int k = 0; k < 3; ++k) {
-            r[k] = fminf(r[k], partial[6 * b + k]);
-            r[3 + k] = fmaxf(r[3 + k], partial[6 * b + 3 + k]);
-        }
-    for (int k = 0; k < 6; ++k) cb[k] = r[k];
+// One block, a partial per thread (one thread folding 512 partials took 72 us).
+constexpr int kBoundsBlocks = 512;
+__global__ __launch_bounds__(kBoundsBlocks) void k_bounds_final(const float *partial, float *cb) {
+    __shared__ float s[6][kBoundsBlocks];
+    const int t = threadIdx.x;
+    for (int k = 0; k < 6; ++k) s[k][t] = partial[6 * t + k];
+    __syncthreads();
+    for (int w = kBoundsBlocks / 2; w > 0; w /= 2) {
+        if (t < w)
+            for (int k = 0; k < 3; ++k) {
+                s[k][t] = fminf(s[k][t], s[k][t + w]);
+                s[3 + k][t] = fmaxf(s[3 + k][t], s[3 + k][t + w]);
+            }
+        __syncthreads();
+    }
+    if (t < 6) cb[t] = s[t][0];
 }
 
 __global__ void k_morton(const Box6 *boxes, int n, const float *cb, uint64_t *keys) {
@@ -93,38 +100,93 @@ __global__ void k_karras(const uint64_t *keys, int n, int *left, int *right, int
         parent_int[r] = i;
 }
 
-__device__ Box6 load_box_coherent(const Box6 *b) {
-    Box6 r;
-    const int *p = reinterpret_cast<const int *>(b);
-    for (int k = 0; k < 3; ++k) {
-        r.lo[k] = as_float(__hip_atomic_load(p + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        r.hi[k] = as_float(__hip_atomic_load(p + 3 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+// Boxes of the internal nodes.  A node's leaves are a range of the sorted
+// primitives, so its box is a union over that range, in any order (min and max
+// are exact).  A block takes kRefitLeaves leaves and joins the nodes whose
+// range it holds bottom-up in LDS; k_refit_wide takes the nodes that span
+// blocks.  (Bottom-up across the whole grid, each step with a device-wide
+// fence for a box that another XCD's L2 may hold, took 1,119 us for 200,064
+// primitives; these two 20 and 17.)
+constexpr int kRefitLeaves = 512;
+
+struct LdsBoxes {
+    float v[6][kRefitLeaves];
+    __device__ Box6 get(int i) const {
+        Box6 b;
+        for (int k = 0; k < 3; ++k) b.lo[k] = v[k][i], b.hi[k] = v[3 + k][i];
+        return b;
     }
-    return r;
+    __device__ void set(int i, const Box6 &b) {
+        for (int k = 0; k < 3; ++k) v[k][i] = b.lo[k], v[3 + k][i] = b.hi[k];
+    }
+};
+
+__device__ Box6 empty_box() {
+    return Box6{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
 }
-__device__ void store_box_coherent(Box6 *b, const Box6 &v) {
-    int *p = reinterpret_cast<int *>(b);
-    for (int k = 0; k < 3; ++k) {
-        __hip_atomic_store(p + k, as_int(v.lo[k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(p + 3 + k, as_int(v.hi[k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+// Union over the wave's lanes; every lane gets it.
+__device__ Box6 wave_union(Box6 b) {
+    for (int off = 32; off > 0; off >>= 1) {
+        Box6 o;
+        for (int k = 0; k < 3; ++k) o.lo[k] = __shfl_xor(b.lo[k], off, 64), o.hi[k] = __shfl_xor(b.hi[k], off, 64);
+        b = box_union(b, o);
+    }
+    return b;
+}
+
+// sbox: the leaf boxes in sorted order; bbox: the union of each block's.
+__global__ __launch_bounds__(kRefitLeaves) void k_refit(const uint64_t *keys, int n, const Box6 *leaf_boxes,
+                                                        const int *left, const int *right, const int *first,
+                                                        const int *last, const int *parent_int,
+                                                        const int *parent_leaf, Box6 *ibox, Box6 *sbox, Box6 *bbox) {
+    __shared__ LdsBoxes leaf, node;  // node i of the tree at i - b0: a node's index is an end of its range
+    __shared__ int arrived[kRefitLeaves];
+    __shared__ Box6 wbox[kRefitLeaves / 64];
+    const int b0 = blockIdx.x * kRefitLeaves, b1 = min(n, b0 + kRefitLeaves), t = threadIdx.x, j = b0 + t;
+    const Box6 mine = j < n ? leaf_boxes[(uint32_t)keys[j]] : empty_box();
+    leaf.set(t, mine);
+    arrived[t] = 0;
+    if (j < n) sbox[j] = mine;
+    const Box6 w = wave_union(mine);
+    if ((t & 63) == 0) wbox[t >> 6] = w;
+    __syncthreads();
+    if (t == 0) {
+        Box6 b = wbox[0];
+        for (int k = 1; k < kRefitLeaves / 64; ++k) b = box_union(b, wbox[k]);
+        bbox[blockIdx.x] = b;
+    }
+    // the second child to arrive at a node joins its children's boxes
+    for (int p = j < n ? parent_leaf[j] : -1; p >= 0; p = p == 0 ? -1 : parent_int[p]) {
+        if (first[p] < b0 || last[p] >= b1) break;
+        __threadfence_block();
+        if (atomicAdd(&arrived[p - b0], 1) == 0) break;
+        __threadfence_block();
+        const int l = left[p], r = right[p];
+        const Box6 b = box_union(l < 0 ? leaf.get(~l - b0) : node.get(l - b0),
+                                 r < 0 ? leaf.get(~r - b0) : node.get(r - b0));
+        node.set(p - b0, b);
+        ibox[p] = b;
     }
 }
 
-// Bottom-up box union: the second child to arrive at a node computes it.
-__global__ void k_refit(const uint64_t *keys, int n, const Box6 *leaf_boxes, const int *left, const int *right,
-                        const int *parent_int, const int *parent_leaf, int *flags, Box6 *ibox) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    int p = parent_leaf[k];
-    while (p >= 0) {
-        __threadfence();
-        if (atomicAdd(&flags[p], 1) == 0) return;
-        __threadfence();
-        const int l = left[p], r = right[p];
-        const Box6 bl = l < 0 ? leaf_boxes[(uint32_t)keys[~l]] : load_box_coherent(&ibox[l]);
-        const Box6 br = r < 0 ? leaf_boxes[(uint32_t)keys[~r]] : load_box_coherent(&ibox[r]);
-        store_box_coherent(&ibox[p], box_union(bl, br));
-        p = p == 0 ? -1 : parent_int[p];
+// The nodes whose range spans blocks, a wave to each: the leaves up to the end
+// of the first block, whole blocks, and the last block's leaves.
+__global__ __launch_bounds__(kBlock) void k_refit_wide(int n, const int *first, const int *last, const Box6 *sbox,
+                                                       const Box6 *bbox, Box6 *ibox) {
+    const int i = blockIdx.x * kBlock + threadIdx.x, lane = threadIdx.x & 63;
+    const int f = i < n - 1 ? first[i] : 0, l = i < n - 1 ? last[i] : 0;
+    unsigned long long wide = __ballot(f / kRefitLeaves != l / kRefitLeaves);
+    for (; wide; wide &= wide - 1) {
+        const int src = __builtin_ctzll(wide);
+        const int nf = __shfl(f, src, 64), nl = __shfl(l, src, 64);
+        const int fb = nf / kRefitLeaves + 1, lb = nl / kRefitLeaves;
+        Box6 b = empty_box();
+        for (int j = nf + lane; j < fb * kRefitLeaves; j += 64) b = box_union(b, sbox[j]);
+        for (int j = fb + lane; j < lb; j += 64) b = box_union(b, bbox[j]);
+        for (int j = lb * kRefitLeaves + lane; j <= nl; j += 64) b = box_union(b, sbox[j]);
+        b = wave_union(b);
+        if (lane == src) ibox[i] = b;
     }
 }
 
@@ -152,10 +214,56 @@ __global__ void k_reorder(const uint64_t *keys, int n, const float4 *src, float4
     for (int j = 0; j < 3; ++j) dst[3 * (size_t)k + j] = src[3 * (size_t)id + j];
 }
 
-// Top BFS levels first (top_first, rt_bvh.hpp); one thread.
-__global__ void k_top_first(const int *left, const int *right, const int *first, const int *last, int n_int,
-                            int *newidx) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) top_first(left, right, first, last, n_int, newidx);
+// Top BFS levels first: top_first (rt_bvh.hpp) by one wave, a level's nodes in
+// its lanes (one thread, a dependent load after another, took 80 us).
+__global__ __launch_bounds__(64) void k_top_first(const int *left, const int *right, const int *first,
+                                                  const int *last, int n_int, int *newidx) {
+    static_assert(kTopNodes <= 64, "a lane per top node");
+    __shared__ int q[kTopNodes], avail[kTopNodes];
+    const int lane = threadIdx.x;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    auto emitted = [&](int v) { return v >= 0 && last[v] - first[v] + 1 > kLeafMax; };
+    if (lane == 0) q[0] = 0;
+    __syncthreads();
+    int head = 0, nq = 1;
+    while (head < nq && nq < kTopNodes) {  // one BFS level, children appended in queue order
+        const int m = nq - head;
+        const int v = lane < m ? q[head + lane] : -1;
+        const int c0 = v >= 0 ? left[v] : -1, c1 = v >= 0 ? right[v] : -1;
+        const bool e0 = emitted(c0), e1 = emitted(c1);
+        const unsigned long long m0 = __ballot(e0), m1 = __ballot(e1);
+        const int at = nq + __popcll(m0 & below) + __popcll(m1 & below);
+        if (e0 && at < kTopNodes) q[at] = c0;
+        if (e1 && at + (e0 ? 1 : 0) < kTopNodes) q[at + (e0 ? 1 : 0)] = c1;
+        head = nq;
+        nq = min(kTopNodes, nq + __popcll(m0) + __popcll(m1));
+        __syncthreads();
+    }
+    // lane j: the emitted node that holds index j, and the index of top node j
+    int holder = -1, cur = -1;
+    if (lane < nq) {
+        int lo = 0, hi = n_int - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (newidx[mid] < lane)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        while (lo < n_int - 1 && !emitted(lo)) ++lo;
+        holder = lo;
+        cur = newidx[q[lane]];
+    }
+    bool top = lane >= nq;  // (nothing to move)
+    for (int i = 0; i < nq; ++i) top = top || holder == q[i];
+    // the displaced holders take, in order, the indices the top nodes leave
+    const bool leaves = lane < nq && cur >= nq;
+    const unsigned long long ml = __ballot(leaves), md = __ballot(!top);
+    if (leaves) avail[__popcll(ml & below)] = cur;
+    __syncthreads();
+    const int d = __popcll(md & below);
+    if (!top && d < __popcll(ml)) newidx[holder] = avail[d];
+    if (lane < nq) newidx[q[lane]] = lane;
 }
 
 // Widening into 4-wide nodes (rt_bvh.hpp): parents of the binary nodes,
@@ -292,7 +400,7 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
         S.topo_n = donor->topo_n, S.topo_emit = donor->topo_emit;
         donor->topo_n = 0, donor->topo_emit = 0;
     }
-    DevBuf raw, mid, sph, prims_u, boxes, keys, flags, ibox, partial, cb, sort_tmp, nodes2;
+    DevBuf raw, mid, sph, prims_u, boxes, keys, flags, ibox, sbox, bbox, partial, cb, sort_tmp, nodes2;
     DevBuf &keys2 = S.t_keys, &left = S.t_left, &right = S.t_right, &first = S.t_first, &last = S.t_last,
            &pint = S.t_pint, &pleaf = S.t_pleaf, &newidx = S.t_newidx;
     if ((st = upload(mid, part_mid, stream)) || (st = upload(sph, spheres, stream))) return st;
@@ -329,15 +437,23 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
                                                                      S.objs.as<DevObject>(), prims_u.as<float4>(),
                                                                      boxes.as<Box6>());
     int root = 0, n_emit = 0;
+    // boxes of the radix tree's internal nodes over the sorted keys, into ibox
+    auto node_boxes = [&](const uint64_t *sk) -> int {
+        const int nb = (n + kRefitLeaves - 1) / kRefitLeaves;
+        if (ensure(ibox, n * sizeof(Box6)) || ensure(sbox, n * sizeof(Box6)) || ensure(bbox, nb * sizeof(Box6)))
+            return fail(RTG_E_NOMEM, "device allocation failed (bvh boxes)");
+        k_refit<<<nb, kRefitLeaves, 0, stream>>>(sk, n, boxes.as<Box6>(), left.as<int>(), right.as<int>(),
+                                                 first.as<int>(), last.as<int>(), pint.as<int>(), pleaf.as<int>(),
+                                                 ibox.as<Box6>(), sbox.as<Box6>(), bbox.as<Box6>());
+        k_refit_wide<<<nblk(n - 1), kBlock, 0, stream>>>(n, first.as<int>(), last.as<int>(), sbox.as<Box6>(),
+                                                         bbox.as<Box6>(), ibox.as<Box6>());
+        return RTG_OK;
+    };
     if (refit) {
         // same topology: leaf boxes from the new primitives, bottom-up union,
         // nodes re-emitted with the same links, primitives into leaf order
-        if (ensure(flags, n * sizeof(int)) || ensure(ibox, n * sizeof(Box6)))
-            return fail(RTG_E_NOMEM, "device allocation failed (bvh refit)");
         const uint64_t *sk = keys2.as<uint64_t>();
-        k_fill_i32<<<nblk(n), kBlock, 0, stream>>>(flags.as<int>(), n, 0);
-        k_refit<<<nblk(n), kBlock, 0, stream>>>(sk, n, boxes.as<Box6>(), left.as<int>(), right.as<int>(), pint.as<int>(),
-                                                pleaf.as<int>(), flags.as<int>(), ibox.as<Box6>());
+        if ((st = node_boxes(sk)) != RTG_OK) return st;
         n_emit = S.topo_emit;
         if (ensure(nodes2, std::max(n_emit, 1) * sizeof(BvhNode))) return fail(RTG_E_NOMEM, "bvh nodes");
         k_emit<<<nblk(n - 1), kBlock, 0, stream>>>(sk, n - 1, boxes.as<Box6>(), left.as<int>(), right.as<int>(),
@@ -347,15 +463,15 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
         k_reorder<<<nblk(n), kBlock, 0, stream>>>(sk, n, prims_u.as<float4>(), S.prims.as<float4>());
         root = 0;
     } else if (n > kLeafMax) {
-        const int nb = 512;
+        const int nb = kBoundsBlocks;
         if (ensure(partial, nb * 6 * sizeof(float)) || ensure(cb, 6 * sizeof(float)) ||
             ensure(keys, n * sizeof(uint64_t)) || ensure(keys2, n * sizeof(uint64_t)) ||
             ensure(left, n * sizeof(int)) || ensure(right, n * sizeof(int)) || ensure(first, n * sizeof(int)) ||
             ensure(last, n * sizeof(int)) || ensure(pint, n * sizeof(int)) || ensure(pleaf, n * sizeof(int)) ||
-            ensure(flags, n * sizeof(int)) || ensure(ibox, n * sizeof(Box6)) || ensure(newidx, n * sizeof(int)))
+            ensure(flags, n * sizeof(int)) || ensure(newidx, n * sizeof(int)))
             return fail(RTG_E_NOMEM, "device allocation failed (bvh build)");
         k_bounds_partial<<<nb, kBlock, 0, stream>>>(boxes.as<Box6>(), n, partial.as<float>());
-        k_bounds_final<<<1, 64, 0, stream>>>(partial.as<float>(), nb, cb.as<float>());
+        k_bounds_final<<<1, kBoundsBlocks, 0, stream>>>(partial.as<float>(), cb.as<float>());
         k_morton<<<nblk(n), kBlock, 0, stream>>>(boxes.as<Box6>(), n, cb.as<float>(), keys.as<uint64_t>());
         size_t tmp_bytes = 0;
         RTG_HIP(rocprim::radix_sort_keys(nullptr, tmp_bytes, keys.as<uint64_t>(), keys2.as<uint64_t>(), (size_t)n, 0, 62,
@@ -365,11 +481,9 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
                                          62, stream));
         const uint64_t *sk = keys2.as<uint64_t>();
         k_fill_i32<<<nblk(n), kBlock, 0, stream>>>(pint.as<int>(), n, -1);
-        k_fill_i32<<<nblk(n), kBlock, 0, stream>>>(flags.as<int>(), n, 0);
         k_karras<<<nblk(n - 1), kBlock, 0, stream>>>(sk, n, left.as<int>(), right.as<int>(), first.as<int>(),
                                                      last.as<int>(), pint.as<int>(), pleaf.as<int>());
-        k_refit<<<nblk(n), kBlock, 0, stream>>>(sk, n, boxes.as<Box6>(), left.as<int>(), right.as<int>(), pint.as<int>(),
-                                                pleaf.as<int>(), flags.as<int>(), ibox.as<Box6>());
+        if ((st = node_boxes(sk)) != RTG_OK) return st;
         // emitted internal nodes: prefix sum of (count > kLeafMax)
         k_emit_flags<<<nblk(n - 1), kBlock, 0, stream>>>(first.as<int>(), last.as<int>(), n - 1, flags.as<int>());
         tmp_bytes = 0;
@@ -384,7 +498,7 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
         RTG_HIP(hipMemcpyAsync(&last_flag, flags.as<int>() + (n - 2), sizeof(int), hipMemcpyDeviceToHost, stream));
         RTG_HIP(hipStreamSynchronize(stream));
         n_emit = last_new + last_flag;
-        k_top_first<<<1, 1, 0, stream>>>(left.as<int>(), right.as<int>(), first.as<int>(), last.as<int>(), n - 1,
+        k_top_first<<<1, 64, 0, stream>>>(left.as<int>(), right.as<int>(), first.as<int>(), last.as<int>(), n - 1,
                                          newidx.as<int>());
         if (ensure(nodes2, std::max(n_emit, 1) * sizeof(BvhNode))) return fail(RTG_E_NOMEM, "bvh nodes");
         k_emit<<<nblk(n - 1), kBlock, 0, stream>>>(sk, n - 1, boxes.as<Box6>(), left.as<int>(), right.as<int>(),
