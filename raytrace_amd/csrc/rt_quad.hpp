@@ -54,10 +54,12 @@ __device__ inline float quad_min(float v) {
     return fminf(v, quad_xor<2>(v));
 }
 
-// One stack per quad: its four lanes' LDS columns side by side (64 entries),
-// the rest in the first lane's spill column.  An entry is written by the lane
-// that holds the child and read by all four; a wave's accesses to LDS, and to
-// one global address, are done in order, and the fences keep the compiler from
+// One stack per quad, in the stack memory of its own four lanes and no other
+// (waves of a block may walk rays by quads and by lanes at the same time):
+// entry e in row e / 4, column e % 4 of their LDS columns, 64 entries; the
+// rest in the first lane's spill column.  An entry is written by the lane that
+// holds the child and read by all four; a wave's accesses to LDS, and to one
+// global address, are done in order, and the fences keep the compiler from
 // moving them.
 struct QuadStack {
     int *lds;
@@ -66,21 +68,21 @@ struct QuadStack {
     int sp;
     const Bvh4Node *top;
     static constexpr int kLds = kLdsStack * kQuadLanes;
-    static constexpr int kQuads = kBlockThreads / kQuadLanes;  // quads of a block: the LDS stride
     __device__ explicit QuadStack(const DevStack &st, int *lds_base)
-        : lds(lds_base + (threadIdx.x / kQuadLanes)), spill(st.spill - (threadIdx.x & (kQuadLanes - 1))),
+        : lds(lds_base + (threadIdx.x & ~(kQuadLanes - 1))), spill(st.spill - (threadIdx.x & (kQuadLanes - 1))),
           gstride(st.gstride), sp(0), top(st.top) {}
     __device__ static void order() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+    static __device__ int at(int e) { return (e / kQuadLanes) * kBlockThreads + (e & (kQuadLanes - 1)); }
     // This lane's child takes entry e.
     __device__ void put(int e, int v) {
 #if defined(__HIP_DEVICE_COMPILE__)
         typedef int __attribute__((address_space(3))) LdsInt;
         if (e < kLds)
-            ((LdsInt *)lds)[e * kQuads] = v;
+            ((LdsInt *)lds)[at(e)] = v;
         else
             spill[(e - kLds) * gstride] = v;
 #endif
@@ -92,7 +94,7 @@ struct QuadStack {
 #if defined(__HIP_DEVICE_COMPILE__)
         typedef const int __attribute__((address_space(3))) LdsInt;
         if (sp < kLds) {
-            v = ((LdsInt *)lds)[sp * kQuads];
+            v = ((LdsInt *)lds)[at(sp)];
             __asm__ volatile("" ::: "memory");  // not merged with the spill read into a flat load
         } else {
             v = spill[(sp - kLds) * gstride];

@@ -600,6 +600,22 @@ __global__ __launch_bounds__(kBlockThreads, 8) void k_occlude(SceneView S0, Wave
     }
 }
 
+// Local lighting of node i from its light mask, over its texel colour.
+template <bool B>
+__device__ inline V3 light_node(const SceneView &S0, const WaveArgs &A, const WNode &nd, unsigned mask) {
+    const SceneView &S = scene_at<B>(S0, A, req_at<B>(A, node_req(nd)).scene);
+    return shade_local(S, V3{nd.dx, nd.dy, nd.dz}, V3{nd.px, nd.py, nd.pz}, V3{nd.nx, nd.ny, nd.nz}, node_mtl(nd),
+                       V3{nd.vr, nd.vg, nd.vb},
+                       [&](int li, const LightTerm &, bool) -> bool { return (mask >> li) & 1u; });
+}
+template <bool B>
+__device__ inline void light_in_place(const SceneView &S0, const WaveArgs &A, WNode *nodes, const unsigned *masks,
+                                      int i) {
+    if (!((nodes[i].bits >> 27) & 1)) return;
+    const V3 L = light_node<B>(S0, A, nodes[i], masks[i]);
+    nodes[i].vr = L.x, nodes[i].vg = L.y, nodes[i].vb = L.z;
+}
+
 template <bool B>
 __global__ __launch_bounds__(kBlockThreads, 8) void k_local(SceneView S0, WaveArgs A, int k, const unsigned *n_ptr,
                                                          WNode *nodes, const unsigned *masks) {
@@ -608,15 +624,129 @@ __global__ __launch_bounds__(kBlockThreads, 8) void k_local(SceneView S0, WaveAr
     const ChunkRange cr = xcd_chunks((n + kBlockThreads - 1) / kBlockThreads);
     for (int c = cr.first; c < cr.end; c += cr.step) {
         const int i = c * kBlockThreads + threadIdx.x;
-        if (i >= n || !((nodes[i].bits >> 27) & 1)) continue;
-        const WNode nd = nodes[i];
-        const WaveReq &R = req_at<B>(A, node_req(nd));
-        const SceneView &S = scene_at<B>(S0, A, R.scene);
-        const unsigned mask = masks[i];
-        const V3 L = shade_local(S, V3{nd.dx, nd.dy, nd.dz}, V3{nd.px, nd.py, nd.pz}, V3{nd.nx, nd.ny, nd.nz},
-                                 node_mtl(nd), V3{nd.vr, nd.vg, nd.vb},
-                                 [&](int li, const LightTerm &, bool) -> bool { return (mask >> li) & 1u; });
-        nodes[i].vr = L.x, nodes[i].vg = L.y, nodes[i].vb = L.z;
+        if (i < n) light_in_place<B>(S0, A, nodes, masks, i);
+    }
+}
+
+// One level of a batch in one launch: the closest hits of level k + 1, the
+// shadow tests of level k and the local lighting of level k - 1, each of which
+// needs only what earlier launches wrote.  A wave takes rays while there are
+// any, then shadow entries, then nodes, so that one kind's tail is filled by
+// the next.  In place of k_extend beside k_occlude on a side stream (12
+// thumbnails 2027 -> 1607 us a batch, burst of 32 requests 2992 -> 2614, 60
+// mixed requests 6283 -> 6042).
+struct StepArgs {
+    int k;  // level of `rays`
+    const WRay *rays;  // null: no rays
+    const unsigned *n_rays;
+    WHit *hits;
+    int4 *cs;
+    LineCtr *sched;
+    const WNode *nodes;  // shadow tests
+    const unsigned *shadow;
+    LevelCtr *ctr;
+    unsigned *masks;
+    WNode *lit;  // nodes to light; null: none
+    const unsigned *n_lit;  // null: level 0
+    const unsigned *lit_masks;
+};
+__global__ __launch_bounds__(kBlockThreads, 6) void k_step(WaveArgs A, StepArgs T) {
+    const SceneView S0{};  // (batches: every ray's scene is in A.scenes)
+    const int n = T.rays ? (int)*T.n_rays : 0, ns = (int)T.ctr->n_shadow.v;
+    const int nl = T.lit ? (T.n_lit ? (int)*T.n_lit : A.n_samples) : 0;
+    const bool qe = n <= A.quad_max, qo = ns <= A.quad_max;
+    const int ce = qe ? (n + 15) >> 4 : (n + 63) >> 6, co = qo ? (ns + 15) >> 4 : (ns + 63) >> 6;
+    const int b2 = (int)blockIdx.x * (kBlockThreads / 64);  // waves before this block's
+    const int cl = (nl + kBlockThreads - 1) / kBlockThreads;
+    if (b2 >= ce + co && (int)blockIdx.x >= cl) return;
+    __shared__ int lds[kLdsStack * kBlockThreads];
+    DevStack st = make_stack(lds, A.spill);
+    if (b2 < ce) {
+        if (qe) {
+            QuadStack qs(st, lds);
+            extend_rays<true, false, true>(S0, A, T.k, T.rays, n, T.hits, T.cs, T.sched, qs);
+        } else {
+            extend_rays<true, false, false>(S0, A, T.k, T.rays, n, T.hits, T.cs, T.sched, st);
+        }
+    }
+    if (b2 < ce + co && ns > 0) {
+        if (qo) {
+            QuadStack qs(st, lds);
+            occlude_entries<true, true>(S0, A, T.nodes, T.shadow, ns, T.ctr->sched[2], T.masks, qs);
+        } else {
+            occlude_entries<true, false>(S0, A, T.nodes, T.shadow, ns, T.ctr->sched[2], T.masks, st);
+        }
+    }
+    for (int c = blockIdx.x; c < cl; c += gridDim.x) {
+        const int i = c * kBlockThreads + threadIdx.x;
+        if (i < nl) light_in_place<true>(S0, A, T.lit, T.lit_masks, i);
+    }
+}
+
+// The colour of level-0 sample i: the pixel at one sample per pixel (the box
+// filter of one sample is that sample, quantised), else its sample slot.
+template <bool B>
+__device__ inline void put_sample(const WaveArgs &A, int i, float4 out, float4 *samples) {
+    const int r = sample_req<B>(A, i);
+    const WaveReq &R = req_at<B>(A, r < 0 ? 0 : r);
+    if (R.spp != 1) {
+        samples[i] = out;
+        return;
+    }
+    int px, py, si;
+    if (r >= 0 && sample_pixel(R, i - R.sample_base, px, py, si)) {
+        uint8_t *p = R.rgb + 3 * ((size_t)py * R.W + px);
+        p[0] = quantize(out.x), p[1] = quantize(out.y), p[2] = quantize(out.z);
+    }
+}
+
+// Colours of every level in one launch, where no hit spawns two rays: a ray's
+// colour goes into one parent and no other, so the thread of a chain's last
+// node (a miss, or a hit with no child traced) walks its links up to level 0.
+// In place of k_combine level by level, whose launches wait for one another
+// and hand the colours on through memory (1080p frame 2033 -> 1993 us, 640x480
+// 645 -> 600 us).  Grid y: the level of the chains' last nodes.
+struct ChainLevel {
+    const WRay *rays;
+    const unsigned *n;  // null: level 0
+    const WNode *nodes;
+    const unsigned *masks;
+    int lit;  // k_local or k_step lit the level's nodes
+};
+struct ChainArgs {
+    ChainLevel lv[Workspace::kLevels];
+};
+template <bool B>
+__global__ __launch_bounds__(kBlockThreads, 8) void k_chain(SceneView S0, WaveArgs A, ChainArgs T, float4 *samples) {
+    if (A.cancel != nullptr && *(volatile unsigned *)A.abort != 0) return;
+    const float4 none = make_float4(0.0f, 0.0f, 0.0f, kMiss);  // no child: black, no Beer factor
+    const int k0 = blockIdx.y;
+    const int n = T.lv[k0].n ? (int)*T.lv[k0].n : A.n_samples;
+    const ChunkRange cr = xcd_chunks((n + kBlockThreads - 1) / kBlockThreads);
+    for (int c = cr.first; c < cr.end; c += cr.step) {
+        int i = c * kBlockThreads + threadIdx.x;
+        if (i >= n) continue;
+        unsigned bits = (unsigned)T.lv[k0].nodes[i].bits;
+        if ((bits >> 27 & 1) && bits >> 30) continue;  // its child's chain passes through it
+        float4 out = none, a = none, b = none;
+        for (int k = k0;; --k) {
+            const ChainLevel &L = T.lv[k];
+            if (bits >> 27 & 1) {
+                const WNode nd = L.nodes[i];
+                const WaveReq &R = req_at<B>(A, node_req(nd));
+                const DevMaterial &m = scene_at<B>(S0, A, R.scene).mtls[node_mtl(nd)];
+                const V3 l = L.lit ? V3{nd.vr, nd.vg, nd.vb} : light_node<B>(S0, A, nd, L.masks[i]);
+                const V3 col = compose(l, m.reflect, R.no_refract ? 0.0f : m.refract, (nd.bits >> 29) & 1,
+                                       (nd.bits >> 28) & 1, m.kd, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, b.w);
+                out = make_float4(col.x, col.y, col.z, nd.t);
+            }
+            if (k == 0) break;
+            const int link = L.rays[i].link;
+            a = link & 1 ? none : out, b = link & 1 ? out : none;
+            i = link >> 1;
+            bits = 1u << 27;  // a parent is a hit
+        }
+        put_sample<B>(A, i, out, samples);
     }
 }
 
@@ -647,12 +777,7 @@ __global__ __launch_bounds__(kBlockThreads, 8) void k_combine(SceneView S0, Wave
             const WaveReq &R = req_at<B>(A, node_req(nd));
             const SceneView &S = scene_at<B>(S0, A, R.scene);
             const int mtl = node_mtl(nd);
-            V3 L = V3{nd.vr, nd.vg, nd.vb};
-            if (!local) {
-                const unsigned mask = masks[i];
-                L = shade_local(S, V3{nd.dx, nd.dy, nd.dz}, V3{nd.px, nd.py, nd.pz}, V3{nd.nx, nd.ny, nd.nz}, mtl,
-                                L, [&](int li, const LightTerm &, bool) -> bool { return (mask >> li) & 1u; });
-            }
+            const V3 L = local ? V3{nd.vr, nd.vg, nd.vb} : light_node<B>(S0, A, nd, masks[i]);
             const DevMaterial &m = S.mtls[mtl];
             const float4 none = make_float4(0.0f, 0.0f, 0.0f, kMiss);  // no child: black, no Beer factor
             const float4 a = (nd.bits >> 30) & 1 ? slots[2 * i] : none;
@@ -661,21 +786,10 @@ __global__ __launch_bounds__(kBlockThreads, 8) void k_combine(SceneView S0, Wave
                                    (nd.bits >> 28) & 1, m.kd, V3{a.x, a.y, a.z}, V3{b.x, b.y, b.z}, b.w);
             out = make_float4(col.x, col.y, col.z, nd.t);
         }
-        if (k != 0) {
+        if (k != 0)
             parent_slots[rays[i].link] = out;
-            continue;
-        }
-        const int r = sample_req<B>(A, i);
-        const WaveReq &Rq = req_at<B>(A, r < 0 ? 0 : r);
-        if (Rq.spp != 1) {
-            samples[i] = out;
-            continue;
-        }
-        int px, py, si;
-        if (r >= 0 && sample_pixel(Rq, i - Rq.sample_base, px, py, si)) {
-            uint8_t *p = Rq.rgb + 3 * ((size_t)py * Rq.W + px);
-            p[0] = quantize(out.x), p[1] = quantize(out.y), p[2] = quantize(out.z);
-        }
+        else
+            put_sample<B>(A, i, out, samples);
     }
 }
 
@@ -920,12 +1034,20 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         if (ws.grow(ws.w_qcount, (size_t)kPassCtrWords * sizeof(unsigned)))
             return fail(RTG_E_NOMEM, "queue counters");
     }
+    // Batches run a level's rays beside the shadow rays of the level before in
+    // one launch (k_step): a captured batch graph put the two streams' kernels
+    // on queues where they waited for one another.  Single frames keep the
+    // side streams (with k_step 64x64 215 -> 227 us, 320x180 3709 -> 3890 us
+    // for three edits, 1080p 1993 -> 2397 us), and so do the FP64 re-test,
+    // which has a kernel of its own, and levels sized by read-backs.
+    const bool fused = B && pl.no_sync && !retest && shadows;
+    const bool chain = pl.fanout <= 1 && !view;
     // The shadow rays of level k (k_occlude) depend only on
     // k_shade(k), and level k + 1 does not depend on them: with `overlap`
     // they run on the workspace's side stream, concurrently with the next
     // level, and join the render stream before k_combine (the last level's
     // stay on the render stream, see below).
-    const bool ov = overlap && shadows;
+    const bool ov = overlap && shadows && !fused;
     if (ov) {
         int st = ws.side_init();
         if (st != RTG_OK) return st;
@@ -979,6 +1101,26 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     size_t n_k = (size_t)pl.n_samples;
     size_t counted[Workspace::kLevels] = {};  // rays of each level, as far as the host knows
     int last = -1;
+    // nodes of level k are lit before the colours are composed
+    auto lit = [&](int k) { return fused ? k < last : early_local && k < pl.max_level; };
+    // k_step for the rays of level k (if `rays`), the shadow tests of level
+    // k - 1 and the lighting of level k - 2
+    auto step = [&](int k, bool rays) {
+        StepArgs t{};
+        t.k = k;
+        if (rays) {
+            t.rays = ws.w_rays[k].as<WRay>(), t.n_rays = &ctr[k - 1].n_next.v;
+            t.hits = ws.w_hits[k].as<WHit>(), t.cs = ws.w_cs[k].as<int4>(), t.sched = ctr[k].sched[0];
+        }
+        t.nodes = ws.w_nodes[k - 1].as<WNode>(), t.shadow = ws.w_shadow[k - 1].as<unsigned>();
+        t.ctr = ctr + (k - 1), t.masks = ws.w_masks[k - 1].as<unsigned>();
+        if (k >= 2) {
+            t.lit = ws.w_nodes[k - 2].as<WNode>(), t.lit_masks = ws.w_masks[k - 2].as<unsigned>();
+            t.n_lit = k == 2 ? nullptr : &ctr[k - 3].n_next.v;
+        }
+        const size_t items = kQuadLanes * ((rays ? pl.bound[k] : 0) + pl.bound[k - 1] * pl.n_on);
+        k_step<<<grid(g.extend, items), kBlockThreads, 0, stream>>>(args, t);
+    };
     const size_t cap = level_ray_cap(pl.n_on);
     for (int k = 0; k <= pl.max_level && n_k > 0; ++k) {
         if (cancel_host && *cancel_host) return join();
@@ -998,7 +1140,9 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         const unsigned *n_ptr = k == 0 ? nullptr : &ctr[k - 1].n_next.v;
         WRay *next = ws.w_rays[k + 1 < Workspace::kLevels ? k + 1 : k].as<WRay>();
         int kt = ktime_begin(A, stream, KT_EXTEND, n_k);
-        if (retest)
+        if (fused && k > 0)
+            step(k, true);
+        else if (retest)
             k_extend<B, true><<<grid(g.extend, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         else
@@ -1023,7 +1167,9 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             RTG_HIP(hipStreamWaitEvent(sk, ws.ev_fork[k], 0));
             (second ? forked2 : forked) = true;
         }
-        if (shadows) {
+        if (fused) {
+            if (k == pl.max_level || pl.bound[k + 1] == 0) step(k + 1, false);
+        } else if (shadows) {
             kt = ktime_begin(A, sk, KT_OCCLUDE, 0);
             k_occlude<B><<<grid(side_k ? g.occlude : g.occlude_alone, kQuadLanes * n_k * pl.n_on), kBlockThreads, 0, sk>>>(
                 S0, side_k ? (second ? oargs2 : oargs) : args, ws.w_nodes[k].as<WNode>(),
@@ -1036,7 +1182,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         // frames with every level enqueued at once only: where levels wait for
         // host read-backs (many lights, deep trees) the extra side work ended
         // up on the frame's path (measured).
-        if (early_local && k < pl.max_level) {
+        if (early_local && !fused && k < pl.max_level) {
             kt = ktime_begin(A, sk, KT_LOCAL, 0);
             k_local<B><<<lgrid(n_k), kBlockThreads, 0, sk>>>(S0, args, k, n_ptr, ws.w_nodes[k].as<WNode>(),
                                                           ws.w_masks[k].as<unsigned>());
@@ -1067,14 +1213,26 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             S0, args, mode, ws.w_hits[0].as<WHit>(), ws.w_masks[0].as<unsigned>(), ws.w_samples.as<float4>());
         ktime_end(A, stream, kt);
     }
-    for (int k = view ? -1 : last; k >= 0; --k) {
+    if (chain && last >= 0) {
+        ChainArgs t{};
+        size_t most = 0;
+        for (int k = 0; k <= last; ++k) {
+            t.lv[k] = ChainLevel{k == 0 ? nullptr : ws.w_rays[k].as<WRay>(), k == 0 ? nullptr : &ctr[k - 1].n_next.v,
+                                 ws.w_nodes[k].as<WNode>(), ws.w_masks[k].as<unsigned>(), lit(k) ? 1 : 0};
+            most = std::max(most, counted[k]);
+        }
+        const int kt = ktime_begin(A, stream, KT_COMBINE, (uint64_t)pl.n_samples);
+        k_chain<B><<<dim3(lgrid(most), last + 1), kBlockThreads, 0, stream>>>(S0, args, t, ws.w_samples.as<float4>());
+        ktime_end(A, stream, kt);
+    }
+    for (int k = view || chain ? -1 : last; k >= 0; --k) {
         const WRay *rays = k == 0 ? nullptr : ws.w_rays[k].as<WRay>();
         const unsigned *n_ptr = k == 0 ? nullptr : &ctr[k - 1].n_next.v;
         const int kt = ktime_begin(A, stream, KT_COMBINE, k == 0 ? (uint64_t)pl.n_samples : 0);
         k_combine<B><<<lgrid(counted[k]), kBlockThreads, 0, stream>>>(
             S0, args, k, rays, n_ptr, ws.w_nodes[k].as<WNode>(), ws.w_masks[k].as<unsigned>(),
             ws.w_slots[k].as<float4>(), k > 0 ? ws.w_slots[k - 1].as<float4>() : nullptr,
-            ws.w_samples.as<float4>(), early_local && k < pl.max_level ? 1 : 0);
+            ws.w_samples.as<float4>(), lit(k) ? 1 : 0);
         ktime_end(A, stream, kt, n_ptr);
     }
     if (B || a.r0.spp != 1) {  // a single frame at one sample per pixel is written by k_combine
