@@ -76,7 +76,7 @@ struct QuadStack {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    static __device__ int at(int e) { return (e / kQuadLanes) * kBlockThreads + (e & (kQuadLanes - 1)); }
+    static __device__ unsigned at(unsigned e) { return (e / kQuadLanes) * kBlockThreads + e % kQuadLanes; }
     // This lane's child takes entry e.
     __device__ void put(int e, int v) {
 #if defined(__HIP_DEVICE_COMPILE__)

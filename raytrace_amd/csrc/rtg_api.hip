@@ -38,16 +38,19 @@ uint64_t hash_bytes(uint64_t h, const void *p, size_t n) {
     return mix64(lanes[0] ^ mix64(lanes[1] ^ mix64(lanes[2] ^ mix64(lanes[3] ^ t))));
 }
 
-// Hash of everything the BVH depends on.
-uint64_t geometry_hash(const rtg_scene_desc &d) {
-    uint64_t h = hash_bytes(0, d.objects, sizeof(rtg_object) * (size_t)d.n_objects);
-    for (int i = 0; i < d.n_parts; ++i) {
+// Hash of everything the BVH depends on: each part's on the pool's threads,
+// then all of them in order.
+uint64_t geometry_hash(const rtg_scene_desc &d, HostPool &pool) {
+    std::vector<uint64_t> parts(d.n_parts);
+    pool.run(d.n_parts, [&](int i) {
         const rtg_part &p = d.parts[i];
-        h = hash_bytes(h, &p.tri_count, sizeof(int32_t) * 2);
+        uint64_t h = hash_bytes((uint64_t)i, &p.tri_count, sizeof(int32_t) * 2);
         h = hash_bytes(h, &p.bmin, sizeof(rtg_vec4) * 2);
         if (p.tris && p.tri_count > 0) h = hash_bytes(h, p.tris, sizeof(rtg_triangle) * (size_t)p.tri_count);
-    }
-    return h;
+        parts[i] = h;
+    });
+    const uint64_t h = hash_bytes(0, d.objects, sizeof(rtg_object) * (size_t)d.n_objects);
+    return hash_bytes(h, parts.data(), parts.size() * sizeof(uint64_t));
 }
 
 // Primitive set and order of a scene (what a BVH topology depends on): each
@@ -331,7 +334,7 @@ int rtg_scene_create(const rtg_scene_desc *desc, rtg_scene_t *out) {
         st = scene_build(s->res, *desc, A.stream);
     }
     if (st != RTG_OK) return st;
-    s->res.geom_hash = geometry_hash(*desc);
+    s->res.geom_hash = geometry_hash(*desc, A.pool);
     s->res.topo_hash = topology_hash(*desc);
     *out = s.release();
     return RTG_OK;
@@ -349,7 +352,7 @@ static int scene_update(rtg_scene_t scene, const rtg_scene_desc *desc, bool allo
     std::lock_guard<std::mutex> l(A.lock);
     // Same geometry (objects, parts, triangles): only materials, lights,
     // textures and the camera can have changed, so the BVH stays.
-    const uint64_t gh = geometry_hash(*desc), th = topology_hash(*desc);
+    const uint64_t gh = geometry_hash(*desc, A.pool), th = topology_hash(*desc);
     SceneRes &R = scene->res;
     if (allow_refit && R.geom_hash != 0 && gh == R.geom_hash) {
         ++R.shading_updates;
@@ -438,38 +441,78 @@ static int ensure_pinned_out(Arena &A, size_t bytes) {
     return RTG_OK;
 }
 
-// Run copy(i) for i in [0, n) on up to 8 host threads (the calling thread
-// included); one thread if no more can be started.
-extern "C++" template <class F>
-static void parallel_copies(int n, F &&copy) {
-    std::atomic<int> next{0};
-    auto work = [&]() {
-        for (int i = next++; i < n; i = next++) copy(i);
-    };
-    const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    const int nt = std::max(1, std::min({8, n, (int)hw}));
-    std::vector<std::thread> pool;
-    try {
-        for (int k = 1; k < nt; ++k) pool.emplace_back(work);
-    } catch (...) {
-        // fewer threads: the ones started and this one finish the work
-    }
-    work();
-    for (std::thread &t : pool) t.join();
-}
-
 }  // extern "C"
 
 namespace rtg {
-void copy_out(const HostCopy *cp, int n) {
-    constexpr size_t kPiece = size_t(1) << 20;
+
+HostPool::~HostPool() {
+    {
+        std::lock_guard<std::mutex> l(m);
+        stop_ = true;
+    }
+    work.notify_all();
+    for (std::thread &t : threads) t.join();
+}
+
+void HostPool::worker() {
+    std::unique_lock<std::mutex> l(m);
+    for (;;) {
+        work.wait(l, [&]() { return stop_ || next_ < n_; });
+        if (stop_) return;
+        const int i = next_++;
+        ++running_;
+        l.unlock();
+        piece_(ctx_, i);
+        l.lock();
+        if (--running_ == 0 && next_ >= n_) idle.notify_one();
+    }
+}
+
+void HostPool::run_pieces(int n, void (*piece)(void *, int), void *ctx) {
+    std::unique_lock<std::mutex> job(one_job, std::try_to_lock);
+    if (n <= 1 || !job.owns_lock()) {
+        for (int i = 0; i < n; ++i) piece(ctx, i);
+        return;
+    }
+    std::unique_lock<std::mutex> l(m);
+    const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
+    try {
+        while ((int)threads.size() < std::min({7, n - 1, hw - 1})) threads.emplace_back([this]() { worker(); });
+    } catch (...) {
+        // fewer threads: the ones started and this one do the pieces
+    }
+    piece_ = piece, ctx_ = ctx, n_ = n, next_ = 0;
+    l.unlock();
+    for (int k = 0; k < std::min(n - 1, (int)threads.size()); ++k) work.notify_one();
+    l.lock();
+    while (next_ < n_) {
+        const int i = next_++;
+        l.unlock();
+        piece(ctx, i);
+        l.lock();
+    }
+    idle.wait(l, [&]() { return running_ == 0; });
+    n_ = next_ = 0;
+}
+
+void copy_out(HostPool &pool, const HostCopy *cp, int n) {
+    constexpr size_t kPiece = size_t(256) << 10;
     std::vector<HostCopy> pieces;
-    for (int i = 0; i < n; ++i)
+    size_t total = 0;
+    for (int i = 0; i < n; ++i) {
+        total += cp[i].bytes;
         for (size_t off = 0; off < cp[i].bytes; off += kPiece)
             pieces.push_back(HostCopy{static_cast<uint8_t *>(cp[i].dst) + off, cp[i].src + off,
                                       std::min(kPiece, cp[i].bytes - off)});
-    parallel_copies((int)pieces.size(), [&](int k) { std::memcpy(pieces[k].dst, pieces[k].src, pieces[k].bytes); });
+    }
+    auto copy = [&](int k) { std::memcpy(pieces[k].dst, pieces[k].src, pieces[k].bytes); };
+    if (total <= 2 * kPiece) {  // less than waking the threads costs
+        for (int k = 0; k < (int)pieces.size(); ++k) copy(k);
+        return;
+    }
+    pool.run((int)pieces.size(), copy);
 }
+
 }  // namespace rtg
 
 extern "C" {
@@ -534,7 +577,7 @@ static int render_host(rtg_scene_t scene, const rtg_params *params, uint8_t *rgb
     if (pst == RTG_OK) {
         const HostCopy cp[3] = {{rgb, A.pinned_out, b_rgb}, {ids, A.pinned_out + o_ids, b_ids},
                                 {tprim, A.pinned_out + o_t, b_t}};
-        copy_out(cp, 3);
+        copy_out(A.pool, cp, 3);
     }
     flag.release();
     const bool cancelled = flag.seen;
@@ -743,7 +786,7 @@ int rtg_render_batch(const rtg_request *reqs, int n, rtg_stats *stats) {
         cp.push_back(HostCopy{reqs[i].rgb, A.pinned_out + off_rgb[i], npix * 3});
         if (reqs[i].ids) cp.push_back(HostCopy{reqs[i].ids, A.pinned_out + rgb_bytes + off_ids[i], npix * 8});
     }
-    copy_out(cp.data(), (int)cp.size());
+    copy_out(A.pool, cp.data(), (int)cp.size());
     float ms = 0;
     RTG_HIP(hipEventElapsedTime(&ms, A.ev0, A.ev1));
     if (stats) {

@@ -8,6 +8,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/rtg.h"
@@ -130,6 +131,39 @@ struct Tuning {
     uint64_t key() const { return (uint64_t)tile_lg | ((uint64_t)grab_lg << 4) | ((uint64_t)grid_pct << 8); }
 };
 
+// Host threads that run the pieces of a job beside the calling thread: at most
+// seven, started at the first job that needs them, kept until rtg_shutdown.
+// (Starting and joining up to seven threads on every call cost 100 us and
+// more.)  A job that finds the pool busy runs on its caller alone.
+class HostPool {
+public:
+    // f(i) for every i in [0, n), in any order and on any of the threads;
+    // returns when all are done.  f must not throw.
+    template <class F>
+    void run(int n, F &&f) {
+        struct Call {
+            static void piece(void *ctx, int i) { (*static_cast<std::remove_reference_t<F> *>(ctx))(i); }
+        };
+        run_pieces(n, &Call::piece, &f);
+    }
+    HostPool() = default;
+    HostPool(const HostPool &) = delete;
+    HostPool &operator=(const HostPool &) = delete;
+    ~HostPool();
+
+private:
+    void run_pieces(int n, void (*piece)(void *, int), void *ctx);
+    void worker();
+    std::mutex one_job;  // held by the caller whose job the pool runs
+    std::mutex m;        // guards what follows
+    std::condition_variable work, idle;
+    std::vector<std::thread> threads;
+    void (*piece_)(void *, int) = nullptr;
+    void *ctx_ = nullptr;
+    int n_ = 0, next_ = 0, running_ = 0;
+    bool stop_ = false;
+};
+
 struct Arena {
     static constexpr int kLevels = Workspace::kLevels;
     Tuning tune;
@@ -165,6 +199,7 @@ struct Arena {
     int kitems_next = 0;
     static constexpr int kItemSlots = 4096;
     std::mutex lock;  // one render at a time on the arena
+    HostPool pool;    // copies of results, hashes of scenes
 };
 
 enum KernelKind { KT_EXTEND, KT_SHADE, KT_OCCLUDE, KT_COMBINE, KT_RESOLVE, KT_MEGA, KT_LOCAL, KT_COUNT };
@@ -261,14 +296,14 @@ int write_raygen_tables(float *tab, int W, int H, double dp, hipStream_t stream)
 int noalloc_setup(int device);
 // Launch one frame of the wavefront engine on `stream` (asynchronous) with
 // the buffers of `ws`; `cancel` may be null.
-// Host copies of device results staged in pinned memory, run on up to 8
-// host threads in pieces of at most 1 MB.
+// Host copies of device results staged in pinned memory, in pieces on the
+// pool's threads.
 struct HostCopy {
     void *dst;
     const uint8_t *src;
     size_t bytes;
 };
-void copy_out(const HostCopy *cp, int n);
+void copy_out(HostPool &pool, const HostCopy *cp, int n);
 
 // Grow `ws` to what one W x H frame of the given depth, fanout and lights
 // reserves before it launches (nothing is allocated while it renders).

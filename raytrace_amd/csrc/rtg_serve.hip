@@ -238,7 +238,7 @@ int serve_run(rtg_serve_request *reqs, int n, const rtg_serve_opts &o, rtg_serve
             for (size_t j = 0; j < s.reqs.size(); ++j)
                 cp[j] = HostCopy{reqs[s.reqs[j]].rgb, s.pinned + s.offs[j],
                                  (size_t)info[s.reqs[j]].W * info[s.reqs[j]].H * 3};
-            copy_out(cp.data(), (int)cp.size());
+            copy_out(A.pool, cp.data(), (int)cp.size());
             const double t = since(t0);
             for (int id : s.reqs) {
                 reqs[id].done_s = t;
