@@ -101,20 +101,51 @@ int resolve_size(const SceneRes &S, const rtg_params *p, int &W, int &H) {
     return RTG_OK;
 }
 
+void *BlockCache::take(size_t n, size_t &cap) {
+    std::lock_guard<std::mutex> l(m);
+    const auto it = blocks.lower_bound(n);
+    if (it == blocks.end() || it->first > n + n / 4) return nullptr;
+    void *const p = it->second;
+    cap = it->first;
+    total -= it->first;
+    blocks.erase(it);
+    return p;
+}
+bool BlockCache::keep(void *p, size_t cap) {
+    std::lock_guard<std::mutex> l(m);
+    if (total + cap > kMost) return false;
+    blocks.emplace(cap, p);
+    total += cap;
+    return true;
+}
+void BlockCache::clear() {
+    std::lock_guard<std::mutex> l(m);
+    for (const auto &b : blocks) (void)hipFree(b.second);
+    blocks.clear();
+    total = 0;
+}
+
 int DevBuf::alloc(size_t n) {
+    if (p != nullptr && reuse) (void)hipDeviceSynchronize();  // renders may still read the old block
     release();
     if (n == 0) n = 16;
-    if (hipMalloc(&p, n) != hipSuccess) {
-        p = nullptr;
-        return RTG_E_NOMEM;
+    BlockCache *const cache = g_arena ? &g_arena->blocks : nullptr;
+    cap = n;
+    if (reuse && cache) p = cache->take(n, cap);
+    if (p == nullptr && hipMalloc(&p, n) != hipSuccess) {
+        if (cache) cache->clear();  // kept blocks make room
+        if (hipMalloc(&p, n) != hipSuccess) {
+            p = nullptr;
+            return RTG_E_NOMEM;
+        }
     }
     bytes = n;
     return RTG_OK;
 }
 void DevBuf::release() {
-    if (p != nullptr) (void)hipFree(p);
+    if (p != nullptr && !(reuse && g_arena && g_arena->blocks.keep(p, cap))) (void)hipFree(p);
     p = nullptr;
-    bytes = 0;
+    bytes = cap = 0;
 }
 int ensure(DevBuf &b, size_t n) {
     if (b.p != nullptr && b.bytes >= n) return RTG_OK;
@@ -304,6 +335,7 @@ int rtg_shutdown(void) {
         A.out_t.release();
         (void)hipHostFree(A.cancel_host);
         if (A.kitems_host) (void)hipHostFree(A.kitems_host);
+        A.blocks.clear();
         if (A.pinned_out) (void)hipHostFree(A.pinned_out);
         A.pinned_out = nullptr;
         A.pinned_out_bytes = 0;
@@ -363,7 +395,8 @@ static int scene_update(rtg_scene_t scene, const rtg_scene_desc *desc, bool allo
     fresh.device = A.device;
     st = scene_build(fresh, *desc, A.stream, refit ? &R : nullptr);
     if (st != RTG_OK) return st;
-    auto take = [](DevBuf &a, DevBuf &b) { std::swap(a.p, b.p), std::swap(a.bytes, b.bytes); };
+    RTG_HIP(hipDeviceSynchronize());  // frames on any stream may read the old arrays, released below
+    auto take = [](DevBuf &a, DevBuf &b) { a.swap(b); };
     take(R.nodes, fresh.nodes), take(R.prims, fresh.prims), take(R.objs, fresh.objs), take(R.brute, fresh.brute);
     take(R.parts, fresh.parts), take(R.tri_nrm, fresh.tri_nrm), take(R.tri_uv, fresh.tri_uv);
     take(R.tri_pos, fresh.tri_pos), take(R.tri_part, fresh.tri_part), take(R.tri_bins, fresh.tri_bins);
@@ -410,7 +443,7 @@ int rtg_scene_destroy(rtg_scene_t scene) {
     if (scene == nullptr) return RTG_OK;
     if (arena()) {
         std::lock_guard<std::mutex> l(arena()->lock);
-        (void)hipStreamSynchronize(arena()->stream);
+        (void)hipDeviceSynchronize();  // frames on any stream may read its arrays
     }
     delete scene;
     return RTG_OK;

@@ -304,10 +304,18 @@ int upload(DevBuf &b, const std::vector<T> &v, hipStream_t s) {
     return RTG_OK;
 }
 
+// Waits for the stream before the temporaries declared ahead of it are
+// released, on every path.
+struct SyncOnExit {
+    hipStream_t stream;
+    ~SyncOnExit() { (void)hipStreamSynchronize(stream); }
+};
+
 // The 4-wide tree of the n2 binary nodes in nodes2 (root 0) into S.nodes;
 // returns its node count in *n4.
 int widen_tree(const DevBuf &nodes2, int n2, SceneRes &S, hipStream_t stream, int *n4) {
-    DevBuf parent2, flags, idx4, scan_tmp;
+    SceneBuf parent2, flags, idx4, scan_tmp;
+    const SyncOnExit idle{stream};
     if (ensure(parent2, n2 * sizeof(int)) || ensure(flags, n2 * sizeof(int)) || ensure(idx4, n2 * sizeof(int)))
         return fail(RTG_E_NOMEM, "device allocation failed (4-wide nodes)");
     k_fill_i32<<<nblk(n2), kBlock, 0, stream>>>(parent2.as<int>(), n2, -1);
@@ -328,7 +336,6 @@ int widen_tree(const DevBuf &nodes2, int n2, SceneRes &S, hipStream_t stream, in
     k_widen<<<nblk(n2), kBlock, 0, stream>>>(nodes2.as<BvhNode>(), flags.as<int>(), idx4.as<int>(), n2,
                                              S.nodes.as<Bvh4Node>());
     RTG_HIP(hipGetLastError());
-    RTG_HIP(hipStreamSynchronize(stream));  // the temporaries are freed on return
     return RTG_OK;
 }
 
@@ -396,11 +403,12 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
         DevBuf *mine[] = {&S.t_keys, &S.t_left, &S.t_right, &S.t_first, &S.t_last, &S.t_pint, &S.t_pleaf, &S.t_newidx};
         DevBuf *theirs[] = {&donor->t_keys, &donor->t_left,  &donor->t_right, &donor->t_first,
                             &donor->t_last, &donor->t_pint, &donor->t_pleaf, &donor->t_newidx};
-        for (int k = 0; k < 8; ++k) std::swap(mine[k]->p, theirs[k]->p), std::swap(mine[k]->bytes, theirs[k]->bytes);
+        for (int k = 0; k < 8; ++k) mine[k]->swap(*theirs[k]);
         S.topo_n = donor->topo_n, S.topo_emit = donor->topo_emit;
         donor->topo_n = 0, donor->topo_emit = 0;
     }
-    DevBuf raw, mid, sph, prims_u, boxes, keys, flags, ibox, sbox, bbox, partial, cb, sort_tmp, nodes2;
+    SceneBuf raw, mid, sph, prims_u, boxes, keys, flags, ibox, sbox, bbox, partial, cb, sort_tmp, scan_tmp, nodes2;
+    const SyncOnExit idle{stream};
     DevBuf &keys2 = S.t_keys, &left = S.t_left, &right = S.t_right, &first = S.t_first, &last = S.t_last,
            &pint = S.t_pint, &pleaf = S.t_pleaf, &newidx = S.t_newidx;
     if ((st = upload(mid, part_mid, stream)) || (st = upload(sph, spheres, stream))) return st;
@@ -489,7 +497,6 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
         tmp_bytes = 0;
         RTG_HIP(rocprim::exclusive_scan(nullptr, tmp_bytes, flags.as<int>(), newidx.as<int>(), 0, (size_t)(n - 1),
                                         rocprim::plus<int>(), stream));
-        DevBuf scan_tmp;
         if (ensure(scan_tmp, std::max<size_t>(tmp_bytes, 16))) return fail(RTG_E_NOMEM, "scan temp");
         RTG_HIP(rocprim::exclusive_scan(scan_tmp.p, tmp_bytes, flags.as<int>(), newidx.as<int>(), 0, (size_t)(n - 1),
                                         rocprim::plus<int>(), stream));

@@ -3,8 +3,9 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
-#include <memory>
 #include <condition_variable>
+#include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -28,8 +29,13 @@ int fail(int code, const std::string &msg);
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
+    size_t cap = 0;       // size of the block behind it
+    bool reuse = false;   // its block comes from and returns to the arena's BlockCache
     int alloc(size_t n);  // RTG_OK / RTG_E_NOMEM
     void release();
+    void swap(DevBuf &o) {
+        std::swap(p, o.p), std::swap(bytes, o.bytes), std::swap(cap, o.cap), std::swap(reuse, o.reuse);
+    }
     ~DevBuf() { release(); }
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
@@ -38,9 +44,33 @@ struct DevBuf {
     T *as() const { return static_cast<T *>(p); }
 };
 
+// A scene's arrays and a build's temporaries: nothing on the GPU may still use
+// the block when it is released (hipFree would wait for the device; a cached
+// block is handed out again at once).
+struct SceneBuf : DevBuf {
+    SceneBuf() { reuse = true; }
+};
+
+// Device blocks of destroyed scenes and finished builds, kept for the next
+// ones: a scene takes some 40 allocations, and each hipFree waits for the
+// device.  At most kMost bytes are kept; rtg_shutdown frees them.
+class BlockCache {
+public:
+    static constexpr size_t kMost = size_t(512) << 20;
+    void *take(size_t n, size_t &cap);  // a kept block of n to 5/4 n bytes, or null
+    bool keep(void *p, size_t cap);     // false: not kept (the caller frees it)
+    void clear();
+    ~BlockCache() { clear(); }
+
+private:
+    std::mutex m;
+    std::multimap<size_t, void *> blocks;
+    size_t total = 0;
+};
+
 struct SceneRes {
     int device = 0;
-    DevBuf nodes, prims, objs, brute, parts, tri_nrm, tri_uv, tri_pos, tri_part, tri_mtl, tri_bins, mtls, lights, texs, texels;
+    SceneBuf nodes, prims, objs, brute, parts, tri_nrm, tri_uv, tri_pos, tri_part, tri_mtl, tri_bins, mtls, lights, texs, texels;
     SceneView view{};
     rtg_camera camera{};
     uint64_t geom_hash = 0;
@@ -56,7 +86,7 @@ struct SceneRes {
     // (primitive id in the low 32 bits), radix-tree children, leaf ranges,
     // parents and emitted-node indices of the Karras tree over topo_n
     // primitives; topo_hash identifies the primitive set and order.
-    DevBuf t_keys, t_left, t_right, t_first, t_last, t_pint, t_pleaf, t_newidx;
+    SceneBuf t_keys, t_left, t_right, t_first, t_last, t_pint, t_pleaf, t_newidx;
     int topo_n = 0, topo_emit = 0;
     uint64_t topo_hash = 0;
 };
@@ -200,6 +230,7 @@ struct Arena {
     static constexpr int kItemSlots = 4096;
     std::mutex lock;  // one render at a time on the arena
     HostPool pool;    // copies of results, hashes of scenes
+    BlockCache blocks;
 };
 
 enum KernelKind { KT_EXTEND, KT_SHADE, KT_OCCLUDE, KT_COMBINE, KT_RESOLVE, KT_MEGA, KT_LOCAL, KT_COUNT };
