@@ -205,9 +205,14 @@ __device__ inline Hit quad_closest(const SceneView &S, const TraceRay &q, QuadSt
     brute_objects(S, q, false, 0.0f, best, before);
     uint64_t bkey = best.kind != HIT_NONE ? hit_key(best.obj, best.prim) : ~0ull;
     float tmax = best.t;
+    int self = 0;  // 1 + slot of the source triangle, where the ray hits it
     quad_walk<true>(S, q.r, tmax, st, [&](int pi) -> bool {
         Hit h;
         if (!closest_prim(q, load_prim(S, pi), before, h)) return false;
+        if (h.kind == HIT_TRI && is_source_tri(q, h.obj, h.prim)) {
+            self = pi + 1;
+            return false;
+        }
         const uint64_t key = hit_key(h.obj, h.prim);
         if (h.t < best.t || (h.t == best.t && key < bkey)) best = h, bkey = key, tmax = fminf(tmax, h.t);
         return false;
@@ -225,6 +230,8 @@ __device__ inline Hit quad_closest(const SceneView &S, const TraceRay &q, QuadSt
     };
     from(std::integral_constant<int, 1>());
     from(std::integral_constant<int, 2>());
+    self = quad_or(self);  // one slot: the triangle is in one leaf
+    if (self) take_source_hit(S, q, self - 1, before, best, bkey);
     return best;
 }
 
@@ -232,13 +239,14 @@ __device__ inline Hit quad_closest(const SceneView &S, const TraceRay &q, QuadSt
 __device__ inline bool quad_any(const SceneView &S, const TraceRay &q, float dis, QuadStack &st) {
     Hit dummy{kMiss, HIT_NONE, -1, -1, 0, 0, 0};
     if (brute_objects(S, q, true, dis, dummy)) return true;
-    int blocked = 0;
+    int blocked = 0, self = 0;
     float tmax = dis;
     quad_walk<false>(S, q.r, tmax, st, [&](int pi) -> bool {
-        if (any_prim(q, load_prim(S, pi), dis)) blocked = 1;
+        if (any_prim(q, load_prim(S, pi), dis, self)) blocked = 1;
         return blocked != 0;
     });
-    return quad_or(blocked) != 0;
+    if (quad_or(blocked)) return true;
+    return quad_or(self) && self_testable(S, q.r, q.src, dis);
 }
 
 }  // namespace rtg

@@ -292,7 +292,6 @@ RTG_HD V3 render_sample(const SceneView &S, int max_level, const TraceRay &prima
                 rc.reflect++;
             else
                 rc.refract++;
-            if (q.src.obj >= 0) q.self_test = self_testable(S, q.r, q.src, kMiss);
             const Hit h = trace_closest<kRetest>(S, q, st, &rc.retests);
             if (q_level == 0) po = PrimaryOut{h.obj, id_prim(S, h), h.t};
             const float zNear = q_level == 0 ? S.cam.zNear : 0.0f;
@@ -311,7 +310,7 @@ RTG_HD V3 render_sample(const SceneView &S, int max_level, const TraceRay &prima
                     sr.type = RAY_SHADOW;
                     sr.inside = 0;
                     sr.src = hr.id;
-                    sr.self_test = self_testable(S, sr.r, hr.id, lt.dis);
+                    sr.self_test = 0;
                     return trace_any(S, sr, lt.dis, st);
                 });
                 Frame &f = fr[sp++];
@@ -470,7 +469,7 @@ RTG_HD V3 debug_sample(const SceneView &S, int mode, const TraceRay &q, Stack &s
         sr.type = RAY_SHADOW;
         sr.inside = 0;
         sr.src = hr.id;
-        sr.self_test = self_testable(S, sr.r, hr.id, lt.dis);
+        sr.self_test = 0;
         return trace_any(S, sr, lt.dis, st);
     });
 }

@@ -12,9 +12,14 @@
 // model's octant bins and skips only the copy whose address is the ray's
 // source (Model.cpp:775); a triangle stored in several bins can therefore be
 // hit again by its own secondary rays.  `self_testable` reproduces that: the
-// source triangle is tested iff the ray's BorderTest / BorderTestEx reach a
-// bin holding another copy of it.
+// source triangle counts iff the ray's BorderTest / BorderTestEx reach a bin
+// holding another copy of it.  It reads the object, the part and the bins one
+// after another, and a ray rarely hits its own triangle, so the walks set a hit
+// of it aside and ask only then, after the walk (asked before every walk:
+// SELF_FIGURES).
 #pragma once
+#include <type_traits>
+
 #include "rt_scene.hpp"
 
 namespace rtg {
@@ -28,7 +33,7 @@ struct TraceRay {
     int type;
     int inside;     // Ray::isInside
     SrcId src;      // HitRes::obj of the parent hit
-    int self_test;  // source triangle may be hit again (see header)
+    int self_test;  // source triangle may be hit again (FP64 re-test walk, see trace_closest)
 };
 
 struct Hit {
@@ -447,13 +452,17 @@ RTG_HD PrimRec load_prim(const SceneView &S, int pi) {
     return r;
 }
 
-// Closest-hit test of one primitive: objects with index < `before` only.
+// The source triangle of a secondary ray.
+RTG_HD bool is_source_tri(const TraceRay &q, int obj, int tri) { return tri == q.src.prim && obj == q.src.obj; }
+
+// Closest-hit test of one primitive: objects with index < `before` only.  A
+// hit of the ray's own source triangle is a hit here (is_source_tri).
 RTG_HD bool closest_prim(const TraceRay &q, const PrimRec &R, int before, Hit &h) {
     const int tag = as_int(R.a.w);
     const V3 p = V3{R.a.x, R.a.y, R.a.z};
     if (tag >= 0) {  // triangle, tag = global index
         const int obj = as_int(R.b.w);
-        if (obj >= before || (tag == q.src.prim && obj == q.src.obj && !q.self_test)) return false;
+        if (obj >= before) return false;
         float w, u, v;
         const float t = tri_test(q.r, V3{R.b.x, R.b.y, R.b.z}, V3{R.c.x, R.c.y, R.c.z}, p, w, u, v);
         h = Hit{t, HIT_TRI, obj, tag, w, u, v};
@@ -466,14 +475,26 @@ RTG_HD bool closest_prim(const TraceRay &q, const PrimRec &R, int before, Hit &h
     return t > 1e-6f && t < kMiss;
 }
 
-// Any-hit test of one primitive: it blocks the segment of length `dis`.
-RTG_HD bool any_prim(const TraceRay &q, const PrimRec &R, float dis) {
+// The hit of the source triangle (primitive slot pi) that a walk set aside
+// becomes the winner if it is closer and the triangle may be hit again.
+RTG_HD void take_source_hit(const SceneView &S, const TraceRay &q, int pi, int before, Hit &best, uint64_t bkey) {
+    Hit h;
+    if (!closest_prim(q, load_prim(S, pi), before, h)) return;
+    if (!(h.t < best.t || (h.t == best.t && hit_key(h.obj, h.prim) < bkey))) return;
+    if (self_testable(S, q.r, q.src, kMiss)) best = h;
+}
+
+// Any-hit test of one primitive: it blocks the segment of length `dis`.  The
+// source triangle does not; `self` is set where the segment meets it.
+RTG_HD bool any_prim(const TraceRay &q, const PrimRec &R, float dis, int &self) {
     const int tag = as_int(R.a.w);
     const V3 p = V3{R.a.x, R.a.y, R.a.z};
     if (tag >= 0) {
-        if (tag == q.src.prim && as_int(R.b.w) == q.src.obj && !q.self_test) return false;
         float w, u, v;
-        return tri_test(q.r, V3{R.b.x, R.b.y, R.b.z}, V3{R.c.x, R.c.y, R.c.z}, p, w, u, v) < dis;
+        if (!(tri_test(q.r, V3{R.b.x, R.b.y, R.b.z}, V3{R.c.x, R.c.y, R.c.z}, p, w, u, v) < dis)) return false;
+        if (!is_source_tri(q, as_int(R.b.w), tag)) return true;
+        self = 1;
+        return false;
     }
     if (q.src.obj == ~tag) return q.inside && R.b.y < dis;  // HitRes(radius) (Basic3DObject.cpp:143-144)
     const float t = sphere_enter_t(q.r, p, R.b.x);
@@ -484,8 +505,12 @@ RTG_HD bool any_prim(const TraceRay &q, const PrimRec &R, float dis) {
 // above); *retested counts the queries that were re-tested.  kBefore: only
 // objects with index < `before` take part (see child_src).
 template <bool kRetest = false, bool kBefore = false, class Stack>
-RTG_HD Hit trace_closest(const SceneView &S, const TraceRay &q, Stack &st, int *retested = nullptr,
+RTG_HD Hit trace_closest(const SceneView &S, const TraceRay &ray, Stack &st, int *retested = nullptr,
                          int before = 0x7fffffff) {
+    std::conditional_t<kRetest, TraceRay, const TraceRay &> q = ray;
+    // the re-test weighs every candidate of the walk, so it asks up front
+    if constexpr (kRetest) q.self_test = self_testable(S, q.r, q.src, kMiss);
+    int self = -1;  // slot of the source triangle, where the ray hits it
     Hit best{kMiss, HIT_NONE, -1, -1, 0, 0, 0};
     brute_objects(S, q, false, 0.0f, best, kBefore ? before : 0x7fffffff);
     uint64_t bkey = best.kind != HIT_NONE ? hit_key(best.obj, best.prim) : ~0ull;
@@ -508,8 +533,12 @@ RTG_HD Hit trace_closest(const SceneView &S, const TraceRay &q, Stack &st, int *
         const PrimRec R = load_prim(S, pi);
         if constexpr (!kRetest) {
             Hit h;
-            if (closest_prim(q, R, kBefore ? before : 0x7fffffff, h))
-                take(h.t, hit_key(h.obj, h.prim), pi, h, tm);
+            if (closest_prim(q, R, kBefore ? before : 0x7fffffff, h)) {
+                if (h.kind == HIT_TRI && is_source_tri(q, h.obj, h.prim))
+                    self = pi;
+                else
+                    take(h.t, hit_key(h.obj, h.prim), pi, h, tm);
+            }
             return false;
         }
         const float4 A = R.a;
@@ -518,7 +547,7 @@ RTG_HD Hit trace_closest(const SceneView &S, const TraceRay &q, Stack &st, int *
         if (tag >= 0) {  // triangle, tag = global index
             const float4 B = R.b, C = R.c;
             const int obj = as_int(B.w);
-            if (tag == q.src.prim && obj == q.src.obj && !q.self_test) return false;
+            if (is_source_tri(q, obj, tag) && !q.self_test) return false;
             const V3 e1 = V3{B.x, B.y, B.z}, e2 = V3{C.x, C.y, C.z};
             // tri_test's values without its early exits (same operations)
             const V3 tmp1 = cross(q.r.d, e2), t2r = q.r.o - p;
@@ -580,6 +609,8 @@ RTG_HD Hit trace_closest(const SceneView &S, const TraceRay &q, Stack &st, int *
                 if (retested) ++*retested;
             }
         }
+    } else if (self >= 0) {
+        take_source_hit(S, q, self, kBefore ? before : 0x7fffffff, best, bkey);
     }
     return best;
 }
@@ -615,11 +646,13 @@ RTG_HD bool trace_any(const SceneView &S, const TraceRay &q, float dis, Stack &s
     Hit dummy{kMiss, HIT_NONE, -1, -1, 0, 0, 0};
     if (brute_objects(S, q, true, dis, dummy)) return true;
     bool blocked = false;
+    int self = 0;
     float tmax = dis;
     bvh_walk<true, false>(S, q.r, tmax, st, [&](int pi, float &) -> bool {
-        blocked = any_prim(q, load_prim(S, pi), dis);
+        blocked = any_prim(q, load_prim(S, pi), dis, self);
         return blocked;
     });
+    if (!blocked && self) blocked = self_testable(S, q.r, q.src, dis) != 0;
     return blocked;
 }
 

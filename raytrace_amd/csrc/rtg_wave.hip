@@ -268,7 +268,6 @@ __device__ inline void extend_rays(const SceneView &S0, const WaveArgs &A, int k
         } else {
             float bwc, mtlrfr;
             q = load_ray(w, bwc, mtlrfr);
-            if (q.src.obj >= 0) q.self_test = self_testable(S, q.r, q.src, kMiss);
         }
         // Pass 0 is the closest hit.  A self re-hit (child_src) takes a second
         // pass over the objects before the source object; the plain kernel
@@ -570,7 +569,7 @@ __device__ inline void occlude_entries(const SceneView &S0, const WaveArgs &A, c
         sr.type = RAY_SHADOW;
         sr.inside = 0;
         sr.src = node_id(nd);
-        sr.self_test = self_testable(S, sr.r, sr.src, lt.dis);
+        sr.self_test = 0;
         if constexpr (Q) {
             if (quad_any(S, sr, lt.dis, st) && (threadIdx.x & (kQuadLanes - 1)) == 0) atomicOr(&masks[i], 1u << li);
         } else {
