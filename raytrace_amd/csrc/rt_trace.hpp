@@ -15,8 +15,9 @@
 // source triangle counts iff the ray's BorderTest / BorderTestEx reach a bin
 // holding another copy of it.  It reads the object, the part and the bins one
 // after another, and a ray rarely hits its own triangle, so the walks set a hit
-// of it aside and ask only then, after the walk (asked before every walk:
-// SELF_FIGURES).
+// of it aside and ask only then, after the walk (us a call, asked before each
+// walk -> after: refraction frame 960x540 at 4 samples 124628 -> 118910, 60
+// mixed requests 5965 -> 5833, 1080p frame 1930 -> 1912).
 #pragma once
 #include <type_traits>
 
