@@ -77,15 +77,28 @@ struct QuadStack {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     static __device__ unsigned at(unsigned e) { return (e / kQuadLanes) * kBlockThreads + e % kQuadLanes; }
-    // This lane's child takes entry e.
-    __device__ void put(int e, int v) {
+    // Entry 0 is kWalkDone (see DevStack).  Every lane of the quad calls it.
+    __device__ void reset() {
+        put_lds(0, kWalkDone);
+        sp = 1;
+    }
+    __device__ void put_lds(int e, int v) {
 #if defined(__HIP_DEVICE_COMPILE__)
         typedef int __attribute__((address_space(3))) LdsInt;
-        if (e < kLds)
-            ((LdsInt *)lds)[at(e)] = v;
-        else
-            spill[(e - kLds) * gstride] = v;
+        ((LdsInt *)lds)[at(e)] = v;
+        __asm__ volatile("" ::: "memory");
 #endif
+    }
+    // The lanes with `mine` put their v into their entry e, at most sp + 2.
+    __device__ void put(bool mine, int e, int v) {
+        if (__ballot(sp > kLds - 3) == 0ull) {
+            if (mine) put_lds(e, v);
+        } else if (mine) {
+            if (e < kLds)
+                put_lds(e, v);
+            else
+                spill[(e - kLds) * gstride] = v;
+        }
     }
     __device__ int pop() {
         --sp;
@@ -93,9 +106,12 @@ struct QuadStack {
         order();
 #if defined(__HIP_DEVICE_COMPILE__)
         typedef const int __attribute__((address_space(3))) LdsInt;
-        if (sp < kLds) {
+        if (__ballot(sp >= kLds) == 0ull) {
             v = ((LdsInt *)lds)[at(sp)];
             __asm__ volatile("" ::: "memory");  // not merged with the spill read into a flat load
+        } else if (sp < kLds) {
+            v = ((LdsInt *)lds)[at(sp)];
+            __asm__ volatile("" ::: "memory");
         } else {
             v = spill[(sp - kLds) * gstride];
         }
@@ -103,7 +119,6 @@ struct QuadStack {
         order();
         return v;
     }
-    __device__ int pop_or_done() { return sp == 0 ? kWalkDone : pop(); }
     template <int N, int D>
     __device__ bool lanes_at_least(bool v) const {
         return D * __popcll(__ballot(v)) >= N * __popcll(__ballot(true));
@@ -132,8 +147,8 @@ struct QuadStack {
 // wave-wide exit of the node loop.  test(primitive) -> true to stop (any-hit).
 template <bool kOrdered, class Test>
 __device__ inline void quad_walk(const SceneView &S, const Ray &r, float &tmax, QuadStack &st, Test &&test) {
-    st.sp = 0;
     if (S.n_prims == 0) return;
+    st.reset();
     const int k = threadIdx.x & (kQuadLanes - 1);
     const V3 inv = safe_inv(r.d);
     int node = S.root;
@@ -157,8 +172,8 @@ __device__ inline void quad_walk(const SceneView &S, const Ray &r, float &tmax, 
             hits = __popc(m);
         }
         const int next = quad_or(h && rank == 0 ? link : 0);
-        if (h && rank > 0) st.put(st.sp + hits - 1 - rank, link);
-        if (hits == 0) return st.pop_or_done();
+        st.put(h && rank > 0, st.sp + hits - 1 - rank, link);
+        if (hits == 0) return st.pop();
         st.sp += hits - 1;
         return next;
     };
@@ -168,14 +183,14 @@ __device__ inline void quad_walk(const SceneView &S, const Ray &r, float &tmax, 
             node = step(node);
             if (node < 0 && node != kWalkDone && leaf2 == 0) {
                 (leaf == 0 ? leaf : leaf2) = node;
-                node = st.pop_or_done();
+                node = st.pop();
             }
             if (kOrdered ? st.template lanes_at_least<1, 2>(leaf != 0) : st.template lanes_at_least<3, 4>(leaf != 0))
                 break;
         }
         if (leaf == 0 && node < 0 && node != kWalkDone) {
             leaf = node;
-            node = st.pop_or_done();
+            node = st.pop();
         }
         while (leaf < 0) {
             // lanes 0 and 1 take the first leaf's primitives, 2 and 3 the second's
@@ -192,7 +207,7 @@ __device__ inline void quad_walk(const SceneView &S, const Ray &r, float &tmax, 
             leaf = leaf2 = 0;
             if (node < 0 && node != kWalkDone) {
                 leaf = node;
-                node = st.pop_or_done();
+                node = st.pop();
             }
         }
         if (node == kWalkDone) return;

@@ -44,14 +44,16 @@ struct alignas(16) Bvh4Node {
 static_assert(sizeof(Bvh4Node) == 64, "64-byte node");
 
 // Internal levels of a 4-wide tree the traversal stack holds: a walk leaves at
-// most 3 entries per level.  A Karras tree over 62-bit keys has under 63
-// internal binary levels, so its even-depth widening stays within this.
-constexpr int kMaxLevels4 = 32;
+// most 3 entries per level.  A Karras tree over 62-bit unique keys has at most
+// 62 internal binary levels (a child's common prefix is longer than its
+// parent's), so its even-depth widening has at most 31.
+constexpr int kMaxLevels4 = 31;
 
 // The first nodes are the top levels of the tree (indices < kTopNodes):
 // traversal kernels that render one scene keep them in LDS.
 constexpr int kTopNodes = 31;
 
+constexpr int kWalkDone = (int)0x80000000;  // no node left: below every leaf code
 RTG_HD bool is_leaf(int c) { return c < 0; }
 RTG_HD int leaf_first(int c) { return (~c) >> 3; }
 RTG_HD int leaf_count(int c) { return ((~c) & 7) + 1; }

@@ -73,11 +73,12 @@ RTG_HD bool slab(V3 o, V3 inv, float lx, float hx, float ly, float hy, float lz,
 // exact (s is a power of two).  The decoded bound org + q s = (m + q) s is a
 // float exactly (quantize_axis), so against `slab`'s fl(fl(org + q s - o) inv)
 // the result is off by at most 6.1 eps |(org - o) inv| + 766 eps |s inv|
-// (eps = 2^-24, the constant term's own rounding included); the constant term
-// moves out by 16 eps |(org - o) inv| + 2048 eps |s inv|, and rounding to
-// nearest keeps the margin's effect monotone.  An overflow makes a term
-// infinite or NaN, which fmaxf / fminf drop: the test then only passes more
-// children.
+// (eps = 2^-24, the constant term's own rounding included).  `slab` scales its
+// exit distance by kFarScale = 1 + 10.1 eps, at most another 10.1 eps
+// |(org - o) inv| + 2576 eps |s inv|.  The constant term moves out by more than
+// both, 32 eps |(org - o) inv| + 4096 eps |s inv|, and rounding to nearest keeps
+// the margin's effect monotone.  An overflow makes a term infinite or NaN,
+// which fmaxf / fminf drop: the test then only passes more children.
 struct Node4Test {
     float sx, sy, sz;  // s inv per axis
     float nx, fx, ny, fy, nz, fz;  // (org - o) inv moved out, for entry and exit
@@ -86,9 +87,10 @@ struct Node4Test {
         const uint32_t e = __builtin_bit_cast(uint32_t, n.org.w);
         sx = pow2f(e & 0xFF) * inv.x, sy = pow2f((e >> 8) & 0xFF) * inv.y, sz = pow2f((e >> 16) & 0xFF) * inv.z;
         const float bx = (n.org.x - o.x) * inv.x, by = (n.org.y - o.y) * inv.y, bz = (n.org.z - o.z) * inv.z;
-        const float mx = fabsf(bx) * 9.5367431640625e-07f + fabsf(sx) * 1.220703125e-04f;  // 2^-20, 2^-13
-        const float my = fabsf(by) * 9.5367431640625e-07f + fabsf(sy) * 1.220703125e-04f;
-        const float mz = fabsf(bz) * 9.5367431640625e-07f + fabsf(sz) * 1.220703125e-04f;
+        constexpr float cb = 1.9073486328125e-06f, cs = 2.44140625e-04f;  // 2^-19, 2^-12
+        const float mx = fmaf(fabsf(bx), cb, fabsf(sx) * cs);
+        const float my = fmaf(fabsf(by), cb, fabsf(sy) * cs);
+        const float mz = fmaf(fabsf(bz), cb, fabsf(sz) * cs);
         nx = bx - mx, fx = bx + mx, ny = by - my, fy = by + my, nz = bz - mz, fz = bz + mz;
         // a negative direction enters a box through its upper bound
         const bool neg_x = inv.x < 0.0f, neg_y = inv.y < 0.0f, neg_z = inv.z < 0.0f;
@@ -106,8 +108,7 @@ struct Node4Test {
         const float tnz = fmaf((float)((qnz >> sh) & 0xFF), sz, nz);
         const float tfz = fmaf((float)((qfz >> sh) & 0xFF), sz, fz);
         near = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, 0.0f));
-        const float far = fminf(fminf(tfx, tfy), tfz) * kFarScale;
-        return near <= fminf(far, tmax);
+        return near <= fminf(fminf(tfx, tfy), fminf(tfz, tmax));
     }
 };
 
@@ -128,7 +129,16 @@ struct ArrayStack {
     RTG_HD Bvh4Node node(const SceneView &S, int i) const { return S.nodes[i]; }
 };
 
-constexpr int kWalkDone = (int)0x80000000;  // no node left: below every leaf code
+// The next entry of a walk's stack, or kWalkDone.
+template <class Stack>
+RTG_HD int pop_or_done(Stack &st) {
+    return st.empty() ? kWalkDone : st.pop();
+}
+// Run the pushes of one node (at most three), f(push).
+template <class Stack, class F>
+RTG_HD void node_pushes(Stack &st, F &&f) {
+    f([&](int v) { st.push(v); });
+}
 
 // Visit the primitives of every leaf the segment [0, tmax] reaches, nearest
 // child first (kOrdered; otherwise in child order, for the any-hit test).
@@ -168,7 +178,7 @@ RTG_HD void bvh_walk(const SceneView &S, const Ray &r, float &tmax, Stack &st, V
         // missing child decode to a point) and the count masks the result,
         // which keeps the wave's four tests free of branches
 #pragma unroll
-        for (int k = 0; k < 4; ++k) h[k] = nt.child(k, tmax, t[k]) & (k < nc);
+        for (int k = 0; k < 4; ++k) h[k] = nt.child(k, tmax, t[k]) & (k < 2 || k < nc);
         int next = kWalkDone;
         if constexpr (kOrdered) {
             // Sort keys: the entry distance's bits (t >= 0, so they order as
@@ -188,20 +198,24 @@ RTG_HD void bvh_walk(const SceneView &S, const Ray &r, float &tmax, Stack &st, V
                 a = lo, b = hi;
             };
             cx(s[0], s[1]), cx(s[2], s[3]), cx(s[0], s[2]), cx(s[1], s[3]), cx(s[1], s[2]);
+            node_pushes(st, [&](auto &&push) {
 #pragma unroll
-            for (int r = 3; r >= 1; --r)
-                if (s[r] != ~0ull) st.push((int)(uint32_t)s[r]);
+                for (int r = 3; r >= 1; --r)
+                    if (s[r] != ~0ull) push((int)(uint32_t)s[r]);
+            });
             if (s[0] != ~0ull) next = (int)(uint32_t)s[0];
         } else {
+            node_pushes(st, [&](auto &&push) {
 #pragma unroll
-            for (int k = 3; k >= 0; --k)
-                if (h[k]) {
-                    if (next != kWalkDone) st.push(next);
-                    next = lk[k];
-                }
+                for (int k = 3; k >= 0; --k)
+                    if (h[k]) {
+                        if (next != kWalkDone) push(next);
+                        next = lk[k];
+                    }
+            });
         }
         if (next != kWalkDone) return next;
-        return st.empty() ? kWalkDone : st.pop();
+        return pop_or_done(st);
     };
     if constexpr (!kSpec) {
         for (;;) {
@@ -214,8 +228,8 @@ RTG_HD void bvh_walk(const SceneView &S, const Ray &r, float &tmax, Stack &st, V
                 st.on_prim();
                 if (visit(first + i, tmax)) return;
             }
-            if (st.empty()) return;
-            node = st.pop();
+            node = pop_or_done(st);
+            if (node == kWalkDone) return;
         }
     } else {
         int leaf = 0, leaf2 = 0;  // postponed leaves (< 0), or 0
@@ -224,7 +238,7 @@ RTG_HD void bvh_walk(const SceneView &S, const Ray &r, float &tmax, Stack &st, V
                 node = step(node);
                 if (node < 0 && node != kWalkDone && leaf2 == 0) {
                     (leaf == 0 ? leaf : leaf2) = node;
-                    node = st.empty() ? kWalkDone : st.pop();
+                    node = pop_or_done(st);
                 }
                 // closest hit: half the lanes; any hit: three quarters
                 if (kOrdered ? st.template lanes_at_least<1, 2>(leaf != 0)
@@ -233,20 +247,28 @@ RTG_HD void bvh_walk(const SceneView &S, const Ray &r, float &tmax, Stack &st, V
             }
             if (leaf == 0 && node < 0 && node != kWalkDone) {
                 leaf = node;
-                node = st.empty() ? kWalkDone : st.pop();
+                node = pop_or_done(st);
             }
-            while (leaf < 0) {
-                const int first = leaf_first(leaf), count = leaf_count(leaf);
-                for (int i = 0; i < count; ++i) {
+            // one loop over the primitives of every held leaf, so that a lane
+            // with a short leaf goes on with its next one
+            if (leaf < 0) {
+                int pi = leaf_first(leaf), end = pi + leaf_count(leaf);
+                for (;;) {
                     st.on_prim();
-                    if (visit(first + i, tmax)) return;
+                    if (visit(pi, tmax)) {
+                        node = kWalkDone;
+                        break;
+                    }
+                    if (++pi < end) continue;
+                    leaf = leaf2, leaf2 = 0;
+                    if (leaf == 0 && node < 0 && node != kWalkDone) {
+                        leaf = node;
+                        node = pop_or_done(st);
+                    }
+                    if (leaf == 0) break;
+                    pi = leaf_first(leaf), end = pi + leaf_count(leaf);
                 }
-                leaf = leaf2;
-                leaf2 = 0;
-                if (leaf == 0 && node < 0 && node != kWalkDone) {
-                    leaf = node;
-                    node = st.empty() ? kWalkDone : st.pop();
-                }
+                leaf = leaf2 = 0;
             }
             if (node == kWalkDone) return;
         }
