@@ -79,7 +79,7 @@ struct DevStack {
     __device__ bool lanes_at_least(bool v) const {
         return D * __popcll(__ballot(v)) >= N * __popcll(__ballot(true));
     }
-    __device__ Bvh4Node node(const SceneView &S, int i) const {
+    __device__ Bvh4Node node(const Bvh4Node *nodes, int i) const {
 #if defined(__HIP_DEVICE_COMPILE__)
         typedef const Bvh4Node __attribute__((address_space(3))) LdsNode;  // `top` points into LDS
         if (top != nullptr && i < kTopNodes) {
@@ -90,10 +90,11 @@ struct DevStack {
             return n;
         }
 #endif
-        return S.nodes[i];
+        return nodes[i];
     }
 };
 
+__device__ inline Bvh4Node node_of(const DevStack &st, const Bvh4Node *nodes, int i) { return st.node(nodes, i); }
 // (the stack's own end mark answers)
 __device__ inline int pop_or_done(DevStack &st) { return st.pop(); }
 template <class F>
@@ -145,27 +146,27 @@ struct alignas(256) LineCtr {
     unsigned pad[63];
 };
 
-// Per-wave dynamic work split: a wave grabs chunks of kStep << grab_lg items,
+// Per-wave dynamic work split: a wave grabs chunks of 1 << (step_lg +
+// grab_lg) items,
 // first from its XCD's contiguous eighth of the range (one counter per XCD, so
 // neighbouring chunks share an L2), then from the other XCDs' eighths once its
-// own is exhausted, and hands a grabbed chunk out kStep items per next() call.
+// own is exhausted, and hands a grabbed chunk out 1 << step_lg items per next() call.
 // `ctr` points to 8 counters that are zero at launch.  Every lane of the wave
-// must call next(); it returns the first item of the next kStep, or -1 when
+// must call next(); it returns the first item of the next ones, or -1 when
 // every chunk is taken.  A region whose counter was seen past its end is never
 // tried again by the wave, so a wave makes at most 8 failed grabs.
-template <int kStepLg = 6>
-struct WaveQueueT {
-    static constexpr int kStep = 1 << kStepLg;
+struct WaveQueue {
     LineCtr *ctr;
-    int n, glg, nchunks, region, x;
+    int n, slg, glg, nchunks, region, x;
     int cur, end;   // the grabbed chunk: next item handed out, end (wave-uniform)
     uint32_t dead;  // regions this wave has seen exhausted
-    __device__ WaveQueueT(LineCtr *c, int n_items, int grab_lg = 0)
-        : ctr(c), n(n_items), glg(grab_lg), nchunks((n_items + (kStep << grab_lg) - 1) >> (kStepLg + grab_lg)),
+    __device__ WaveQueue(LineCtr *c, int n_items, int grab_lg = 0, int step_lg = 6)
+        : ctr(c), n(n_items), slg(step_lg), glg(grab_lg),
+          nchunks((n_items + (1 << (step_lg + grab_lg)) - 1) >> (step_lg + grab_lg)),
           region((nchunks + 7) >> 3), x(blockIdx.x & 7), cur(0), end(0), dead(0) {}
     __device__ int region_len(int r) const { return max(0, min(region, nchunks - r * region)); }
     __device__ int next() {
-        if (cur + kStep < end) return cur += kStep;
+        if (cur + (1 << slg) < end) return cur += 1 << slg;
         if (nchunks == 0) return -1;
         const int lane = __lane_id();
         for (;;) {
@@ -173,8 +174,8 @@ struct WaveQueueT {
             if (lane == 0) c = (int)atomicAdd(&ctr[x].v, 1u);
             c = __builtin_amdgcn_readfirstlane(c);  // wave-uniform: an SGPR
             if (c < region_len(x)) {
-                cur = (x * region + c) << (kStepLg + glg);
-                end = min(n, cur + (kStep << glg));
+                cur = (x * region + c) << (slg + glg);
+                end = min(n, cur + (1 << (slg + glg)));
                 return cur;
             }
             dead |= 1u << x;
@@ -190,7 +191,6 @@ struct WaveQueueT {
         }
     }
 };
-using WaveQueue = WaveQueueT<>;
 
 __device__ inline uint32_t wave_sum_u32(uint32_t v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

@@ -126,9 +126,13 @@ struct ArrayStack {
     RTG_HD bool lanes_at_least(bool v) const {  // one lane
         return v;
     }
-    RTG_HD Bvh4Node node(const SceneView &S, int i) const { return S.nodes[i]; }
 };
 
+// Node i, from the stack's copy of the top nodes where it keeps one.
+template <class Stack>
+RTG_HD Bvh4Node node_of(const Stack &, const Bvh4Node *nodes, int i) {
+    return nodes[i];
+}
 // The next entry of a walk's stack, or kWalkDone.
 template <class Stack>
 RTG_HD int pop_or_done(Stack &st) {
@@ -138,6 +142,62 @@ RTG_HD int pop_or_done(Stack &st) {
 template <class Stack, class F>
 RTG_HD void node_pushes(Stack &st, F &&f) {
     f([&](int v) { st.push(v); });
+}
+
+// One 4-wide node: the next node to enter (the nearest child the segment
+// reaches), the other children it reaches pushed farthest first; the
+// popped entry when it reaches none.
+template <bool kOrdered, class Stack>
+RTG_HD int node_step(const Bvh4Node *nodes, int nd, V3 o, V3 inv, float tmax, Stack &st) {
+    st.on_node();
+    const Bvh4Node n = node_of(st, nodes, nd);
+    const int nc = node4_count(n);
+    const int lk[4] = {n.link.x, n.link.y, n.link.z, n.link.w};
+    float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    bool h[4];
+    const Node4Test nt(n, o, inv);
+    // a node has 2 to 4 children; all four are tested (the bytes of a
+    // missing child decode to a point) and the count masks the result,
+    // which keeps the wave's four tests free of branches
+#pragma unroll
+    for (int k = 0; k < 4; ++k) h[k] = nt.child(k, tmax, t[k]) & (k < 2 || k < nc);
+    int next = kWalkDone;
+    if constexpr (kOrdered) {
+        // Sort keys: the entry distance's bits (t >= 0, so they order as
+        // the distances do) above the child's link, or ~0 for a child the
+        // segment misses; five compare-exchanges sort them, nearest first.
+        // The links travel in the keys: picking them by index afterwards
+        // would send the node to scratch memory.  Only the order of the
+        // walk depends on the sort.
+        uint64_t s[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            s[k] = h[k] ? ((uint64_t)__builtin_bit_cast(uint32_t, t[k] > 0.0f ? t[k] : 0.0f) << 32 |
+                           (uint32_t)lk[k])
+                        : ~0ull;
+        auto cx = [](uint64_t &a, uint64_t &b) {
+            const uint64_t lo = a < b ? a : b, hi = a < b ? b : a;
+            a = lo, b = hi;
+        };
+        cx(s[0], s[1]), cx(s[2], s[3]), cx(s[0], s[2]), cx(s[1], s[3]), cx(s[1], s[2]);
+        node_pushes(st, [&](auto &&push) {
+#pragma unroll
+            for (int r = 3; r >= 1; --r)
+                if (s[r] != ~0ull) push((int)(uint32_t)s[r]);
+        });
+        if (s[0] != ~0ull) next = (int)(uint32_t)s[0];
+    } else {
+        node_pushes(st, [&](auto &&push) {
+#pragma unroll
+            for (int k = 3; k >= 0; --k)
+                if (h[k]) {
+                    if (next != kWalkDone) push(next);
+                    next = lk[k];
+                }
+        });
+    }
+    if (next != kWalkDone) return next;
+    return pop_or_done(st);
 }
 
 // Visit the primitives of every leaf the segment [0, tmax] reaches, nearest
@@ -163,60 +223,7 @@ RTG_HD void bvh_walk(const SceneView &S, const Ray &r, float &tmax, Stack &st, V
     if (S.n_prims == 0) return;
     const V3 inv = safe_inv(r.d);
     int node = S.root;
-    // One 4-wide node: the next node to enter (the nearest child the segment
-    // reaches), the other children it reaches pushed farthest first; the
-    // popped entry when it reaches none.
-    auto step = [&](int nd) -> int {
-        st.on_node();
-        const Bvh4Node n = st.node(S, nd);
-        const int nc = node4_count(n);
-        const int lk[4] = {n.link.x, n.link.y, n.link.z, n.link.w};
-        float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        bool h[4];
-        const Node4Test nt(n, r.o, inv);
-        // a node has 2 to 4 children; all four are tested (the bytes of a
-        // missing child decode to a point) and the count masks the result,
-        // which keeps the wave's four tests free of branches
-#pragma unroll
-        for (int k = 0; k < 4; ++k) h[k] = nt.child(k, tmax, t[k]) & (k < 2 || k < nc);
-        int next = kWalkDone;
-        if constexpr (kOrdered) {
-            // Sort keys: the entry distance's bits (t >= 0, so they order as
-            // the distances do) above the child's link, or ~0 for a child the
-            // segment misses; five compare-exchanges sort them, nearest first.
-            // The links travel in the keys: picking them by index afterwards
-            // would send the node to scratch memory.  Only the order of the
-            // walk depends on the sort.
-            uint64_t s[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                s[k] = h[k] ? ((uint64_t)__builtin_bit_cast(uint32_t, t[k] > 0.0f ? t[k] : 0.0f) << 32 |
-                               (uint32_t)lk[k])
-                            : ~0ull;
-            auto cx = [](uint64_t &a, uint64_t &b) {
-                const uint64_t lo = a < b ? a : b, hi = a < b ? b : a;
-                a = lo, b = hi;
-            };
-            cx(s[0], s[1]), cx(s[2], s[3]), cx(s[0], s[2]), cx(s[1], s[3]), cx(s[1], s[2]);
-            node_pushes(st, [&](auto &&push) {
-#pragma unroll
-                for (int r = 3; r >= 1; --r)
-                    if (s[r] != ~0ull) push((int)(uint32_t)s[r]);
-            });
-            if (s[0] != ~0ull) next = (int)(uint32_t)s[0];
-        } else {
-            node_pushes(st, [&](auto &&push) {
-#pragma unroll
-                for (int k = 3; k >= 0; --k)
-                    if (h[k]) {
-                        if (next != kWalkDone) push(next);
-                        next = lk[k];
-                    }
-            });
-        }
-        if (next != kWalkDone) return next;
-        return pop_or_done(st);
-    };
+    auto step = [&](int nd) { return node_step<kOrdered>(S.nodes, nd, r.o, inv, tmax, st); };
     if constexpr (!kSpec) {
         for (;;) {
             while (node >= 0) {
@@ -463,8 +470,8 @@ RTG_HD bool retest64(const SceneView &S, const TraceRay &q, int pi, double &t64,
 struct PrimRec {
     float4 a, b, c;
 };
-RTG_HD PrimRec load_prim(const SceneView &S, int pi) {
-    const float4 *p = S.prims + 3 * (size_t)pi;
+RTG_HD PrimRec load_prim(const float4 *prims, int pi) {
+    const float4 *p = prims + 3 * (size_t)pi;
     PrimRec r{p[0], p[1], p[2]};
 #if defined(__HIP_DEVICE_COMPILE__)
     // uses every component here (no instruction), so the three reads are
@@ -474,6 +481,7 @@ RTG_HD PrimRec load_prim(const SceneView &S, int pi) {
 #endif
     return r;
 }
+RTG_HD PrimRec load_prim(const SceneView &S, int pi) { return load_prim(S.prims, pi); }
 
 // The source triangle of a secondary ray.
 RTG_HD bool is_source_tri(const TraceRay &q, int obj, int tri) { return tri == q.src.prim && obj == q.src.obj; }

@@ -237,38 +237,48 @@ __device__ inline int grab_lg_for(int n, int lg) {
     return lg;
 }
 
-// Closest hits of the queue's rays: one lane per ray, or with Q four
-// (rt_quad.hpp; lane 0 of the quad writes).
-template <bool B, bool R, bool Q, class Stack>
-__device__ inline void extend_rays(const SceneView &S0, const WaveArgs &A, int k, const WRay *rays, int n, WHit *hits,
-                                   int4 *cs, LineCtr *sched, Stack &st) {
-    WaveQueueT<Q ? 4 : 6> wq(sched, n, Q ? 0 : A.grab_lg);
+// Ray i of level k's queue (level 0: the primary ray of sample i).  Returns its
+// request (-1: a padding sample); `valid` says whether there is a ray.
+template <bool B>
+__device__ inline int queue_ray(const SceneView &S0, const WaveArgs &A, int k, const WRay *rays, int i, TraceRay &q,
+                                bool &valid) {
+    int r = 0;
+    WRay w{};
+    if (k == 0) {
+        r = sample_req<B>(A, i);
+    } else {
+        w = rays[i];
+        r = w.flags >> 8;
+    }
+    valid = r >= 0;
+    if (k == 0) {
+        const WaveReq &Rq = req_at<B>(A, r < 0 ? 0 : r);
+        int px = 0, py = 0, si = 0;
+        if (valid) valid = sample_pixel(Rq, i - Rq.sample_base, px, py, si);
+        if (valid) q = primary_ray_w(scene_at<B>(S0, A, Rq.scene), Rq, px, py, si);
+    } else {
+        float bwc, mtlrfr;
+        q = load_ray(w, bwc, mtlrfr);
+    }
+    return r;
+}
+
+// Closest hits of the queue's rays, a lane per ray walked on its own: where
+// some request asks for the FP64 re-test (R), and long queues.
+template <bool B, bool R>
+__device__ inline void extend_lanes(const SceneView &S0, const WaveArgs &A, int k, const WRay *rays, int n, WHit *hits,
+                                   int4 *cs, LineCtr *sched, DevStack &st) {
+    WaveQueue wq(sched, n, A.grab_lg);
     uint32_t c_prim = 0, c_refl = 0, c_refr = 0;
     int n_retest = 0;
-    const bool writer = !Q || (threadIdx.x & (kQuadLanes - 1)) == 0;
     for (int base = wq.next(); base >= 0; base = wq.next()) {
-        const int i = base + (Q ? __lane_id() / kQuadLanes : __lane_id());
+        const int i = base + __lane_id();
         if (i >= n) continue;
-        int r = 0;
-        WRay w{};
-        if (k == 0) {
-            r = sample_req<B>(A, i);
-        } else {
-            w = rays[i];
-            r = w.flags >> 8;
-        }
+        TraceRay q;
+        bool valid;
+        const int r = queue_ray<B>(S0, A, k, rays, i, q, valid);
         const WaveReq &Rq = req_at<B>(A, r < 0 ? 0 : r);
         const SceneView &S = scene_at<B>(S0, A, Rq.scene);
-        TraceRay q;
-        int px = 0, py = 0, si = 0;
-        bool valid = r >= 0;
-        if (k == 0) {
-            if (valid) valid = sample_pixel(Rq, i - Rq.sample_base, px, py, si);
-            if (valid) q = primary_ray_w(S, Rq, px, py, si);
-        } else {
-            float bwc, mtlrfr;
-            q = load_ray(w, bwc, mtlrfr);
-        }
         // Pass 0 is the closest hit.  A self re-hit (child_src) takes a second
         // pass over the objects before the source object; the plain kernel
         // runs it through the same walk (one inlined copy of the traversal),
@@ -279,17 +289,15 @@ __device__ inline void extend_rays(const SceneView &S0, const WaveArgs &A, int k
             if (valid) {
                 if constexpr (R)
                     h = Rq.retest ? trace_closest<true>(S, q, st, &n_retest) : trace_closest<false>(S, q, st);
-                else if constexpr (Q)
-                    h = quad_closest(S, q, st, before);
                 else
                     h = trace_closest<false, true>(S, q, st, nullptr, before);
             }
             if (before != 0x7fffffff) {
                 const SrcId c = child_src_of(S, q, h);
-                if (writer) cs[i] = int4{c.obj, c.prim, c.bin, 0};
+                cs[i] = int4{c.obj, c.prim, c.bin, 0};
                 break;
             }
-            if (valid && writer) {
+            if (valid) {
                 if (k == 0)
                     ++c_prim;
                 else if (q.type == RAY_REFLECT)
@@ -298,7 +306,7 @@ __device__ inline void extend_rays(const SceneView &S0, const WaveArgs &A, int k
                     ++c_refr;
             }
             const bool self = valid && h.kind != HIT_NONE && is_self_rehit(q, h);
-            if (writer) hits[i] = WHit{h.t, h.w, h.u, h.v, h.kind, h.obj, h.prim, self ? 1 : 0};
+            hits[i] = WHit{h.t, h.w, h.u, h.v, h.kind, h.obj, h.prim, self ? 1 : 0};
             if (!self) break;
             if constexpr (R) {
                 const SrcId c = child_src(S, q, h, st);
@@ -315,14 +323,74 @@ __device__ inline void extend_rays(const SceneView &S0, const WaveArgs &A, int k
     }
 }
 
-// R: some request asks for the FP64 near-tie re-test (a separate kernel, so
-// the plain closest-hit walk keeps its registers).
-template <bool B, bool R>
-__global__ __launch_bounds__(kBlockThreads, 6) void k_extend(SceneView S0, WaveArgs A, int k, const WRay *rays,
-                                                             const unsigned *n_ptr, WHit *hits, int4 *cs,
-                                                             LineCtr *sched) {
+// Closest hits of the queue's rays, one lane per ray, or with `quads` four (lane
+// 0 of the quad writes); the whole wave goes through every step (rt_quad.hpp).
+template <bool B>
+__device__ inline void extend_rays(bool quads, const SceneView &S0, const WaveArgs &A, int k, const WRay *rays, int n,
+                                   WHit *hits, int4 *cs, LineCtr *sched, DevStack &st, int *lds) {
+    WaveQueue wq(sched, n, quads ? 0 : A.grab_lg, quads ? 4 : 6);
+    uint32_t c_prim = 0, c_refl = 0, c_refr = 0;
+    const bool writer = !quads || (threadIdx.x & (kQuadLanes - 1)) == 0;
+    for (int base = wq.next(); base >= 0; base = wq.next()) {
+        const int i = base + (quads ? __lane_id() / kQuadLanes : __lane_id());
+        TraceRay q{};
+        q.src = no_src();
+        bool valid = false;
+        int r = -1;
+        if (i < n) r = queue_ray<B>(S0, A, k, rays, i, q, valid);
+        const SceneView &S = scene_at<B>(S0, A, req_at<B>(A, r < 0 ? 0 : r).scene);
+        // Pass 0 is the closest hit.  A self re-hit (child_src) takes a second
+        // pass over the objects before the source object, through the same
+        // walk (one inlined copy of the traversal), after the hit record is
+        // stored so that little state stays live.
+        int before = 0x7fffffff;
+        bool walks = valid;
+        for (int pass = 0;; ++pass) {
+            const Hit h = wave_closest<!B>(quads, S, q, st, lds, before, walks);
+            if (pass == 1) {
+                if (walks && writer) {
+                    const SrcId c = child_src_of(S, q, h);
+                    cs[i] = int4{c.obj, c.prim, c.bin, 0};
+                }
+                break;
+            }
+            const bool self = valid && h.kind != HIT_NONE && is_self_rehit(q, h);
+            if (writer && i < n) {
+                if (valid) {
+                    if (k == 0)
+                        ++c_prim;
+                    else if (q.type == RAY_REFLECT)
+                        ++c_refl;
+                    else
+                        ++c_refr;
+                }
+                hits[i] = WHit{h.t, h.w, h.u, h.v, h.kind, h.obj, h.prim, self ? 1 : 0};
+            }
+            if (__ballot(self) == 0ull) break;
+            walks = self;
+            before = self ? h.obj : 0;
+        }
+    }
+    add_counts(A.counts, c_prim, 0, c_refl, c_refr);
+}
+
+// How a kernel walks its queue.  WALK_WAVE: the waves' rays together
+// (rt_quad.hpp), at 4 (k_occlude 6) waves per SIMD: at 6 (8) its node loops
+// spill, and a wave's steps, not the number of waves, bound a level with a tail
+// (801x451 frame at 4 samples: 1829 us at 6 and 8 waves, 1686 at 4 and 6; 60
+// mixed requests 4507 of 5196, 5736 of 7143).  WALK_LANES: lane by lane, at
+// fewer registers and 6 (8) waves, for queues so long that the GPU is full all
+// the time and waves hide the loads (a refraction frame whose levels hold
+// millions of rays: 108.7 ms, 122.6 by WALK_WAVE).  WALK_RETEST: lane by lane
+// with the FP64 near-tie re-test.
+enum Walk { WALK_WAVE, WALK_LANES, WALK_RETEST };
+
+template <bool B, Walk W>
+__global__ __launch_bounds__(kBlockThreads, W == WALK_WAVE ? 4 : 6)
+void k_extend(SceneView S0, WaveArgs A, int k, const WRay *rays, const unsigned *n_ptr, WHit *hits, int4 *cs,
+              LineCtr *sched) {
     const int n = k == 0 ? A.n_samples : (int)*n_ptr;
-    const bool quads = !R && n <= A.quad_max;
+    const bool quads = W == WALK_WAVE && n <= A.quad_max;
     if (quads ? surplus_block<4>(n) : surplus_block(n)) return;
     __shared__ int lds[kLdsStack * kBlockThreads];
     DevStack st = make_stack(lds, A.spill);
@@ -331,13 +399,10 @@ __global__ __launch_bounds__(kBlockThreads, 6) void k_extend(SceneView S0, WaveA
         stack_top_nodes(st, top_nodes, S0);
     }
     if (wave_cancelled(A)) return;
-    if constexpr (!R)
-        if (quads) {
-            QuadStack qs(st, lds);
-            extend_rays<B, R, true>(S0, A, k, rays, n, hits, cs, sched, qs);
-            return;
-        }
-    extend_rays<B, R, false>(S0, A, k, rays, n, hits, cs, sched, st);
+    if constexpr (W == WALK_WAVE)
+        extend_rays<B>(quads, S0, A, k, rays, n, hits, cs, sched, st, lds);
+    else
+        extend_lanes<B, W == WALK_RETEST>(S0, A, k, rays, n, hits, cs, sched, st);
 }
 
 // k_shade's appends are staged per wave in LDS and reach their queue a buffer
@@ -549,40 +614,65 @@ __global__ __launch_bounds__(kBlockThreads, 4) void k_shade(SceneView S0, WaveAr
     add_counts(A.counts, 0, c_shadow, 0, 0);
 }
 
-// Shadow tests of the queue's entries: one lane per entry, or with Q four.
-template <bool B, bool Q, class Stack>
-__device__ inline void occlude_entries(const SceneView &S0, const WaveArgs &A, const WNode *nodes,
-                                       const unsigned *shadow, int n, LineCtr *sched, unsigned *masks, Stack &st) {
-    WaveQueueT<Q ? 4 : 6> wq(sched, n, Q ? 0 : A.grab_lg);
+// Shadow ray of queue entry e and its length; returns its scene.
+template <bool B>
+__device__ inline const SceneView &entry_ray(const SceneView &S0, const WaveArgs &A, const WNode *nodes, unsigned e,
+                                             TraceRay &sr, float &dis) {
+    const int i = (int)(e >> 5), li = (int)(e & 31);
+    const WNode nd = nodes[i];
+    const SceneView &S = scene_at<B>(S0, A, req_at<B>(A, node_req(nd)).scene);
+    const V3 P = V3{nd.px, nd.py, nd.pz};
+    const LightTerm lt = light_term(S.lights[li], P);
+    sr.r.o = P;
+    sr.r.d = lt.p2l;
+    sr.type = RAY_SHADOW;
+    sr.inside = 0;
+    sr.src = node_id(nd);
+    sr.self_test = 0;
+    dis = lt.dis;
+    return S;
+}
+
+// Shadow tests of the queue's entries, a lane per entry walked on its own.
+template <bool B>
+__device__ inline void occlude_lanes(const SceneView &S0, const WaveArgs &A, const WNode *nodes,
+                                       const unsigned *shadow, int n, LineCtr *sched, unsigned *masks, DevStack &st) {
+    WaveQueue wq(sched, n, A.grab_lg);
     for (int base = wq.next(); base >= 0; base = wq.next()) {
-        const int j = base + (Q ? __lane_id() / kQuadLanes : __lane_id());
+        const int j = base + __lane_id();
         if (j >= n) continue;
         const unsigned e = shadow[j];
-        const int i = (int)(e >> 5), li = (int)(e & 31);
-        const WNode nd = nodes[i];
-        const SceneView &S = scene_at<B>(S0, A, req_at<B>(A, node_req(nd)).scene);
-        const V3 P = V3{nd.px, nd.py, nd.pz};
-        const LightTerm lt = light_term(S.lights[li], P);
         TraceRay sr;
-        sr.r.o = P;
-        sr.r.d = lt.p2l;
-        sr.type = RAY_SHADOW;
-        sr.inside = 0;
-        sr.src = node_id(nd);
-        sr.self_test = 0;
-        if constexpr (Q) {
-            if (quad_any(S, sr, lt.dis, st) && (threadIdx.x & (kQuadLanes - 1)) == 0) atomicOr(&masks[i], 1u << li);
-        } else {
-            if (trace_any(S, sr, lt.dis, st)) atomicOr(&masks[i], 1u << li);
-        }
+        float dis;
+        const SceneView &S = entry_ray<B>(S0, A, nodes, e, sr, dis);
+        if (trace_any(S, sr, dis, st)) atomicOr(&masks[e >> 5], 1u << (e & 31));
     }
 }
 
+// Shadow tests of the queue's entries, one lane per entry, or with `quads` four.
 template <bool B>
-__global__ __launch_bounds__(kBlockThreads, 8) void k_occlude(SceneView S0, WaveArgs A, const WNode *nodes,
-                                                           const unsigned *shadow, LevelCtr *ctr, unsigned *masks) {
+__device__ inline void occlude_entries(bool quads, const SceneView &S0, const WaveArgs &A, const WNode *nodes,
+                                       const unsigned *shadow, int n, LineCtr *sched, unsigned *masks, DevStack &st,
+                                       int *lds) {
+    WaveQueue wq(sched, n, quads ? 0 : A.grab_lg, quads ? 4 : 6);
+    const bool writer = !quads || (threadIdx.x & (kQuadLanes - 1)) == 0;
+    for (int base = wq.next(); base >= 0; base = wq.next()) {
+        const int j = base + (quads ? __lane_id() / kQuadLanes : __lane_id());
+        const bool valid = j < n;
+        const unsigned e = shadow[valid ? j : base];  // (past the end: an entry again, not walked)
+        TraceRay sr;
+        float dis;
+        const SceneView &S = entry_ray<B>(S0, A, nodes, e, sr, dis);
+        if (wave_any<!B>(quads, S, sr, dis, st, lds, valid) && valid && writer)
+            atomicOr(&masks[e >> 5], 1u << (e & 31));
+    }
+}
+
+template <bool B, Walk W>
+__global__ __launch_bounds__(kBlockThreads, W == WALK_WAVE ? 6 : 8)
+void k_occlude(SceneView S0, WaveArgs A, const WNode *nodes, const unsigned *shadow, LevelCtr *ctr, unsigned *masks) {
     const int n = (int)ctr->n_shadow.v;
-    const bool quads = n <= A.quad_max;
+    const bool quads = W == WALK_WAVE && n <= A.quad_max;
     if (quads ? surplus_block<4>(n) : surplus_block(n)) return;
     __shared__ int lds[kLdsStack * kBlockThreads];
     DevStack st = make_stack(lds, A.spill);
@@ -591,12 +681,10 @@ __global__ __launch_bounds__(kBlockThreads, 8) void k_occlude(SceneView S0, Wave
         stack_top_nodes(st, top_nodes, S0);
     }
     if (wave_cancelled(A)) return;
-    if (quads) {
-        QuadStack qs(st, lds);
-        occlude_entries<B, true>(S0, A, nodes, shadow, n, ctr->sched[2], masks, qs);
-    } else {
-        occlude_entries<B, false>(S0, A, nodes, shadow, n, ctr->sched[2], masks, st);
-    }
+    if constexpr (W == WALK_WAVE)
+        occlude_entries<B>(quads, S0, A, nodes, shadow, n, ctr->sched[2], masks, st, lds);
+    else
+        occlude_lanes<B>(S0, A, nodes, shadow, n, ctr->sched[2], masks, st);
 }
 
 // Local lighting of node i from its light mask, over its texel colour.
@@ -649,7 +737,7 @@ struct StepArgs {
     const unsigned *n_lit;  // null: level 0
     const unsigned *lit_masks;
 };
-__global__ __launch_bounds__(kBlockThreads, 6) void k_step(WaveArgs A, StepArgs T) {
+__global__ __launch_bounds__(kBlockThreads, 4) void k_step(WaveArgs A, StepArgs T) {
     const SceneView S0{};  // (batches: every ray's scene is in A.scenes)
     const int n = T.rays ? (int)*T.n_rays : 0, ns = (int)T.ctr->n_shadow.v;
     const int nl = T.lit ? (T.n_lit ? (int)*T.n_lit : A.n_samples) : 0;
@@ -660,22 +748,9 @@ __global__ __launch_bounds__(kBlockThreads, 6) void k_step(WaveArgs A, StepArgs 
     if (b2 >= ce + co && (int)blockIdx.x >= cl) return;
     __shared__ int lds[kLdsStack * kBlockThreads];
     DevStack st = make_stack(lds, A.spill);
-    if (b2 < ce) {
-        if (qe) {
-            QuadStack qs(st, lds);
-            extend_rays<true, false, true>(S0, A, T.k, T.rays, n, T.hits, T.cs, T.sched, qs);
-        } else {
-            extend_rays<true, false, false>(S0, A, T.k, T.rays, n, T.hits, T.cs, T.sched, st);
-        }
-    }
-    if (b2 < ce + co && ns > 0) {
-        if (qo) {
-            QuadStack qs(st, lds);
-            occlude_entries<true, true>(S0, A, T.nodes, T.shadow, ns, T.ctr->sched[2], T.masks, qs);
-        } else {
-            occlude_entries<true, false>(S0, A, T.nodes, T.shadow, ns, T.ctr->sched[2], T.masks, st);
-        }
-    }
+    if (b2 < ce) extend_rays<true>(qe, S0, A, T.k, T.rays, n, T.hits, T.cs, T.sched, st, lds);
+    if (b2 < ce + co && ns > 0)
+        occlude_entries<true>(qo, S0, A, T.nodes, T.shadow, ns, T.ctr->sched[2], T.masks, st, lds);
     for (int c = blockIdx.x; c < cl; c += gridDim.x) {
         const int i = c * kBlockThreads + threadIdx.x;
         if (i < nl) light_in_place<true>(S0, A, T.lit, T.lit_masks, i);
@@ -915,6 +990,12 @@ constexpr int kNoSyncMaxSamples = 1 << 22;
 // Level-0 samples per pass of a frame whose rays branch (see launch_wavefront).
 constexpr int kPassSamples = 1 << 21;
 
+// Levels known to hold this many rays are walked lane by lane (Walk): two and
+// more for each lane the GPU has, so that a tail is short beside the rest (us a
+// frame at limits of 2^18, 2^20, 2^22: 1080p 1686, 1735, 1882 of 1756, 1793,
+// 1922; 801x451 at 4 samples 1740, 1733, 1670 of 1840, 1848, 1834).
+constexpr size_t kFullRays = size_t(1) << 20;
+
 // Resident blocks per CU of a kernel at kBlockThreads threads (registers and
 // LDS permitting).
 template <class K>
@@ -926,18 +1007,28 @@ static int blocks_per_cu(K kernel) {
 
 template <bool B>
 struct Grids {
-    int extend, shade, occlude, occlude_alone;
+    int extend, extend_alone, extend_lanes, shade, occlude, occlude_lanes, occlude_alone, occlude_lanes_alone;
     // pct: percent of the resident blocks (at least one block per CU).
     // k_shade takes half that share: its waves mostly wait on their appends
     // and stores, and fewer of them finish sooner (measured).  Shadow rays
     // that run beside no traversal of a next level (the last level's, or all
-    // of them on one stream) take every resident block.
+    // of them on one stream) take every resident block.  A k_extend beside
+    // shadow rays takes three quarters: at 128 registers its resident waves
+    // hold every register of a SIMD, and none is left for k_occlude's (of the
+    // share: all, three quarters, half: 640x480 sphere frame 568, 570, 572 us,
+    // 1080p frame 1735, 1673, 1697, 801x451 at 4 samples 1733, 1782, 1849).
     explicit Grids(int cus, int pct = 100) {
-        static const int oe = blocks_per_cu(k_extend<B, false>), os = blocks_per_cu(k_shade<B>),
-                         oo = blocks_per_cu(k_occlude<B>);
+        static const int oe = blocks_per_cu(k_extend<B, WALK_WAVE>), os = blocks_per_cu(k_shade<B>),
+                         oo = blocks_per_cu(k_occlude<B, WALK_WAVE>), oel = blocks_per_cu(k_extend<B, WALK_LANES>),
+                         ool = blocks_per_cu(k_occlude<B, WALK_LANES>);
         auto part = [&](int o, int p) { return std::max(cus, cus * o * p / 100); };
-        extend = part(oe, pct), shade = part(os, pct / 2), occlude = part(oo, pct), occlude_alone = part(oo, 100);
+        extend_alone = part(oe, pct), extend = part(oe, pct * 3 / 4), extend_lanes = part(oel, pct), shade = part(os, pct / 2);
+        occlude = part(oo, pct), occlude_lanes = part(ool, pct);
+        occlude_alone = part(oo, 100), occlude_lanes_alone = part(ool, 100);
     }
+    // most blocks of a kernel that walks on the render stream, and on a side stream
+    int most() const { return std::max({extend_alone, extend_lanes, occlude_alone, occlude_lanes_alone}); }
+    int most_side() const { return std::max(occlude, occlude_lanes); }
 };
 
 // Shape of a wavefront: what bounds its queues.
@@ -1002,9 +1093,9 @@ static int reserve_level(Workspace &ws, const WavePlan &pl, int k, size_t n_k) {
 static int reserve_all(Workspace &ws, const WavePlan &pl, int cus) {
     const Grids<false> g0(cus);
     const Grids<true> g1(cus);
-    const int gmax = std::max(std::max(g0.extend, g0.occlude_alone), std::max(g1.extend, g1.occlude_alone));
+    const int gmax = std::max(g0.most(), g1.most());
     if (ws.grow(ws.spill, spill_ints(gmax) * sizeof(int))) return fail(RTG_E_NOMEM, "spill");
-    if (ws.grow(ws.spill2, spill_ints(std::max(g0.occlude, g1.occlude)) * sizeof(int)))
+    if (ws.grow(ws.spill2, spill_ints(std::max(g0.most_side(), g1.most_side())) * sizeof(int)))
         return fail(RTG_E_NOMEM, "spill");
     if (ws.grow(ws.w_qcount, (size_t)kPassCtrWords * sizeof(unsigned))) return fail(RTG_E_NOMEM, "counters");
     if (ws.grow(ws.w_samples, (size_t)pl.n_samples * sizeof(float4))) return fail(RTG_E_NOMEM, "samples");
@@ -1028,7 +1119,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     const int cus = A.cus > 0 ? A.cus : 256;
     const Grids<B> g(cus, A.tune.grid_pct);
     if (!pl.no_sync) {
-        if (ws.grow(ws.spill, spill_ints(std::max(g.extend, g.occlude_alone)) * sizeof(int)))
+        if (ws.grow(ws.spill, spill_ints(g.most()) * sizeof(int)))
             return fail(RTG_E_NOMEM, "spill");
         if (ws.grow(ws.w_qcount, (size_t)kPassCtrWords * sizeof(unsigned)))
             return fail(RTG_E_NOMEM, "queue counters");
@@ -1050,7 +1141,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     if (ov) {
         int st = ws.side_init();
         if (st != RTG_OK) return st;
-        if (ws.grow(ws.spill2, spill_ints(g.occlude) * sizeof(int))) return fail(RTG_E_NOMEM, "spill");
+        if (ws.grow(ws.spill2, spill_ints(g.most_side()) * sizeof(int))) return fail(RTG_E_NOMEM, "spill");
     }
     hipStream_t so = ov ? ws.side : stream;
     // A large single frame on a caller's stream, all levels enqueued at once,
@@ -1062,7 +1153,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     // do not bound the frame.
     const bool ov2 = !B && ov && pl.no_sync && pl.n_samples >= (1 << 20) && A.stream != nullptr &&
                      A.stream != stream && A.stream != ws.side;
-    if (ov2 && ws.grow(ws.spill3, spill_ints(g.occlude) * sizeof(int))) return fail(RTG_E_NOMEM, "spill");
+    if (ov2 && ws.grow(ws.spill3, spill_ints(g.most_side()) * sizeof(int))) return fail(RTG_E_NOMEM, "spill");
     hipStream_t so2 = ov2 ? A.stream : so;
     bool forked = false, forked2 = false;  // a side stream took work (the join waits for it)
     auto join = [&]() -> int {
@@ -1118,7 +1209,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             t.n_lit = k == 2 ? nullptr : &ctr[k - 3].n_next.v;
         }
         const size_t items = kQuadLanes * ((rays ? pl.bound[k] : 0) + pl.bound[k - 1] * pl.n_on);
-        k_step<<<grid(g.extend, items), kBlockThreads, 0, stream>>>(args, t);
+        k_step<<<grid(g.extend_alone, items), kBlockThreads, 0, stream>>>(args, t);
     };
     const size_t cap = level_ray_cap(pl.n_on);
     for (int k = 0; k <= pl.max_level && n_k > 0; ++k) {
@@ -1138,14 +1229,20 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         const WRay *rays = k == 0 ? nullptr : ws.w_rays[k].as<WRay>();
         const unsigned *n_ptr = k == 0 ? nullptr : &ctr[k - 1].n_next.v;
         WRay *next = ws.w_rays[k + 1 < Workspace::kLevels ? k + 1 : k].as<WRay>();
+        // known to be that many rays; or a tree that lies in LDS whole, whose
+        // short walks have no tail (640x480 sphere frame 580 -> 543 us)
+        const bool full = (n_k >= kFullRays && (k == 0 || !pl.no_sync)) || (!B && S0.n_nodes <= kTopNodes);
         int kt = ktime_begin(A, stream, KT_EXTEND, n_k);
         if (fused && k > 0)
             step(k, true);
         else if (retest)
-            k_extend<B, true><<<grid(g.extend, n_k), kBlockThreads, 0, stream>>>(
+            k_extend<B, WALK_RETEST><<<grid(g.extend_lanes, n_k), kBlockThreads, 0, stream>>>(
+                S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
+        else if (full)
+            k_extend<B, WALK_LANES><<<grid(g.extend_lanes, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         else
-            k_extend<B, false><<<grid(g.extend, kQuadLanes * n_k), kBlockThreads, 0, stream>>>(
+            k_extend<B, WALK_WAVE><<<grid(ov && k > 0 ? g.extend : g.extend_alone, kQuadLanes * n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         ktime_end(A, stream, kt, n_ptr);
         if (!view || shadows) {
@@ -1170,9 +1267,17 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             if (k == pl.max_level || pl.bound[k + 1] == 0) step(k + 1, false);
         } else if (shadows) {
             kt = ktime_begin(A, sk, KT_OCCLUDE, 0);
-            k_occlude<B><<<grid(side_k ? g.occlude : g.occlude_alone, kQuadLanes * n_k * pl.n_on), kBlockThreads, 0, sk>>>(
-                S0, side_k ? (second ? oargs2 : oargs) : args, ws.w_nodes[k].as<WNode>(),
-                ws.w_shadow[k].as<unsigned>(), ctr + k, ws.w_masks[k].as<unsigned>());
+            const WaveArgs &oa = side_k ? (second ? oargs2 : oargs) : args;
+            if (full)
+                k_occlude<B, WALK_LANES><<<grid(side_k ? g.occlude_lanes : g.occlude_lanes_alone, n_k * pl.n_on),
+                                           kBlockThreads, 0, sk>>>(S0, oa, ws.w_nodes[k].as<WNode>(),
+                                                                   ws.w_shadow[k].as<unsigned>(), ctr + k,
+                                                                   ws.w_masks[k].as<unsigned>());
+            else
+                k_occlude<B, WALK_WAVE><<<grid(side_k ? g.occlude : g.occlude_alone, kQuadLanes * n_k * pl.n_on),
+                                          kBlockThreads, 0, sk>>>(S0, oa, ws.w_nodes[k].as<WNode>(),
+                                                                  ws.w_shadow[k].as<unsigned>(), ctr + k,
+                                                                  ws.w_masks[k].as<unsigned>());
             ktime_end(A, sk, kt, &ctr[k].n_shadow.v);
         }
         // Local lighting of every level but the last, once its shadow rays are
@@ -1254,7 +1359,7 @@ int reserve_frame(Workspace &ws, int W, int H, int spp, int max_level, int fanou
     if (st == RTG_OK) st = ws.side_init();
     if (st != RTG_OK) return st;
     if (ws.grow(ws.tables, ((size_t)W + H) * sizeof(float))) return fail(RTG_E_NOMEM, "tables");
-    if (ws.grow(ws.spill2, spill_ints(Grids<false>(A.cus > 0 ? A.cus : 256).occlude) * sizeof(int)))
+    if (ws.grow(ws.spill2, spill_ints(Grids<false>(A.cus > 0 ? A.cus : 256).most_side()) * sizeof(int)))
         return fail(RTG_E_NOMEM, "spill");
     const size_t samples = frame_samples(W, H, spp, A.tune.tile_lg);
     // what launch_wavefront reserves up front: a no-sync plan of one pass
