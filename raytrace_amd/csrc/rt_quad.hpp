@@ -38,6 +38,12 @@ constexpr int kQuadLanes = 4;
 // of 1854 / 1928 of 1832; burst of 32 requests 1568 of 1954 / 1479 of 1861 /
 // 1532 of 1845.
 constexpr int kQuadRaysPerCu = 24 * 16;
+// Queues of up to this many rays per CU (4,096 on 256 CUs) go four to a wave, a
+// wave on every SIMD, and its twelve other quads take subtrees over from the
+// second round on.  Limits of 4k / 16k / 32k rays, against quads alone: 64x64
+// frame 1.06 / 1.03 / 1.05x, 12 thumbnails in a batch 1.10 / 1.05 / 1.01x, burst
+// of 32 requests 1.04 / 1.02 / 0.96x, 1080p frame 1.00 / 1.00 / 0.99x.
+constexpr int kFewRaysPerCu = 16;
 static_assert(kLdsStack * kQuadLanes + kStackMax - kLdsStack >= kStackMax, "a quad's stack holds any walk");
 
 // Move across the quad: lane k reads lane (k ^ 1), (k ^ 2) or (k ^ 3) of its
@@ -175,8 +181,8 @@ constexpr int kHelpFrom = 8, kHelpAfter = 8;
 // walk without it).
 constexpr int kTailAfter = 4;
 
-// The walks of a wave's rays, bvh_walk<true, kOrdered> with a lane or, with
-// `quads`, a quad per ray: the same postponed leaves and wave-wide exit of the
+// The walks of a wave's 1 << lg rays, bvh_walk<true, kOrdered> with a lane
+// (lg 6) or a quad per ray: the same postponed leaves and wave-wide exit of the
 // node loop.  Every lane of the wave calls it; lanes without a ray come with
 // root kWalkDone.
 //
@@ -197,9 +203,11 @@ constexpr int kTailAfter = 4;
 // the ray hits it.  Any hit: best.t comes as the segment's length; returns
 // whether the segment is blocked.
 template <bool kOrdered, bool kOneScene>
-__device__ inline bool wave_rays(bool quads, const SceneView &S0, const Bvh4Node *nodes, const float4 *prims, int root,
+__device__ inline bool wave_rays(int lg, const SceneView &S0, const Bvh4Node *nodes, const float4 *prims, int root,
                                  TraceRay q, int before, DevStack &ds, int *lds_base, Hit &best, int &self) {
+    const bool quads = lg < 6;
     const int lane = __lane_id(), k = lane & (kQuadLanes - 1), me = lane / kQuadLanes;
+    const int help_after = lg < 4 ? 1 : kHelpAfter;
     const unsigned long long leaders = 0x1111111111111111ull;
     V3 inv = safe_inv(q.r.d);
     float tmax = best.t;
@@ -381,7 +389,7 @@ __device__ inline bool wave_rays(bool quads, const SceneView &S0, const Bvh4Node
         const bool busy = node != kWalkDone || leaf < 0;
         const unsigned long long idle = ~__ballot(busy) & leaders;
         if (idle == leaders) break;
-        if (round >= kHelpAfter && __popcll(idle) >= kHelpFrom) {
+        if (round >= help_after && __popcll(idle) >= kHelpFrom) {
             const bool spare = busy && st.sp - st.base > 1 && st.base + 1 < QuadStack::kLds;
             const unsigned long long give = __ballot(spare) & leaders;
             if (give != 0ull) {
@@ -509,11 +517,11 @@ __device__ inline bool wave_rays(bool quads, const SceneView &S0, const Bvh4Node
     return blocked != 0;
 }
 
-// trace_closest<false, true> and trace_any of the wave's rays (those of lanes
-// with `valid`), a lane or, with `quads`, a quad per ray.  All lanes of the
+// trace_closest<false, true> and trace_any of the wave's 1 << lg rays (those of
+// lanes with `valid`), a lane or, with lg < 6, a quad per ray.  All lanes of the
 // wave call it; every lane of a quad gets its ray's answer.
 template <bool kOneScene>
-__device__ inline Hit wave_closest(bool quads, const SceneView &S, const TraceRay &q, DevStack &st, int *lds, int before,
+__device__ inline Hit wave_closest(int lg, const SceneView &S, const TraceRay &q, DevStack &st, int *lds, int before,
                                    bool valid) {
     Hit best{kMiss, HIT_NONE, -1, -1, 0, 0, 0};
     int root = kWalkDone, self;
@@ -523,12 +531,12 @@ __device__ inline Hit wave_closest(bool quads, const SceneView &S, const TraceRa
         brute_objects(S, q, false, 0.0f, best, before);
         if (S.n_prims > 0) root = S.root, nodes = S.nodes, prims = S.prims;
     }
-    wave_rays<true, kOneScene>(quads, S, nodes, prims, root, q, before, st, lds, best, self);
+    wave_rays<true, kOneScene>(lg, S, nodes, prims, root, q, before, st, lds, best, self);
     if (self) take_source_hit(S, q, self - 1, before, best, best.kind != HIT_NONE ? hit_key(best.obj, best.prim) : ~0ull);
     return best;
 }
 template <bool kOneScene>
-__device__ inline bool wave_any(bool quads, const SceneView &S, const TraceRay &q, float dis, DevStack &st, int *lds,
+__device__ inline bool wave_any(int lg, const SceneView &S, const TraceRay &q, float dis, DevStack &st, int *lds,
                                 bool valid) {
     Hit best{dis, HIT_NONE, -1, -1, 0, 0, 0};
     int root = kWalkDone, self;
@@ -540,7 +548,7 @@ __device__ inline bool wave_any(bool quads, const SceneView &S, const TraceRay &
         blocked = brute_objects(S, q, true, dis, dummy);
         if (S.n_prims > 0 && !blocked) root = S.root, nodes = S.nodes, prims = S.prims;
     }
-    if (wave_rays<false, kOneScene>(quads, S, nodes, prims, root, q, 0, st, lds, best, self)) blocked = true;
+    if (wave_rays<false, kOneScene>(lg, S, nodes, prims, root, q, 0, st, lds, best, self)) blocked = true;
     return blocked || (self && self_testable(S, q.r, q.src, dis));
 }
 

@@ -94,7 +94,7 @@ struct WaveArgs {
     const int *chunk_req;     // B = true: request of each 64-sample chunk of level 0 (-1: padding)
     int n_samples;            // level-0 queue length
     int grab_lg;              // WaveQueue grabs of 64 << grab_lg items
-    int quad_max;  // longest queue walked with four lanes per ray (rt_quad.hpp)
+    int quad_max, few_max;  // longest queues walked with four and with sixteen lanes per ray (rt_quad.hpp)
     unsigned long long *counts;
     unsigned long long *retests;  // closest-hit queries re-tested in FP64
     int *spill;
@@ -216,14 +216,18 @@ __device__ inline int sample_req(const WaveArgs &A, int i) {
         return 0;
 }
 
+// log2 of the rays a wave starts with, for a queue of n: a lane, four lanes or
+// sixteen lanes per ray (rt_quad.hpp).
+__device__ inline int walk_lg(const WaveArgs &A, int n) { return n <= A.few_max ? 2 : n <= A.quad_max ? 4 : 6; }
+
 // A persistent traversal grid is sized for the level's bound, and the deep
 // levels hold far fewer items: a block whose waves would each start past the
-// last 64-item chunk finds no work, and leaves before copying the top nodes
-// into LDS (block-uniform, so ahead of the barrier there).  The blocks that
-// stay take every chunk: waves keep grabbing until the queue is empty.
-template <int kStepLg = 6>
-__device__ inline bool surplus_block(int n) {
-    return (int)blockIdx.x * (kBlockThreads / 64) >= ((n + (1 << kStepLg) - 1) >> kStepLg);
+// last chunk (1 << step_lg items) finds no work, and leaves before copying the
+// top nodes into LDS (block-uniform, so ahead of the barrier there).  The blocks
+// that stay take every chunk: waves keep grabbing until the queue is empty.
+__device__ inline int chunks_of(int n, int step_lg) { return (n + (1 << step_lg) - 1) >> step_lg; }
+__device__ inline bool surplus_block(int n, int step_lg = 6) {
+    return (int)blockIdx.x * (kBlockThreads / 64) >= chunks_of(n, step_lg);
 }
 
 // Grab size (64 << lg items) for n items: the tuning's, doubled up to eight
@@ -323,16 +327,18 @@ __device__ inline void extend_lanes(const SceneView &S0, const WaveArgs &A, int 
     }
 }
 
-// Closest hits of the queue's rays, one lane per ray, or with `quads` four (lane
-// 0 of the quad writes); the whole wave goes through every step (rt_quad.hpp).
+// Closest hits of the queue's rays, 1 << lg of them to a wave (walk_lg; with
+// quads, lane 0 writes); the whole wave goes through every step (rt_quad.hpp).
 template <bool B>
-__device__ inline void extend_rays(bool quads, const SceneView &S0, const WaveArgs &A, int k, const WRay *rays, int n,
+__device__ inline void extend_rays(int lg, const SceneView &S0, const WaveArgs &A, int k, const WRay *rays, int n,
                                    WHit *hits, int4 *cs, LineCtr *sched, DevStack &st, int *lds) {
-    WaveQueue wq(sched, n, quads ? 0 : A.grab_lg, quads ? 4 : 6);
+    const bool quads = lg < 6;
+    WaveQueue wq(sched, n, quads ? 0 : A.grab_lg, lg);
     uint32_t c_prim = 0, c_refl = 0, c_refr = 0;
     const bool writer = !quads || (threadIdx.x & (kQuadLanes - 1)) == 0;
+    const int slot = quads ? __lane_id() / kQuadLanes : __lane_id();
     for (int base = wq.next(); base >= 0; base = wq.next()) {
-        const int i = base + (quads ? __lane_id() / kQuadLanes : __lane_id());
+        const int i = slot < (1 << lg) ? base + slot : n;
         TraceRay q{};
         q.src = no_src();
         bool valid = false;
@@ -346,7 +352,7 @@ __device__ inline void extend_rays(bool quads, const SceneView &S0, const WaveAr
         int before = 0x7fffffff;
         bool walks = valid;
         for (int pass = 0;; ++pass) {
-            const Hit h = wave_closest<!B>(quads, S, q, st, lds, before, walks);
+            const Hit h = wave_closest<!B>(lg, S, q, st, lds, before, walks);
             if (pass == 1) {
                 if (walks && writer) {
                     const SrcId c = child_src_of(S, q, h);
@@ -390,8 +396,8 @@ __global__ __launch_bounds__(kBlockThreads, W == WALK_WAVE ? 4 : 6)
 void k_extend(SceneView S0, WaveArgs A, int k, const WRay *rays, const unsigned *n_ptr, WHit *hits, int4 *cs,
               LineCtr *sched) {
     const int n = k == 0 ? A.n_samples : (int)*n_ptr;
-    const bool quads = W == WALK_WAVE && n <= A.quad_max;
-    if (quads ? surplus_block<4>(n) : surplus_block(n)) return;
+    const int lg = W == WALK_WAVE ? walk_lg(A, n) : 6;
+    if (surplus_block(n, lg)) return;
     __shared__ int lds[kLdsStack * kBlockThreads];
     DevStack st = make_stack(lds, A.spill);
     if constexpr (!B) {  // one scene: its top nodes in LDS
@@ -400,7 +406,7 @@ void k_extend(SceneView S0, WaveArgs A, int k, const WRay *rays, const unsigned 
     }
     if (wave_cancelled(A)) return;
     if constexpr (W == WALK_WAVE)
-        extend_rays<B>(quads, S0, A, k, rays, n, hits, cs, sched, st, lds);
+        extend_rays<B>(lg, S0, A, k, rays, n, hits, cs, sched, st, lds);
     else
         extend_lanes<B, W == WALK_RETEST>(S0, A, k, rays, n, hits, cs, sched, st);
 }
@@ -649,21 +655,23 @@ __device__ inline void occlude_lanes(const SceneView &S0, const WaveArgs &A, con
     }
 }
 
-// Shadow tests of the queue's entries, one lane per entry, or with `quads` four.
+// Shadow tests of the queue's entries, 1 << lg of them to a wave.
 template <bool B>
-__device__ inline void occlude_entries(bool quads, const SceneView &S0, const WaveArgs &A, const WNode *nodes,
+__device__ inline void occlude_entries(int lg, const SceneView &S0, const WaveArgs &A, const WNode *nodes,
                                        const unsigned *shadow, int n, LineCtr *sched, unsigned *masks, DevStack &st,
                                        int *lds) {
-    WaveQueue wq(sched, n, quads ? 0 : A.grab_lg, quads ? 4 : 6);
+    const bool quads = lg < 6;
+    WaveQueue wq(sched, n, quads ? 0 : A.grab_lg, lg);
     const bool writer = !quads || (threadIdx.x & (kQuadLanes - 1)) == 0;
+    const int slot = quads ? __lane_id() / kQuadLanes : __lane_id();
     for (int base = wq.next(); base >= 0; base = wq.next()) {
-        const int j = base + (quads ? __lane_id() / kQuadLanes : __lane_id());
-        const bool valid = j < n;
+        const int j = base + slot;
+        const bool valid = slot < (1 << lg) && j < n;
         const unsigned e = shadow[valid ? j : base];  // (past the end: an entry again, not walked)
         TraceRay sr;
         float dis;
         const SceneView &S = entry_ray<B>(S0, A, nodes, e, sr, dis);
-        if (wave_any<!B>(quads, S, sr, dis, st, lds, valid) && valid && writer)
+        if (wave_any<!B>(lg, S, sr, dis, st, lds, valid) && valid && writer)
             atomicOr(&masks[e >> 5], 1u << (e & 31));
     }
 }
@@ -672,8 +680,8 @@ template <bool B, Walk W>
 __global__ __launch_bounds__(kBlockThreads, W == WALK_WAVE ? 6 : 8)
 void k_occlude(SceneView S0, WaveArgs A, const WNode *nodes, const unsigned *shadow, LevelCtr *ctr, unsigned *masks) {
     const int n = (int)ctr->n_shadow.v;
-    const bool quads = W == WALK_WAVE && n <= A.quad_max;
-    if (quads ? surplus_block<4>(n) : surplus_block(n)) return;
+    const int lg = W == WALK_WAVE ? walk_lg(A, n) : 6;
+    if (surplus_block(n, lg)) return;
     __shared__ int lds[kLdsStack * kBlockThreads];
     DevStack st = make_stack(lds, A.spill);
     if constexpr (!B) {  // one scene: its top nodes in LDS
@@ -682,7 +690,7 @@ void k_occlude(SceneView S0, WaveArgs A, const WNode *nodes, const unsigned *sha
     }
     if (wave_cancelled(A)) return;
     if constexpr (W == WALK_WAVE)
-        occlude_entries<B>(quads, S0, A, nodes, shadow, n, ctr->sched[2], masks, st, lds);
+        occlude_entries<B>(lg, S0, A, nodes, shadow, n, ctr->sched[2], masks, st, lds);
     else
         occlude_lanes<B>(S0, A, nodes, shadow, n, ctr->sched[2], masks, st);
 }
@@ -741,16 +749,15 @@ __global__ __launch_bounds__(kBlockThreads, 4) void k_step(WaveArgs A, StepArgs 
     const SceneView S0{};  // (batches: every ray's scene is in A.scenes)
     const int n = T.rays ? (int)*T.n_rays : 0, ns = (int)T.ctr->n_shadow.v;
     const int nl = T.lit ? (T.n_lit ? (int)*T.n_lit : A.n_samples) : 0;
-    const bool qe = n <= A.quad_max, qo = ns <= A.quad_max;
-    const int ce = qe ? (n + 15) >> 4 : (n + 63) >> 6, co = qo ? (ns + 15) >> 4 : (ns + 63) >> 6;
+    const int lge = walk_lg(A, n), lgo = walk_lg(A, ns), ce = chunks_of(n, lge), co = chunks_of(ns, lgo);
     const int b2 = (int)blockIdx.x * (kBlockThreads / 64);  // waves before this block's
     const int cl = (nl + kBlockThreads - 1) / kBlockThreads;
     if (b2 >= ce + co && (int)blockIdx.x >= cl) return;
     __shared__ int lds[kLdsStack * kBlockThreads];
     DevStack st = make_stack(lds, A.spill);
-    if (b2 < ce) extend_rays<true>(qe, S0, A, T.k, T.rays, n, T.hits, T.cs, T.sched, st, lds);
+    if (b2 < ce) extend_rays<true>(lge, S0, A, T.k, T.rays, n, T.hits, T.cs, T.sched, st, lds);
     if (b2 < ce + co && ns > 0)
-        occlude_entries<true>(qo, S0, A, T.nodes, T.shadow, ns, T.ctr->sched[2], T.masks, st, lds);
+        occlude_entries<true>(lgo, S0, A, T.nodes, T.shadow, ns, T.ctr->sched[2], T.masks, st, lds);
     for (int c = blockIdx.x; c < cl; c += gridDim.x) {
         const int i = c * kBlockThreads + threadIdx.x;
         if (i < nl) light_in_place<true>(S0, A, T.lit, T.lit_masks, i);
@@ -1176,13 +1183,17 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     auto grid = [](int gmax, size_t items) {
         return (int)std::max<size_t>(8, std::min<size_t>(gmax, (items + 127) / 128));
     };
+    // lanes of a queue of up to n rays: sixteen a ray for the few, then four
+    auto lanes_of = [&](size_t n) {
+        return kQuadLanes * std::max(n, kQuadLanes * std::min<size_t>(n, cus * kFewRaysPerCu));
+    };
     // k_local, k_combine: at most 16 blocks per CU, no more than the level's
     // bound needs (the blocks of an empty 4096-block grid take 4-5 us to
     // dispatch); whole eighths (xcd_chunks)
     auto lgrid = [&](size_t items) { return (std::min(cus * 16, grid(cus * 16, items)) + 7) & ~7; };
     WaveArgs args = a;
     args.spill = ws.spill.as<int>();
-    args.quad_max = cus * kQuadRaysPerCu;
+    args.quad_max = cus * kQuadRaysPerCu, args.few_max = cus * kFewRaysPerCu;
     args.cancel = cancel ? cancel->dev : nullptr;
     args.abort = ws.w_qcount.as<unsigned>() + Workspace::kLevels * kCtrWords;
     WaveArgs oargs = args, oargs2 = args;
@@ -1208,7 +1219,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             t.lit = ws.w_nodes[k - 2].as<WNode>(), t.lit_masks = ws.w_masks[k - 2].as<unsigned>();
             t.n_lit = k == 2 ? nullptr : &ctr[k - 3].n_next.v;
         }
-        const size_t items = kQuadLanes * ((rays ? pl.bound[k] : 0) + pl.bound[k - 1] * pl.n_on);
+        const size_t items = (rays ? lanes_of(pl.bound[k]) : 0) + lanes_of(pl.bound[k - 1] * pl.n_on);
         k_step<<<grid(g.extend_alone, items), kBlockThreads, 0, stream>>>(args, t);
     };
     const size_t cap = level_ray_cap(pl.n_on);
@@ -1242,7 +1253,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             k_extend<B, WALK_LANES><<<grid(g.extend_lanes, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         else
-            k_extend<B, WALK_WAVE><<<grid(ov && k > 0 ? g.extend : g.extend_alone, kQuadLanes * n_k), kBlockThreads, 0, stream>>>(
+            k_extend<B, WALK_WAVE><<<grid(ov && k > 0 ? g.extend : g.extend_alone, lanes_of(n_k)), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         ktime_end(A, stream, kt, n_ptr);
         if (!view || shadows) {
@@ -1274,7 +1285,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
                                                                    ws.w_shadow[k].as<unsigned>(), ctr + k,
                                                                    ws.w_masks[k].as<unsigned>());
             else
-                k_occlude<B, WALK_WAVE><<<grid(side_k ? g.occlude : g.occlude_alone, kQuadLanes * n_k * pl.n_on),
+                k_occlude<B, WALK_WAVE><<<grid(side_k ? g.occlude : g.occlude_alone, lanes_of(n_k * pl.n_on)),
                                           kBlockThreads, 0, sk>>>(S0, oa, ws.w_nodes[k].as<WNode>(),
                                                                   ws.w_shadow[k].as<unsigned>(), ctr + k,
                                                                   ws.w_masks[k].as<unsigned>());

@@ -1,7 +1,7 @@
 """The walks of a level (rtg_wave.hip, Walk): lane by lane where a level is
 known to hold 2^20 rays or the tree lies in LDS whole, else the wave's rays
 together, whose last 16 go on with four lanes each and whose idle lanes take
-subtrees over (rt_quad.hpp).  Around the limits, and with a few slow rays among
+subtrees over (rt_quad.hpp); four rays to a wave up to 4096.  Around the limits, and with a few slow rays among
 quick ones, frames must equal the megakernel's, which always walks one ray per
 lane on its own, bit for bit."""
 from __future__ import annotations
@@ -32,7 +32,7 @@ def _spheres(rt, n):
 @pytest.mark.parametrize("scene,size", [
     ("spheres 0", (97, 61)), ("spheres 1", (97, 61)), ("spheres 3", (97, 61)), ("spheres 30", (200, 133)),
     ("spheres 130", (200, 133)), ("spheres 600", (1024, 1023)), ("soup", (1024, 1023)), ("soup", (1024, 1024)),
-    ("field", (640, 401))], ids=lambda v: v if isinstance(v, str) else "%dx%d" % v)
+    ("field", (640, 401)), ("soup", (64, 64)), ("soup", (65, 64)), ("field", (64, 60))], ids=lambda v: v if isinstance(v, str) else "%dx%d" % v)
 def test_walks_equal_single_rays(rt_gpu, scene, size):
     rt = rt_gpu
     if scene.startswith("spheres"):
