@@ -1026,8 +1026,8 @@ struct Grids {
     // 1080p frame 1735, 1673, 1697, 801x451 at 4 samples 1733, 1782, 1849).
     explicit Grids(int cus, int pct = 100) {
         static const int oe = blocks_per_cu(k_extend<B, WALK_WAVE>), os = blocks_per_cu(k_shade<B>),
-                         oo = blocks_per_cu(k_occlude<B, WALK_WAVE>), oel = blocks_per_cu(k_extend<B, WALK_LANES>),
-                         ool = blocks_per_cu(k_occlude<B, WALK_LANES>);
+                         oo = blocks_per_cu(k_occlude<B, WALK_WAVE>), oel = blocks_per_cu(k_extend<B, B ? WALK_RETEST : WALK_LANES>),
+                         ool = blocks_per_cu(k_occlude<B, B ? WALK_WAVE : WALK_LANES>);
         auto part = [&](int o, int p) { return std::max(cus, cus * o * p / 100); };
         extend_alone = part(oe, pct), extend = part(oe, pct * 3 / 4), extend_lanes = part(oel, pct), shade = part(os, pct / 2);
         occlude = part(oo, pct), occlude_lanes = part(ool, pct);
@@ -1241,8 +1241,10 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         const unsigned *n_ptr = k == 0 ? nullptr : &ctr[k - 1].n_next.v;
         WRay *next = ws.w_rays[k + 1 < Workspace::kLevels ? k + 1 : k].as<WRay>();
         // known to be that many rays; or a tree that lies in LDS whole, whose
-        // short walks have no tail (640x480 sphere frame 580 -> 543 us)
-        const bool full = (n_k >= kFullRays && (k == 0 || !pl.no_sync)) || (!B && S0.n_nodes <= kTopNodes);
+        // short walks have no tail (640x480 sphere frame 580 -> 543 us).  Not
+        // batches: their scenes' trees differ, and so do their rays' walks
+        // (60 mixed requests 5730 -> 5616 us with level 0 walked together)
+        const bool full = !B && ((n_k >= kFullRays && (k == 0 || !pl.no_sync)) || S0.n_nodes <= kTopNodes);
         int kt = ktime_begin(A, stream, KT_EXTEND, n_k);
         if (fused && k > 0)
             step(k, true);
@@ -1250,7 +1252,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             k_extend<B, WALK_RETEST><<<grid(g.extend_lanes, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         else if (full)
-            k_extend<B, WALK_LANES><<<grid(g.extend_lanes, n_k), kBlockThreads, 0, stream>>>(
+            k_extend<false, WALK_LANES><<<grid(g.extend_lanes, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         else
             k_extend<B, WALK_WAVE><<<grid(ov && k > 0 ? g.extend : g.extend_alone, lanes_of(n_k)), kBlockThreads, 0, stream>>>(
@@ -1280,7 +1282,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             kt = ktime_begin(A, sk, KT_OCCLUDE, 0);
             const WaveArgs &oa = side_k ? (second ? oargs2 : oargs) : args;
             if (full)
-                k_occlude<B, WALK_LANES><<<grid(side_k ? g.occlude_lanes : g.occlude_lanes_alone, n_k * pl.n_on),
+                k_occlude<false, WALK_LANES><<<grid(side_k ? g.occlude_lanes : g.occlude_lanes_alone, n_k * pl.n_on),
                                            kBlockThreads, 0, sk>>>(S0, oa, ws.w_nodes[k].as<WNode>(),
                                                                    ws.w_shadow[k].as<unsigned>(), ctr + k,
                                                                    ws.w_masks[k].as<unsigned>());
