@@ -245,10 +245,10 @@ void ktime_end(Arena &A, hipStream_t s, int rec, const unsigned *dev_items) {
     }
 }
 
-// Render one frame into device outputs; the caller holds A.lock.  `cancel`:
-// the job's cancel flag (asynchronous jobs), else null.
-static int render_device(SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                         Arena &A, const Cancel *cancel) {
+// Check a frame's parameters and enqueue it; what it clears is emptied from
+// `init` once that is enqueued.
+static int enqueue_frame(SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
+                         Arena &A, const Cancel *cancel, FrameInit &init) {
     A.ktimes = (p.flags & RTG_FLAG_KERNEL_TIMES) != 0;
     if (A.ktimes && A.kitems_host == nullptr)
         RTG_HIP(hipHostMalloc(reinterpret_cast<void **>(&A.kitems_host), Arena::kItemSlots * sizeof(unsigned),
@@ -270,10 +270,22 @@ static int render_device(SceneRes &S, const rtg_params &p, int W, int H, const R
     int st = A.ws.order_before(stream);
     if (st != RTG_OK) return st;
     st = engine == RTG_ENGINE_WAVEFRONT
-             ? launch_wavefront(S, p, W, H, o, stream, A.ws, A, cancel, init_of(o, W, H))
-             : launch_megakernel(S, p, W, H, o, stream, A, cancel);
+             ? launch_wavefront(S, p, W, H, o, stream, A.ws, A, cancel, init)
+             : launch_megakernel(S, p, W, H, o, stream, A, cancel, init);
     const int st2 = A.ws.mark_done(stream);
     return st != RTG_OK ? st : st2;
+}
+
+// Render one frame into device outputs; the caller holds A.lock.  `cancel`:
+// the job's cancel flag (asynchronous jobs), else null.  A frame that is
+// refused, or fails before its first kernel, leaves its outputs cleared: the
+// host entry points copy them out whatever became of the frame.
+static int render_device(SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
+                         Arena &A, const Cancel *cancel) {
+    FrameInit init = init_of(o, W, H);
+    const int st = enqueue_frame(S, p, W, H, o, stream, A, cancel, init);
+    if (st != RTG_OK && init.rgb != nullptr) (void)launch_init(init, nullptr, 0, stream);
+    return st;
 }
 
 }  // namespace rtg
@@ -789,8 +801,8 @@ int rtg_render_batch(const rtg_request *reqs, int n, rtg_stats *stats) {
         const int e = batch_group_end(samples.data(), n, b, cap);
         if (e == b + 1 && batch_bucket(samples[b]) > cap) {
             const RenderOut o{items[b].rgb, items[b].ids, nullptr, counts, counts + 4};
-            st = launch_wavefront(*items[b].scene, items[b].params, items[b].W, items[b].H, o, s, A.ws, A, nullptr,
-                                  FrameInit{});
+            FrameInit none;
+            st = launch_wavefront(*items[b].scene, items[b].params, items[b].W, items[b].H, o, s, A.ws, A, nullptr, none);
         } else {
             int rep = 0;
             st = launch_batch(items.data() + b, e - b, counts, counts + 4, s, A.ws, A, eager ? 0 : 1, &rep);
@@ -901,7 +913,7 @@ int rtg_autotune(const rtg_request *reqs, int n, int reps, rtg_tuning *best, rtg
     hipStream_t s = A.stream;
     unsigned long long *counts = A.counters.as<unsigned long long>();
     auto run = [&]() -> int {
-        const FrameInit zero{nullptr, 0, nullptr, 0, counts, counts + 4};
+        FrameInit zero{nullptr, 0, nullptr, 0, counts, counts + 4};
         int st = A.ws.order_before(s);
         if (st != RTG_OK) return st;
         if (n == 1) {

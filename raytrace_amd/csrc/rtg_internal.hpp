@@ -273,7 +273,9 @@ struct RenderOut {
 
 // What the first kernel of a frame or batch clears: RGB to 127 (the reference
 // clears its output to it, RayTracer.cpp:620), ids to -1, the ray counts (and
-// the FP64 re-test count) to 0.  Null pointers are left out.
+// the FP64 re-test count) to 0.  Null pointers are left out.  A launch that
+// takes one by reference empties it once it enqueued the kernel: what is still
+// in it after a failed launch has not been cleared (render_device then does).
 struct FrameInit {
     uint8_t *rgb = nullptr;
     size_t rgb_bytes = 0;
@@ -306,7 +308,7 @@ struct Cancel {
 // Launch one frame of the megakernel on `stream` (asynchronous); `cancel`
 // may be null.
 int launch_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                      Arena &A, const Cancel *cancel);
+                      Arena &A, const Cancel *cancel, FrameInit &init);
 // The megakernel's scratch: ray-generation tables (W + H floats, written for
 // the frame's W, H and `dp`), the traversal stacks' spill area for `blocks`
 // persistent blocks (spill_ints(blocks) ints).
@@ -316,10 +318,10 @@ struct MegaScratch {
     int blocks;
     double dp;
 };
-// Enqueue the megakernel with the given scratch (tables already written) and
-// the launch that clears its outputs and counters; allocates nothing.
+// Enqueue the launch that clears `init` and the megakernel with the given
+// scratch (tables already written); allocates nothing.
 int enqueue_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                       Arena &A, const Cancel *cancel, const MegaScratch &ms);
+                       Arena &A, const Cancel *cancel, const MegaScratch &ms, FrameInit &init);
 // Enqueue the ray-generation tables (float)((x - W/2) dp), (float)((y - H/2) dp)
 // into W + H floats at `tab` on `stream`; allocates nothing.
 int write_raygen_tables(float *tab, int W, int H, double dp, hipStream_t stream);
@@ -348,7 +350,7 @@ int reserve_batch(Workspace &ws, size_t samples, int n_reqs, int n_scenes, size_
 // The primary-only modes (depth, normal, texture, material, shadow test) take
 // the same path: level 0's rays, and k_view in place of the shading kernels.
 int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                     Workspace &ws, Arena &A, const Cancel *cancel, const FrameInit &init);
+                     Workspace &ws, Arena &A, const Cancel *cancel, FrameInit &init);
 
 // One request of a batch (rtg_render_batch): a frame of `scene` into device
 // outputs.

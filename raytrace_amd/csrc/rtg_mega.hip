@@ -142,7 +142,7 @@ int upload_raygen_tables(const SceneRes &S, int W, int H, hipStream_t stream, Wo
 int persistent_blocks(const Arena &A) { return std::max(8, (A.cus > 0 ? A.cus : 256) * 8); }
 
 int enqueue_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                       Arena &A, const Cancel *cancel, const MegaScratch &ms) {
+                       Arena &A, const Cancel *cancel, const MegaScratch &ms, FrameInit &init) {
     MegaArgs a;
     a.W = W, a.H = H, a.spp = p.spp > 0 ? p.spp : 1, a.max_level = p.max_level, a.tile_compat = p.tile_compat;
     a.mode = p.mode;
@@ -156,8 +156,9 @@ int enqueue_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, con
     a.counts = o.counts;
     a.cancel = cancel ? cancel->dev : nullptr;
     a.spill = ms.spill;
-    const int st = launch_init(init_of(o, W, H), nullptr, 0, stream);
+    const int st = launch_init(init, nullptr, 0, stream);
     if (st != RTG_OK) return st;
+    init = FrameInit{};
     const int kt = ktime_begin(A, stream, KT_MEGA, (uint64_t)W * H * a.spp);
     k_megakernel<<<ms.blocks, kBlockThreads, 0, stream>>>(S.view, a);
     ktime_end(A, stream, kt);
@@ -166,7 +167,7 @@ int enqueue_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, con
 }
 
 int launch_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                      Arena &A, const Cancel *cancel) {
+                      Arena &A, const Cancel *cancel, FrameInit &init) {
     MegaScratch ms{};
     int st = upload_raygen_tables(S, W, H, stream, A.ws, ms.dp);
     if (st != RTG_OK) return st;
@@ -174,7 +175,7 @@ int launch_megakernel(const SceneRes &S, const rtg_params &p, int W, int H, cons
     if (A.ws.grow(A.ws.spill, spill_ints(ms.blocks) * sizeof(int))) return fail(RTG_E_NOMEM, "spill");
     ms.tables = A.ws.tables.as<float>();
     ms.spill = A.ws.spill.as<int>();
-    return enqueue_megakernel(S, p, W, H, o, stream, A, cancel, ms);
+    return enqueue_megakernel(S, p, W, H, o, stream, A, cancel, ms, init);
 }
 
 }  // namespace rtg

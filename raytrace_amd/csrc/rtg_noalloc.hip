@@ -88,7 +88,8 @@ extern "C" int rtg_render_device_noalloc(rtg_scene_t scene, const rtg_params *pa
     const bool kt = A.ktimes;
     A.ktimes = false;
     const RenderOut o{rgb_dev, ids_dev, tprim_dev, counts, nullptr};
-    st = enqueue_megakernel(scene->res, p, W, H, o, s, A, nullptr, ms);
+    FrameInit init = init_of(o, W, H);
+    st = enqueue_megakernel(scene->res, p, W, H, o, s, A, nullptr, ms, init);
     A.ktimes = kt;
     return st;
 }

@@ -102,7 +102,7 @@ static int slot_launch(ServeSlot &s, rtg_serve_request *reqs, const std::vector<
     int st = slot_reserve(s, bytes);
     if (st != RTG_OK) return st;
     unsigned long long *counts = s.counts.as<unsigned long long>();  // 4 ray counts + FP64 re-tests
-    const FrameInit init{s.out.as<uint8_t>(), bytes, nullptr, 0, counts, counts + 4};
+    FrameInit init{s.out.as<uint8_t>(), bytes, nullptr, 0, counts, counts + 4};
     if (plain || ids.size() == 1) {  // a batch of one takes the single-frame path (uniform kernel arguments)
         const rtg_serve_request &q = reqs[ids[0]];
         const RenderOut o{s.out.as<uint8_t>(), nullptr, nullptr, counts, counts + 4};

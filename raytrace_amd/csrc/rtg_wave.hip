@@ -1119,7 +1119,7 @@ static int reserve_all(Workspace &ws, const WavePlan &pl, int cus) {
 template <bool B>
 static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &pl, hipStream_t stream,
                         Workspace &ws, Arena &A, const Cancel *cancel, bool retest, bool overlap,
-                        const FrameInit &init, int mode) {
+                        FrameInit &init, int mode) {
     const int *cancel_host = cancel ? cancel->host : nullptr;
     const bool view = primary_only(mode);  // (one level) k_view shades the hits
     const bool shadows = pl.n_on > 0 && (!view || mode == RTG_MODE_SHADOWTEST);
@@ -1178,6 +1178,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     {
         const int st = launch_init(init, ws.w_qcount.as<unsigned>(), kPassCtrWords, stream);
         if (st != RTG_OK) return st;
+        init = FrameInit{};  // (later passes of a frame clear only their queue counters)
     }
     const bool early_local = !B && pl.no_sync;
     auto grid = [](int gmax, size_t items) {
@@ -1382,7 +1383,7 @@ int reserve_frame(Workspace &ws, int W, int H, int spp, int max_level, int fanou
 }
 
 int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const RenderOut &o, hipStream_t stream,
-                     Workspace &ws, Arena &A, const Cancel *cancel, const FrameInit &init) {
+                     Workspace &ws, Arena &A, const Cancel *cancel, FrameInit &init) {
     const int *cancel_host = cancel ? cancel->host : nullptr;
     double dp;
     int st = upload_raygen_tables(S, W, H, stream, ws, dp);
@@ -1429,7 +1430,7 @@ int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const
         if (r.n_samples > kNoSyncMaxSamples) pl.no_sync = false;
         if (pl.no_sync && (st = reserve_all(ws, pl, A.cus > 0 ? A.cus : 256)) != RTG_OK) return st;
         st = enqueue_wave<false>(S.view, a, pl, stream, ws, A, cancel, r.retest != 0,
-                                 (p.flags & RTG_FLAG_ONE_STREAM) == 0, row0 == 0 ? init : FrameInit{}, p.mode);
+                                 (p.flags & RTG_FLAG_ONE_STREAM) == 0, init, p.mode);
         if (st != RTG_OK || (cancel_host && *cancel_host)) return st;
     }
     return RTG_OK;
@@ -1585,8 +1586,9 @@ int launch_batch(const BatchItem *items, int n, unsigned long long *counts, unsi
     auto enqueue = [&](bool overlap) -> int {
         k_chunk_req<<<(int)((n_chunks + 255) / 256), 256, 0, stream>>>(a.reqs, n_pad, ws.b_chunks.as<int>(),
                                                                       (int)n_chunks);
-        return enqueue_wave<true>(SceneView{}, a, pl, stream, ws, A, nullptr, any_retest, overlap && !one_stream,
-                                  FrameInit{}, RTG_MODE_RAYTRACE);
+        FrameInit none;  // (the batch's caller clears the outputs)
+        return enqueue_wave<true>(SceneView{}, a, pl, stream, ws, A, nullptr, any_retest, overlap && !one_stream, none,
+                                  RTG_MODE_RAYTRACE);
     };
     if (use_graph && capture_at > 1 && !(ws.graph != nullptr && ws.graph_key == key)) {
         int slot = -1;
