@@ -101,57 +101,6 @@ int resolve_size(const SceneRes &S, const rtg_params *p, int &W, int &H) {
     return RTG_OK;
 }
 
-void *BlockCache::take(size_t n, size_t &cap) {
-    std::lock_guard<std::mutex> l(m);
-    const auto it = blocks.lower_bound(n);
-    if (it == blocks.end() || it->first > n + n / 4) return nullptr;
-    void *const p = it->second;
-    cap = it->first;
-    total -= it->first;
-    blocks.erase(it);
-    return p;
-}
-bool BlockCache::keep(void *p, size_t cap) {
-    std::lock_guard<std::mutex> l(m);
-    if (total + cap > kMost) return false;
-    blocks.emplace(cap, p);
-    total += cap;
-    return true;
-}
-void BlockCache::clear() {
-    std::lock_guard<std::mutex> l(m);
-    for (const auto &b : blocks) (void)hipFree(b.second);
-    blocks.clear();
-    total = 0;
-}
-
-int DevBuf::alloc(size_t n) {
-    if (p != nullptr && reuse) (void)hipDeviceSynchronize();  // renders may still read the old block
-    release();
-    if (n == 0) n = 16;
-    BlockCache *const cache = g_arena ? &g_arena->blocks : nullptr;
-    cap = n;
-    if (reuse && cache) p = cache->take(n, cap);
-    if (p == nullptr && hipMalloc(&p, n) != hipSuccess) {
-        if (cache) cache->clear();  // kept blocks make room
-        if (hipMalloc(&p, n) != hipSuccess) {
-            p = nullptr;
-            return RTG_E_NOMEM;
-        }
-    }
-    bytes = n;
-    return RTG_OK;
-}
-void DevBuf::release() {
-    if (p != nullptr && !(reuse && g_arena && g_arena->blocks.keep(p, cap))) (void)hipFree(p);
-    p = nullptr;
-    bytes = cap = 0;
-}
-int ensure(DevBuf &b, size_t n) {
-    if (b.p != nullptr && b.bytes >= n) return RTG_OK;
-    return b.alloc(n);
-}
-
 int Workspace::grow(DevBuf &b, size_t n) {
     if (b.p != nullptr && b.bytes >= n) return RTG_OK;
     ++epoch;
@@ -211,6 +160,7 @@ void Workspace::release() {
 }
 
 Arena *arena() { return g_arena; }
+BlockCache *block_cache() { return g_arena ? &g_arena->blocks : nullptr; }
 
 static hipEvent_t take_event(Arena &A) {
     if (!A.kevents.empty()) {

@@ -4,7 +4,6 @@
 
 #include <atomic>
 #include <condition_variable>
-#include <map>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -14,6 +13,7 @@
 
 #include "../../include/rtg.h"
 #include "rt_shade.hpp"
+#include "rtg_mem.hpp"
 
 namespace rtg {
 
@@ -24,49 +24,6 @@ int fail(int code, const std::string &msg);
         hipError_t e_ = (call);                                                                \
         if (e_ != hipSuccess) return fail(RTG_E_DEVICE, std::string(#call) + ": " + hipGetErrorString(e_)); \
     } while (0)
-
-// Device allocation owned by a scene or the render arena.
-struct DevBuf {
-    void *p = nullptr;
-    size_t bytes = 0;
-    size_t cap = 0;       // size of the block behind it
-    bool reuse = false;   // its block comes from and returns to the arena's BlockCache
-    int alloc(size_t n);  // RTG_OK / RTG_E_NOMEM
-    void release();
-    void swap(DevBuf &o) {
-        std::swap(p, o.p), std::swap(bytes, o.bytes), std::swap(cap, o.cap), std::swap(reuse, o.reuse);
-    }
-    ~DevBuf() { release(); }
-    DevBuf() = default;
-    DevBuf(const DevBuf &) = delete;
-    DevBuf &operator=(const DevBuf &) = delete;
-    template <class T>
-    T *as() const { return static_cast<T *>(p); }
-};
-
-// A scene's arrays and a build's temporaries: nothing on the GPU may still use
-// the block when it is released (hipFree would wait for the device; a cached
-// block is handed out again at once).
-struct SceneBuf : DevBuf {
-    SceneBuf() { reuse = true; }
-};
-
-// Device blocks of destroyed scenes and finished builds, kept for the next
-// ones: a scene takes some 40 allocations, and each hipFree waits for the
-// device.  At most kMost bytes are kept; rtg_shutdown frees them.
-class BlockCache {
-public:
-    static constexpr size_t kMost = size_t(512) << 20;
-    void *take(size_t n, size_t &cap);  // a kept block of n to 5/4 n bytes, or null
-    bool keep(void *p, size_t cap);     // false: not kept (the caller frees it)
-    void clear();
-    ~BlockCache() { clear(); }
-
-private:
-    std::mutex m;
-    std::multimap<size_t, void *> blocks;
-    size_t total = 0;
-};
 
 struct SceneRes {
     int device = 0;
@@ -248,7 +205,6 @@ double raygen_tables(float fovy, int W, int H, float *tab);
 int persistent_blocks(const Arena &A);
 
 Arena *arena();
-int ensure(DevBuf &b, size_t bytes);
 
 // Build S from d.  With `donor` holding the topology of a tree over the same
 // primitive set (same count and order), that topology moves into S and the

@@ -1,0 +1,62 @@
+// rtg_mem.hip — device buffers and the block cache (rtg_mem.hpp).
+#include "rtg_mem.hpp"
+
+namespace rtg {
+
+void *BlockCache::take(size_t n, size_t &cap) {
+    std::lock_guard<std::mutex> l(m);
+    const auto it = blocks.lower_bound(n);
+    if (it == blocks.end() || it->first > n + n / 4) return nullptr;
+    void *const p = it->second;
+    cap = it->first;
+    total -= it->first;
+    blocks.erase(it);
+    return p;
+}
+bool BlockCache::keep(void *p, size_t cap) {
+    std::lock_guard<std::mutex> l(m);
+    if (total + cap > kMost) return false;
+    blocks.emplace(cap, p);
+    total += cap;
+    return true;
+}
+void BlockCache::clear() {
+    std::lock_guard<std::mutex> l(m);
+    for (const auto &b : blocks) (void)hipFree(b.second);
+    blocks.clear();
+    total = 0;
+}
+
+int DevBuf::alloc(size_t n) {
+    if (p != nullptr && reuse) (void)hipDeviceSynchronize();  // renders may still read the old block
+    release();
+    if (n == 0) n = 16;
+    BlockCache *const cache = block_cache();
+    cap = n;
+    if (reuse && cache) p = cache->take(n, cap);
+    // The runtime stores a failed call's error until it is read, and the check
+    // after a kernel launch reads it: each failure here is answered here.
+    if (p == nullptr && hipMalloc(&p, n) != hipSuccess) {
+        (void)hipGetLastError();
+        if (cache) cache->clear();  // kept blocks make room
+        if (hipMalloc(&p, n) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return RTG_E_NOMEM;
+        }
+    }
+    bytes = n;
+    return RTG_OK;
+}
+void DevBuf::release() {
+    BlockCache *const cache = reuse ? block_cache() : nullptr;
+    if (p != nullptr && !(cache && cache->keep(p, cap))) (void)hipFree(p);
+    p = nullptr;
+    bytes = cap = 0;
+}
+int ensure(DevBuf &b, size_t n) {
+    if (b.p != nullptr && b.bytes >= n) return RTG_OK;
+    return b.alloc(n);
+}
+
+}  // namespace rtg

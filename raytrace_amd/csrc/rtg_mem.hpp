@@ -1,0 +1,63 @@
+// rtg_mem.hpp — device memory of the library: buffers, and the cache of the
+// blocks of destroyed scenes and finished builds.  Host code only, without
+// kernels, so that it also runs against a stand-in for the runtime
+// (tests/cpu_emul/mem.cpp).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <map>
+#include <mutex>
+#include <utility>
+
+#include "../../include/rtg.h"
+
+namespace rtg {
+
+// Device allocation owned by a scene or the render arena.
+struct DevBuf {
+    void *p = nullptr;
+    size_t bytes = 0;
+    size_t cap = 0;       // size of the block behind it
+    bool reuse = false;   // its block comes from and returns to the arena's BlockCache
+    int alloc(size_t n);  // RTG_OK / RTG_E_NOMEM
+    void release();
+    void swap(DevBuf &o) {
+        std::swap(p, o.p), std::swap(bytes, o.bytes), std::swap(cap, o.cap), std::swap(reuse, o.reuse);
+    }
+    ~DevBuf() { release(); }
+    DevBuf() = default;
+    DevBuf(const DevBuf &) = delete;
+    DevBuf &operator=(const DevBuf &) = delete;
+    template <class T>
+    T *as() const { return static_cast<T *>(p); }
+};
+
+// A scene's arrays and a build's temporaries: nothing on the GPU may still use
+// the block when it is released (hipFree would wait for the device; a cached
+// block is handed out again at once).
+struct SceneBuf : DevBuf {
+    SceneBuf() { reuse = true; }
+};
+
+// Device blocks of destroyed scenes and finished builds, kept for the next
+// ones: a scene takes some 40 allocations, and each hipFree waits for the
+// device.  At most kMost bytes are kept; rtg_shutdown frees them.
+class BlockCache {
+public:
+    static constexpr size_t kMost = size_t(512) << 20;
+    void *take(size_t n, size_t &cap);  // a kept block of n to 5/4 n bytes, or null
+    bool keep(void *p, size_t cap);     // false: not kept (the caller frees it)
+    void clear();
+    ~BlockCache() { clear(); }
+
+private:
+    std::mutex m;
+    std::multimap<size_t, void *> blocks;
+    size_t total = 0;
+};
+
+// The arena's cache; null before rtg_init and after rtg_shutdown.
+BlockCache *block_cache();
+int ensure(DevBuf &b, size_t bytes);
+
+}  // namespace rtg

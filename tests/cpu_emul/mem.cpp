@@ -1,0 +1,81 @@
+// Device buffers and the block cache (rtg_mem.hip) on a stand-in for the HIP
+// runtime: host blocks of a bounded "device", with the runtime's rules that
+// the library relies on (a failed call's error is stored until it is read).
+#include <cstdlib>
+#include <map>
+
+#include "../../raytrace_amd/csrc/rtg_mem.hip"
+
+namespace {
+size_t g_room = 0, g_used = 0;  // bytes of the device, and in use
+std::map<void *, size_t> g_live;
+hipError_t g_stored = hipSuccess;
+int g_mallocs = 0, g_frees = 0;
+rtg::BlockCache *g_cache = nullptr;
+
+hipError_t answer(hipError_t e) {
+    if (e != hipSuccess) g_stored = e;
+    return e;
+}
+}  // namespace
+
+extern "C" {
+
+hipError_t hipMalloc(void **p, size_t n) {
+    if (g_used + n > g_room) return answer(hipErrorOutOfMemory);
+    *p = malloc(16);
+    g_live[*p] = n;
+    g_used += n;
+    ++g_mallocs;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p) {
+    const auto it = g_live.find(p);
+    if (it == g_live.end()) return answer(hipErrorInvalidValue);
+    g_used -= it->second;
+    g_live.erase(it);
+    free(p);
+    ++g_frees;
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+    const hipError_t e = g_stored;
+    g_stored = hipSuccess;
+    return e;
+}
+
+}  // extern "C"
+
+rtg::BlockCache *rtg::block_cache() { return g_cache; }
+
+namespace {
+// A fresh device of `room` bytes and an empty cache for the life of one case.
+struct Case {
+    rtg::BlockCache cache;
+    explicit Case(size_t room) {
+        g_room = room, g_used = 0, g_stored = hipSuccess, g_mallocs = g_frees = 0;
+        g_cache = &cache;
+    }
+    ~Case() {
+        cache.clear();
+        g_cache = nullptr;
+    }
+};
+constexpr size_t kMB = size_t(1) << 20;
+}  // namespace
+
+extern "C" {
+
+// A kept block makes room for an allocation that would fail without it: the
+// allocation succeeds and leaves no stored error behind (bit 0: its status,
+// bit 1: the stored error); one that fails all the same leaves none either.
+int mem_no_stored_error(int fits) {
+    Case c(100 * kMB);
+    { rtg::SceneBuf a; (void)a.alloc(60 * kMB); }  // into the cache
+    rtg::DevBuf b;
+    const int st = b.alloc((fits ? 90 : 110) * kMB);
+    return (st == (fits ? RTG_OK : RTG_E_NOMEM) ? 0 : 1) | (hipGetLastError() == hipSuccess ? 0 : 2);
+}
+
+}  // extern "C"
