@@ -265,7 +265,7 @@ int rtg_init(int device) {
     int st = noalloc_setup(device);
     if (st != RTG_OK) return st;
     std::unique_ptr<Arena> A(new Arena());
-    A->device = device;
+    A->device = A->blocks.device = device;
     hipDeviceProp_t prop;
     RTG_HIP(hipGetDeviceProperties(&prop, device));
     A->cus = prop.multiProcessorCount;
@@ -327,7 +327,10 @@ int rtg_scene_create(const rtg_scene_desc *desc, rtg_scene_t *out) {
         std::lock_guard<std::mutex> l(A.lock);
         st = scene_build(s->res, *desc, A.stream);
     }
-    if (st != RTG_OK) return st;
+    if (st != RTG_OK) {
+        s->res.not_idle();
+        return st;
+    }
     s->res.geom_hash = geometry_hash(*desc, A.pool);
     s->res.topo_hash = topology_hash(*desc);
     *out = s.release();
@@ -356,8 +359,12 @@ static int scene_update(rtg_scene_t scene, const rtg_scene_desc *desc, bool allo
     SceneRes fresh;
     fresh.device = A.device;
     st = scene_build(fresh, *desc, A.stream, refit ? &R : nullptr);
-    if (st != RTG_OK) return st;
-    RTG_HIP(hipDeviceSynchronize());  // frames on any stream may read the old arrays, released below
+    if (st != RTG_OK) {
+        fresh.not_idle();
+        return st;
+    }
+    // frames on any stream may read the old arrays, released below
+    const bool idle = device_idle();
     auto take = [](DevBuf &a, DevBuf &b) { a.swap(b); };
     take(R.nodes, fresh.nodes), take(R.prims, fresh.prims), take(R.objs, fresh.objs), take(R.brute, fresh.brute);
     take(R.parts, fresh.parts), take(R.tri_nrm, fresh.tri_nrm), take(R.tri_uv, fresh.tri_uv);
@@ -367,6 +374,7 @@ static int scene_update(rtg_scene_t scene, const rtg_scene_desc *desc, bool allo
     take(R.t_keys, fresh.t_keys), take(R.t_left, fresh.t_left), take(R.t_right, fresh.t_right);
     take(R.t_first, fresh.t_first), take(R.t_last, fresh.t_last), take(R.t_pint, fresh.t_pint);
     take(R.t_pleaf, fresh.t_pleaf), take(R.t_newidx, fresh.t_newidx);
+    if (!idle) fresh.not_idle();
     R.topo_n = fresh.topo_n, R.topo_emit = fresh.topo_emit;
     R.topo_hash = th;
     R.view = fresh.view;
@@ -405,7 +413,8 @@ int rtg_scene_destroy(rtg_scene_t scene) {
     if (scene == nullptr) return RTG_OK;
     if (arena()) {
         std::lock_guard<std::mutex> l(arena()->lock);
-        (void)hipDeviceSynchronize();  // frames on any stream may read its arrays
+        // frames on any stream may read its arrays
+        if (!device_idle()) scene->res.not_idle();
     }
     delete scene;
     return RTG_OK;

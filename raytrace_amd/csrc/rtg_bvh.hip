@@ -304,18 +304,11 @@ int upload(DevBuf &b, const std::vector<T> &v, hipStream_t s) {
     return RTG_OK;
 }
 
-// Waits for the stream before the temporaries declared ahead of it are
-// released, on every path.
-struct SyncOnExit {
-    hipStream_t stream;
-    ~SyncOnExit() { (void)hipStreamSynchronize(stream); }
-};
-
 // The 4-wide tree of the n2 binary nodes in nodes2 (root 0) into S.nodes;
 // returns its node count in *n4.
 int widen_tree(const DevBuf &nodes2, int n2, SceneRes &S, hipStream_t stream, int *n4) {
     SceneBuf parent2, flags, idx4, scan_tmp;
-    const SyncOnExit idle{stream};
+    const SyncOnExit<4> idle{stream, {&parent2, &flags, &idx4, &scan_tmp}};
     if (ensure(parent2, n2 * sizeof(int)) || ensure(flags, n2 * sizeof(int)) || ensure(idx4, n2 * sizeof(int)))
         return fail(RTG_E_NOMEM, "device allocation failed (4-wide nodes)");
     k_fill_i32<<<nblk(n2), kBlock, 0, stream>>>(parent2.as<int>(), n2, -1);
@@ -408,7 +401,8 @@ int scene_build(SceneRes &S, const rtg_scene_desc &d, hipStream_t stream, SceneR
         donor->topo_n = 0, donor->topo_emit = 0;
     }
     SceneBuf raw, mid, sph, prims_u, boxes, keys, flags, ibox, sbox, bbox, partial, cb, sort_tmp, scan_tmp, nodes2;
-    const SyncOnExit idle{stream};
+    const SyncOnExit<15> idle{stream, {&raw, &mid, &sph, &prims_u, &boxes, &keys, &flags, &ibox, &sbox, &bbox, &partial,
+                                       &cb, &sort_tmp, &scan_tmp, &nodes2}};
     DevBuf &keys2 = S.t_keys, &left = S.t_left, &right = S.t_right, &first = S.t_first, &last = S.t_last,
            &pint = S.t_pint, &pleaf = S.t_pleaf, &newidx = S.t_newidx;
     if ((st = upload(mid, part_mid, stream)) || (st = upload(sph, spheres, stream))) return st;

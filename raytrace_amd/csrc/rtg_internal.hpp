@@ -46,6 +46,13 @@ struct SceneRes {
     SceneBuf t_keys, t_left, t_right, t_first, t_last, t_pint, t_pleaf, t_newidx;
     int topo_n = 0, topo_emit = 0;
     uint64_t topo_hash = 0;
+    // The GPU may still use the arrays: releasing them waits (hipFree).
+    void not_idle() {
+        for (SceneBuf *b : {&nodes, &prims, &objs, &brute, &parts, &tri_nrm, &tri_uv, &tri_pos, &tri_part, &tri_mtl,
+                            &tri_bins, &mtls, &lights, &texs, &texels, &t_keys, &t_left, &t_right, &t_first, &t_last,
+                            &t_pint, &t_pleaf, &t_newidx})
+            b->idle = false;
+    }
 };
 
 // Device memory of one in-flight render (or batch): traversal spill stacks,

@@ -28,7 +28,7 @@ void BlockCache::clear() {
 }
 
 int DevBuf::alloc(size_t n) {
-    if (p != nullptr && reuse) (void)hipDeviceSynchronize();  // renders may still read the old block
+    if (p != nullptr && reuse && !device_idle()) idle = false;  // renders may still read the old block
     release();
     if (n == 0) n = 16;
     BlockCache *const cache = block_cache();
@@ -46,14 +46,26 @@ int DevBuf::alloc(size_t n) {
         }
     }
     bytes = n;
+    idle = true;
     return RTG_OK;
 }
 void DevBuf::release() {
-    BlockCache *const cache = reuse ? block_cache() : nullptr;
+    BlockCache *const cache = reuse && idle ? block_cache() : nullptr;
     if (p != nullptr && !(cache && cache->keep(p, cap))) (void)hipFree(p);
     p = nullptr;
     bytes = cap = 0;
 }
+bool device_idle() {
+    const BlockCache *const cache = block_cache();
+    int cur = -1;
+    if (cache == nullptr || hipGetDevice(&cur) != hipSuccess) return false;
+    const bool other = cur != cache->device;
+    const bool ok = (!other || hipSetDevice(cache->device) == hipSuccess) && hipDeviceSynchronize() == hipSuccess;
+    if (other) (void)hipSetDevice(cur);
+    if (!ok) (void)hipGetLastError();  // answered here, not by the next launch's check
+    return ok;
+}
+
 int ensure(DevBuf &b, size_t n) {
     if (b.p != nullptr && b.bytes >= n) return RTG_OK;
     return b.alloc(n);

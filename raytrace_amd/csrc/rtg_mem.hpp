@@ -18,11 +18,13 @@ struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
     size_t cap = 0;       // size of the block behind it
-    bool reuse = false;   // its block comes from and returns to the arena's BlockCache
+    bool reuse = false;   // its block comes from the arena's BlockCache
+    bool idle = true;     // and returns to it: false once a wait for its users failed
     int alloc(size_t n);  // RTG_OK / RTG_E_NOMEM
     void release();
     void swap(DevBuf &o) {
         std::swap(p, o.p), std::swap(bytes, o.bytes), std::swap(cap, o.cap), std::swap(reuse, o.reuse);
+        std::swap(idle, o.idle);
     }
     ~DevBuf() { release(); }
     DevBuf() = default;
@@ -34,7 +36,8 @@ struct DevBuf {
 
 // A scene's arrays and a build's temporaries: nothing on the GPU may still use
 // the block when it is released (hipFree would wait for the device; a cached
-// block is handed out again at once).
+// block is handed out again at once).  Where the wait before that failed,
+// `idle` is cleared, and the block goes to hipFree.
 struct SceneBuf : DevBuf {
     SceneBuf() { reuse = true; }
 };
@@ -44,6 +47,7 @@ struct SceneBuf : DevBuf {
 // device.  At most kMost bytes are kept; rtg_shutdown frees them.
 class BlockCache {
 public:
+    int device = -1;  // of its blocks
     static constexpr size_t kMost = size_t(512) << 20;
     void *take(size_t n, size_t &cap);  // a kept block of n to 5/4 n bytes, or null
     bool keep(void *p, size_t cap);     // false: not kept (the caller frees it)
@@ -58,6 +62,23 @@ private:
 
 // The arena's cache; null before rtg_init and after rtg_shutdown.
 BlockCache *block_cache();
+// Wait for everything enqueued on the arena's device, whichever device is the
+// calling thread's.  false: the wait failed (a stream captures, a device error).
+bool device_idle();
+
+// Waits for the stream before the buffers of a build are released, on every
+// path; declared after them.
+template <size_t N>
+struct SyncOnExit {
+    hipStream_t stream;
+    SceneBuf *bufs[N];
+    ~SyncOnExit() {
+        if (hipStreamSynchronize(stream) == hipSuccess) return;
+        (void)hipGetLastError();
+        for (SceneBuf *b : bufs) b->idle = false;
+    }
+};
+
 int ensure(DevBuf &b, size_t bytes);
 
 }  // namespace rtg

@@ -11,6 +11,8 @@ size_t g_room = 0, g_used = 0;  // bytes of the device, and in use
 std::map<void *, size_t> g_live;
 hipError_t g_stored = hipSuccess;
 int g_mallocs = 0, g_frees = 0;
+int g_device = 0, g_waited = -1;  // the thread's device, and the one last waited for
+bool g_capturing = false;         // waits are refused, as while a stream captures
 rtg::BlockCache *g_cache = nullptr;
 
 hipError_t answer(hipError_t e) {
@@ -38,7 +40,22 @@ hipError_t hipFree(void *p) {
     ++g_frees;
     return hipSuccess;
 }
-hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipGetDevice(int *d) {
+    *d = g_device;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int d) {
+    g_device = d;
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize(void) {
+    if (g_capturing) return answer(hipErrorStreamCaptureUnsupported);
+    g_waited = g_device;
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) {
+    return g_capturing ? answer(hipErrorStreamCaptureUnsupported) : hipSuccess;
+}
 hipError_t hipGetLastError(void) {
     const hipError_t e = g_stored;
     g_stored = hipSuccess;
@@ -55,6 +72,7 @@ struct Case {
     rtg::BlockCache cache;
     explicit Case(size_t room) {
         g_room = room, g_used = 0, g_stored = hipSuccess, g_mallocs = g_frees = 0;
+        g_device = cache.device = 0, g_waited = -1, g_capturing = false;
         g_cache = &cache;
     }
     ~Case() {
@@ -76,6 +94,38 @@ int mem_no_stored_error(int fits) {
     rtg::DevBuf b;
     const int st = b.alloc((fits ? 90 : 110) * kMB);
     return (st == (fits ? RTG_OK : RTG_E_NOMEM) ? 0 : 1) | (hipGetLastError() == hipSuccess ? 0 : 2);
+}
+
+// A block that a refused wait could not show to be unused goes to hipFree, and
+// the refusal leaves no stored error: how = 0 a buffer allocated anew, 1 a
+// build's temporary, 2 (control) the same buffer after a wait that succeeded.
+int mem_refused_wait(int how) {
+    Case c(100 * kMB);
+    {
+        rtg::SceneBuf a;
+        (void)a.alloc(kMB);
+        g_capturing = how != 2;
+        if (how == 1) {
+            const rtg::SyncOnExit<1> idle{nullptr, {&a}};
+        } else {
+            (void)a.alloc(2 * kMB);
+        }
+    }
+    g_capturing = false;
+    // how 0: the first block freed, the second kept; 1: freed; 2: both kept
+    const bool frees = g_frees == (how == 2 ? 0 : 1);
+    return (frees ? 0 : 1) | (hipGetLastError() == hipSuccess ? 0 : 2);
+}
+
+// The wait is for the cache's device, also on a thread whose device is another.
+int mem_waits_for_its_device(int thread_device) {
+    Case c(100 * kMB);
+    c.cache.device = 3;
+    rtg::SceneBuf a;
+    (void)a.alloc(kMB);
+    g_device = thread_device;
+    (void)a.alloc(2 * kMB);
+    return (g_waited == 3 ? 0 : 1) | (g_device == thread_device ? 0 : 2);
 }
 
 }  // extern "C"

@@ -18,3 +18,13 @@ def mem():
 @pytest.mark.parametrize("fits", [1, 0], ids=["after making room", "no room at all"])
 def test_allocation_leaves_no_stored_error(mem, fits):
     assert mem.mem_no_stored_error(fits) == 0
+
+
+@pytest.mark.parametrize("how", [0, 1, 2], ids=["allocated anew", "temporary of a build", "wait succeeds"])
+def test_blocks_that_may_be_in_use_are_not_kept(mem, how):
+    assert mem.mem_refused_wait(how) == 0
+
+
+@pytest.mark.parametrize("thread_device", [0, 3])
+def test_waits_for_the_device_of_its_blocks(mem, thread_device):
+    assert mem.mem_waits_for_its_device(thread_device) == 0
