@@ -197,7 +197,10 @@ typedef struct rtg_job_s *rtg_job_t;
 /* Replaces RayTracer::RayTracer (RayTracer.cpp:600-606): select the device
  * and create the library's stream.  Idempotent per device. */
 int rtg_init(int device);
-/* Release every library resource (scenes must be destroyed first). */
+/* Release every library resource (scenes must be destroyed first): streams,
+ * workspaces, the device memory kept from destroyed scenes (see
+ * rtg_scene_destroy) and the host threads the library keeps for copies of
+ * results and hashes of scenes (at most seven, started when first needed). */
 int rtg_shutdown(void);
 /* Thread-local message of the last failing call (never NULL). */
 const char *rtg_last_error(void);
@@ -222,8 +225,14 @@ int rtg_scene_update(rtg_scene_t scene, const rtg_scene_desc *desc);
 /* rtg_scene_update that always rebuilds the BVH (a fresh tree after many
  * refits have moved objects far from where the tree was built). */
 int rtg_scene_rebuild(rtg_scene_t scene, const rtg_scene_desc *desc);
+/* Waits for the device.  Up to 512 MB of device memory of destroyed and replaced
+ * scenes and of finished builds stay with the library for the next ones; past
+ * that, the memory kept longest is freed first.  rtg_shutdown frees all of it,
+ * and so does an allocation of the library that would fail otherwise. */
 int rtg_scene_destroy(rtg_scene_t scene);
-/* Device bytes held by the scene (geometry + BVH + the topology kept for refits). */
+/* Device bytes held by the scene (geometry + BVH + the topology kept for
+ * refits), as asked for: a kept block that serves an array may be up to a
+ * quarter larger. */
 int rtg_scene_bytes(rtg_scene_t scene, uint64_t *bytes);
 /* Device time (ms) of the scene's last BVH build or refit. */
 int rtg_scene_build_ms(rtg_scene_t scene, double *ms);

@@ -3,27 +3,43 @@
 
 namespace rtg {
 
+void BlockCache::drop(std::multimap<size_t, Blocks::iterator>::iterator it) {
+    total -= charge(it->first);
+    blocks.erase(it->second);
+    by_size.erase(it);
+}
 void *BlockCache::take(size_t n, size_t &cap) {
     std::lock_guard<std::mutex> l(m);
-    const auto it = blocks.lower_bound(n);
-    if (it == blocks.end() || it->first > n + n / 4) return nullptr;
-    void *const p = it->second;
+    const auto it = by_size.lower_bound(n);
+    if (it == by_size.end() || it->first > n + n / 4) return nullptr;
+    void *const p = it->second->p;
     cap = it->first;
-    total -= it->first;
-    blocks.erase(it);
+    drop(it);
     return p;
 }
-bool BlockCache::keep(void *p, size_t cap) {
+bool BlockCache::keep(void *p, size_t cap) try {
+    if (charge(cap) > kMost) return false;
     std::lock_guard<std::mutex> l(m);
-    if (total + cap > kMost) return false;
-    blocks.emplace(cap, p);
-    total += cap;
+    Blocks one{Block{p, cap}};
+    const auto at = by_size.emplace(cap, one.begin());  // before anything is displaced: it may throw
+    while (total + charge(cap) > kMost) {
+        const Blocks::iterator old = blocks.begin();
+        auto it = by_size.lower_bound(old->cap);
+        while (it->second != old) ++it;  // (blocks of one size: the oldest is the first)
+        (void)hipFree(old->p);
+        drop(it);
+    }
+    blocks.splice(blocks.end(), one);
+    total += charge(at->first);
     return true;
+} catch (...) {  // no memory for the entry
+    return false;
 }
 void BlockCache::clear() {
     std::lock_guard<std::mutex> l(m);
-    for (const auto &b : blocks) (void)hipFree(b.second);
+    for (const Block &b : blocks) (void)hipFree(b.p);
     blocks.clear();
+    by_size.clear();
     total = 0;
 }
 

@@ -5,6 +5,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <list>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -44,19 +45,30 @@ struct SceneBuf : DevBuf {
 
 // Device blocks of destroyed scenes and finished builds, kept for the next
 // ones: a scene takes some 40 allocations, and each hipFree waits for the
-// device.  At most kMost bytes are kept; rtg_shutdown frees them.
+// device.  At most kMost bytes are kept, each block counted in whole pages, as
+// the runtime hands them out; a block that does not fit displaces the ones kept
+// longest, so that sizes nobody asks for any more make way.  rtg_shutdown frees
+// them, and so does an allocation of the library that fails.
 class BlockCache {
 public:
     int device = -1;  // of its blocks
-    static constexpr size_t kMost = size_t(512) << 20;
+    static constexpr size_t kMost = size_t(512) << 20, kPage = 4096;
     void *take(size_t n, size_t &cap);  // a kept block of n to 5/4 n bytes, or null
     bool keep(void *p, size_t cap);     // false: not kept (the caller frees it)
     void clear();
     ~BlockCache() { clear(); }
 
 private:
+    struct Block {
+        void *p;
+        size_t cap;
+    };
+    using Blocks = std::list<Block>;
+    static size_t charge(size_t cap) { return (cap + kPage - 1) / kPage * kPage; }
+    void drop(std::multimap<size_t, Blocks::iterator>::iterator it);  // forget it
     std::mutex m;
-    std::multimap<size_t, void *> blocks;
+    Blocks blocks;  // the one kept longest first
+    std::multimap<size_t, Blocks::iterator> by_size;
     size_t total = 0;
 };
 

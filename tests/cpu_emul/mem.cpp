@@ -3,6 +3,7 @@
 // the library relies on (a failed call's error is stored until it is read).
 #include <cstdlib>
 #include <map>
+#include <memory>
 
 #include "../../raytrace_amd/csrc/rtg_mem.hip"
 
@@ -126,6 +127,33 @@ int mem_waits_for_its_device(int thread_device) {
     g_device = thread_device;
     (void)a.alloc(2 * kMB);
     return (g_waited == 3 ? 0 : 1) | (g_device == thread_device ? 0 : 2);
+}
+
+// A program that moves on to other sizes: 512 MB of kept blocks that nobody
+// takes any more, then `n` rounds of a buffer of `bytes` that comes and goes.
+// Returns the rounds that had to allocate; -1 when more than 512 MB stay kept.
+int mem_moves_on(int n, unsigned long long bytes) {
+    Case c(~size_t(0) / 2);
+    {
+        rtg::SceneBuf old[128];
+        for (rtg::SceneBuf &b : old) (void)b.alloc(4 * kMB);
+    }
+    const int before = g_mallocs;
+    for (int k = 0; k < n; ++k) {
+        rtg::SceneBuf b;
+        (void)b.alloc((size_t)bytes);
+    }
+    return g_used > 512 * kMB ? -1 : g_mallocs - before;
+}
+
+// Blocks kept after `n` buffers of 16 bytes each are released.
+int mem_small_blocks_kept(int n) {
+    Case c(~size_t(0) / 2);
+    {
+        std::unique_ptr<rtg::SceneBuf[]> b(new rtg::SceneBuf[n]);
+        for (int k = 0; k < n; ++k) (void)b[k].alloc(16);
+    }
+    return (int)g_live.size();
 }
 
 }  // extern "C"

@@ -28,3 +28,16 @@ def test_blocks_that_may_be_in_use_are_not_kept(mem, how):
 @pytest.mark.parametrize("thread_device", [0, 3])
 def test_waits_for_the_device_of_its_blocks(mem, thread_device):
     assert mem.mem_waits_for_its_device(thread_device) == 0
+
+
+@pytest.mark.parametrize("megabytes,allocations", [(1, 1), (6, 1), (512, 1), (513, 5)])
+def test_full_cache_makes_way_for_the_sizes_in_use(mem, megabytes, allocations):
+    """Five rounds of one size after 512 MB of another: allocated once and kept
+    (513 MB fit no cache: allocated each time)."""
+    f = mem.mem_moves_on
+    f.argtypes = [C.c_int, C.c_ulonglong]
+    assert f(5, megabytes << 20) == allocations
+
+
+def test_small_blocks_count_as_pages(mem):
+    assert mem.mem_small_blocks_kept(140000) == (512 << 20) // 4096
