@@ -997,6 +997,16 @@ constexpr int kNoSyncMaxSamples = 1 << 22;
 // Level-0 samples per pass of a frame whose rays branch (see launch_wavefront).
 constexpr int kPassSamples = 1 << 21;
 
+// Longest batch (level-0 samples) whose levels run as k_step: the levels of
+// longer ones fill the GPU by themselves, and their shadow rays gain more from
+// k_occlude's six waves per SIMD than from filling another kernel's tail (us a
+// batch, k_step / side streams: 16 frames of 1080p of one scene, 33 M samples,
+// 24034 / 22511; 4 at 4 samples per pixel, 33 M, 20254 / 19058; the same over
+// three scenes 26227 / 25216; 80 of 512x512 over three scenes, 21 M, 29651 /
+// 29510; 8 of 1080p, 17 M, one scene 12554 / 12250, three 14967 / 15218; 6 over
+// three scenes, 12 M, 11259 / 11770; 4 of one scene, 8 M, 6762 / 6748).
+constexpr int kStepMaxSamples = 1 << 24;
+
 // Levels known to hold this many rays are walked lane by lane (Walk): two and
 // more for each lane the GPU has, so that a tail is short beside the rest (us a
 // frame at limits of 2^18, 2^20, 2^22: 1080p 1686, 1735, 1882 of 1756, 1793,
@@ -1136,8 +1146,9 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     // on queues where they waited for one another.  Single frames keep the
     // side streams (with k_step 64x64 215 -> 227 us, 320x180 3709 -> 3890 us
     // for three edits, 1080p 1993 -> 2397 us), and so do the FP64 re-test,
-    // which has a kernel of its own, and levels sized by read-backs.
-    const bool fused = B && pl.no_sync && !retest && shadows;
+    // which has a kernel of its own, levels sized by read-backs and batches
+    // past kStepMaxSamples.
+    const bool fused = B && pl.no_sync && !retest && shadows && pl.n_samples <= kStepMaxSamples;
     const bool chain = pl.fanout <= 1 && !view;
     // The shadow rays of level k (k_occlude) depend only on
     // k_shade(k), and level k + 1 does not depend on them: with `overlap`
