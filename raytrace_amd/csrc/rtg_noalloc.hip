@@ -6,8 +6,8 @@
 // It renders with the megakernel, whose scratch is bounded by the persistent
 // grid rather than by the frame: the ray-generation tables (W + H floats) and
 // the traversal stacks' spill area (80 ints per thread of the grid).  The
-// wavefront engine's queues grow with the frame (about 1 KB per sample at
-// depth 4, 2.2 GB for a 1080p frame), too much for a fixed array.
+// wavefront engine's queues grow with the frame (0.9 KB per sample at
+// depth 4, with headroom 2.3 GB for a 1080p frame), too much for a fixed array.
 //
 // That scratch is `scratch`, a file-scope device array of kScratchBytes: each
 // GPU holds its own copy for the life of the process.  Every call on a GPU

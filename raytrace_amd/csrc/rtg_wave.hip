@@ -456,7 +456,7 @@ __global__ __launch_bounds__(kBlockThreads, 4) void k_shade(SceneView S0, WaveAr
                                                          const unsigned *n_ptr, const WHit *hits, const int4 *cs,
                                                          WNode *nodes,
                                                          unsigned *masks, WRay *next, LevelCtr *ctr,
-                                                         unsigned *shadow, float4 *slots) {
+                                                         unsigned *shadow) {
     const int n = k == 0 ? A.n_samples : (int)*n_ptr;
     if (surplus_block(n)) return;
     if (wave_cancelled(A)) return;
@@ -1055,12 +1055,17 @@ struct WavePlan {
     int fanout;     // most child rays per hit
     int n_on;       // most switched-on lights of a scene
     int n_reqs;     // grid y of k_resolve
+    bool shade;     // hits become nodes (k_shade); a view without shadow rays has hits only
     size_t bound[Workspace::kLevels];
     bool no_sync;
+    // two child slots a ray, for k_combine (k_chain passes colours on in registers)
+    bool slots() const { return fanout >= 2; }
 };
 
-static size_t per_ray_bytes(int n_on) {
-    return sizeof(WRay) + sizeof(WHit) + sizeof(int4) + sizeof(WNode) + sizeof(unsigned) + 2 * sizeof(float4) +
+static size_t per_ray_bytes(int fanout, int n_on, bool shade) {
+    const size_t hit = sizeof(WHit) + sizeof(int4);
+    if (!shade) return hit;
+    return hit + sizeof(WRay) + sizeof(WNode) + sizeof(unsigned) + (fanout >= 2 ? 2 * sizeof(float4) : 0) +
            (size_t)n_on * sizeof(unsigned);
 }
 
@@ -1069,17 +1074,19 @@ size_t batch_queue_bytes(size_t samples, int max_level, int fanout, int n_on, si
     const size_t cap = level_ray_cap(n_on);
     for (int k = 0; k <= max_level && b > 0; ++k) {
         if (b > cap) return 0;
-        need += b * per_ray_bytes(n_on);
+        need += b * per_ray_bytes(fanout, n_on, true);
         if (need > budget) return 0;
         b *= (size_t)fanout;
     }
     return need;
 }
 
-static WavePlan make_plan(int n_samples, int max_level, int fanout, int n_on, int n_reqs, size_t budget) {
+static WavePlan make_plan(int n_samples, int max_level, int fanout, int n_on, int n_reqs, size_t budget,
+                          bool shade = true) {
     WavePlan pl{};
     pl.n_samples = n_samples, pl.max_level = max_level, pl.fanout = fanout, pl.n_on = n_on, pl.n_reqs = n_reqs;
-    const size_t per_ray = per_ray_bytes(n_on), cap = level_ray_cap(n_on);
+    pl.shade = shade;
+    const size_t per_ray = per_ray_bytes(fanout, n_on, shade), cap = level_ray_cap(n_on);
     size_t need = 0;
     pl.no_sync = true;
     for (int k = 0; k <= max_level; ++k) {
@@ -1096,9 +1103,11 @@ static WavePlan make_plan(int n_samples, int max_level, int fanout, int n_on, in
 static int reserve_level(Workspace &ws, const WavePlan &pl, int k, size_t n_k) {
     const size_t cap_next = k < pl.max_level ? (size_t)std::max(1, pl.fanout) * n_k : 1;
     const int kn = k + 1 < Workspace::kLevels ? k + 1 : k;
-    if (ws.grow(ws.w_hits[k], n_k * sizeof(WHit)) || ws.grow(ws.w_cs[k], n_k * sizeof(int4)) ||
-        ws.grow(ws.w_nodes[k], n_k * sizeof(WNode)) ||
-        ws.grow(ws.w_masks[k], n_k * sizeof(unsigned)) || ws.grow(ws.w_slots[k], 2 * n_k * sizeof(float4)) ||
+    if (ws.grow(ws.w_hits[k], n_k * sizeof(WHit)) || ws.grow(ws.w_cs[k], n_k * sizeof(int4)))
+        return fail(RTG_E_NOMEM, "wavefront queues");
+    if (!pl.shade) return RTG_OK;
+    if (ws.grow(ws.w_nodes[k], n_k * sizeof(WNode)) || ws.grow(ws.w_masks[k], n_k * sizeof(unsigned)) ||
+        (pl.slots() && ws.grow(ws.w_slots[k], 2 * n_k * sizeof(float4))) ||
         ws.grow(ws.w_shadow[k], std::max<size_t>(1, n_k * pl.n_on) * sizeof(unsigned)) ||
         ws.grow(ws.w_rays[kn], cap_next * sizeof(WRay)))
         return fail(RTG_E_NOMEM, "wavefront queues");
@@ -1132,7 +1141,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
                         FrameInit &init, int mode) {
     const int *cancel_host = cancel ? cancel->host : nullptr;
     const bool view = primary_only(mode);  // (one level) k_view shades the hits
-    const bool shadows = pl.n_on > 0 && (!view || mode == RTG_MODE_SHADOWTEST);
+    const bool shadows = pl.n_on > 0;
     const int cus = A.cus > 0 ? A.cus : 256;
     const Grids<B> g(cus, A.tune.grid_pct);
     if (!pl.no_sync) {
@@ -1149,7 +1158,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     // which has a kernel of its own, levels sized by read-backs and batches
     // past kStepMaxSamples.
     const bool fused = B && pl.no_sync && !retest && shadows && pl.n_samples <= kStepMaxSamples;
-    const bool chain = pl.fanout <= 1 && !view;
+    const bool chain = !pl.slots() && !view;
     // The shadow rays of level k (k_occlude) depend only on
     // k_shade(k), and level k + 1 does not depend on them: with `overlap`
     // they run on the workspace's side stream, concurrently with the next
@@ -1270,12 +1279,11 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             k_extend<B, WALK_WAVE><<<grid(ov && k > 0 ? g.extend : g.extend_alone, lanes_of(n_k)), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ctr[k].sched[0]);
         ktime_end(A, stream, kt, n_ptr);
-        if (!view || shadows) {
+        if (pl.shade) {
             kt = ktime_begin(A, stream, KT_SHADE, n_k);
             k_shade<B><<<grid(g.shade, n_k), kBlockThreads, 0, stream>>>(
                 S0, args, k, rays, n_ptr, ws.w_hits[k].as<WHit>(), ws.w_cs[k].as<int4>(), ws.w_nodes[k].as<WNode>(),
-                ws.w_masks[k].as<unsigned>(), next, ctr + k, ws.w_shadow[k].as<unsigned>(),
-                ws.w_slots[k].as<float4>());
+                ws.w_masks[k].as<unsigned>(), next, ctr + k, ws.w_shadow[k].as<unsigned>());
             ktime_end(A, stream, kt, n_ptr);
         }
         // The last level has no next level to overlap: its shadow rays stay
@@ -1425,7 +1433,7 @@ int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const
     // run in passes of whole block rows, at most kPassSamples level-0
     // samples each, so that the queues of all levels stay a few GB.
     const int rows = (H + th - 1) / th, per_row = r.bw * 64 * r.spp;
-    const int n_on = __builtin_popcount(S.lights_on);
+    const int n_on = view && p.mode != RTG_MODE_SHADOWTEST ? 0 : __builtin_popcount(S.lights_on);
     int rows_per_pass = frame_rows_per_pass(rows, (size_t)per_row, fanout, n_on, kPassSamples);
     if (view) rows_per_pass = std::min(rows_per_pass, std::max(1, kNoSyncMaxSamples / per_row));
     if (cancel && cancel->pass_samples > 0)
@@ -1434,7 +1442,7 @@ int launch_wavefront(const SceneRes &S, const rtg_params &p, int W, int H, const
         r.row0 = row0;
         r.n_samples = std::min(rows_per_pass, rows - row0) * per_row;
         a.n_samples = r.n_samples;
-        WavePlan pl = make_plan(r.n_samples, r.max_level, fanout, n_on, 1, A.no_sync_budget);
+        WavePlan pl = make_plan(r.n_samples, r.max_level, fanout, n_on, 1, A.no_sync_budget, !view || n_on > 0);
         // A very large frame keeps the GPU busy at every level; there the
         // host round trip per level costs little, and sizing each level from
         // the previous level's count saves the worst-case queue memory.
