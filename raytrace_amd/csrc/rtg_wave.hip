@@ -1007,11 +1007,18 @@ constexpr int kPassSamples = 1 << 21;
 // three scenes, 12 M, 11259 / 11770; 4 of one scene, 8 M, 6762 / 6748).
 constexpr int kStepMaxSamples = 1 << 24;
 
-// Levels known to hold this many rays are walked lane by lane (Walk): two and
-// more for each lane the GPU has, so that a tail is short beside the rest (us a
-// frame at limits of 2^18, 2^20, 2^22: 1080p 1686, 1735, 1882 of 1756, 1793,
-// 1922; 801x451 at 4 samples 1740, 1733, 1670 of 1840, 1848, 1834).
-constexpr size_t kFullRays = size_t(1) << 20;
+// Levels known to hold this many rays per CU (2^20 on 256 CUs) are walked lane
+// by lane (Walk); known are level 0 and the levels counted by read-backs.  Device
+// time of a frame in us at limits of 2^18, 2^20, 2^21, 2^22 rays and of none.
+// Read-backs, for which the rule is there: refraction frame 960x540 at 4 samples
+// 96161, 96376, 96935, 98175, 109431; triangle soup at 3840x2160 6371, 6398,
+// 6527, 6562, 6582.  Frames whose levels are all enqueued at once, level 0 only:
+// below 2^20 the walk together is as good or better (soup at 1024x768 1570, 1544,
+// 1548, 1556, 1550; height field 767, 718, 733, 716, 734), and above it the
+// scenes differ (at 1920x1080 200,000-triangle mesh 1983, 1984, 2010, 2026, 2010,
+// soup 2200, 2205, 2158, 2171, 2156, height field 1009, 1014, 958, 959, 956; soup
+// 801x451 at 4 samples 1657, 1649, 1581, 1586, 1586).
+constexpr size_t kFullRaysPerCu = 4096;
 
 // Resident blocks per CU of a kernel at kBlockThreads threads (registers and
 // LDS permitting).
@@ -1265,7 +1272,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
         // short walks have no tail (640x480 sphere frame 580 -> 543 us).  Not
         // batches: their scenes' trees differ, and so do their rays' walks
         // (60 mixed requests 5730 -> 5616 us with level 0 walked together)
-        const bool full = !B && ((n_k >= kFullRays && (k == 0 || !pl.no_sync)) || S0.n_nodes <= kTopNodes);
+        const bool full = !B && ((n_k >= cus * kFullRaysPerCu && (k == 0 || !pl.no_sync)) || S0.n_nodes <= kTopNodes);
         int kt = ktime_begin(A, stream, KT_EXTEND, n_k);
         if (fused && k > 0)
             step(k, true);
