@@ -997,14 +997,17 @@ constexpr int kNoSyncMaxSamples = 1 << 22;
 // Level-0 samples per pass of a frame whose rays branch (see launch_wavefront).
 constexpr int kPassSamples = 1 << 21;
 
-// Longest batch (level-0 samples) whose levels run as k_step: the levels of
-// longer ones fill the GPU by themselves, and their shadow rays gain more from
-// k_occlude's six waves per SIMD than from filling another kernel's tail (us a
-// batch, k_step / side streams: 16 frames of 1080p of one scene, 33 M samples,
-// 24034 / 22511; 4 at 4 samples per pixel, 33 M, 20254 / 19058; the same over
-// three scenes 26227 / 25216; 80 of 512x512 over three scenes, 21 M, 29651 /
-// 29510; 8 of 1080p, 17 M, one scene 12554 / 12250, three 14967 / 15218; 6 over
-// three scenes, 12 M, 11259 / 11770; 4 of one scene, 8 M, 6762 / 6748).
+// Longest batch (level-0 samples) whose levels run as k_step.  The levels of
+// longer ones fill the GPU by themselves: their shadow rays gain more from
+// k_occlude's six waves per SIMD than from filling another kernel's tail, and
+// nothing from a side stream, which only makes the kernels of a captured graph
+// wait for one another.  ms a batch, k_step / two streams / one stream: 256 mixed
+// requests over eight scenes, 25 M samples, 22.5 / 21.9 / 21.5; 16 frames of 1080p
+// of one scene, 33 M, 24.1 / 22.8 / 22.4; 4 at 4 samples per pixel, 33 M, 20.4 /
+// 19.4 / 19.0, the same over three scenes 26.3 / 25.4 / 24.8; 80 of 512x512 over
+// three scenes, 21 M, 29.7 / 29.4 / 28.1.  Below, k_step / two streams: 8 of 1080p,
+// 17 M, one scene 12.6 / 12.3, three 15.0 / 15.2; 6 over three scenes, 12 M, 11.3 /
+// 11.8; 4 of one scene, 8 M, 6.76 / 6.75.
 constexpr int kStepMaxSamples = 1 << 24;
 
 // Levels known to hold this many rays per CU (2^20 on 256 CUs) are walked lane
@@ -1159,19 +1162,21 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     }
     // Batches run a level's rays beside the shadow rays of the level before in
     // one launch (k_step): a captured batch graph put the two streams' kernels
-    // on queues where they waited for one another.  Single frames keep the
-    // side streams (with k_step 64x64 215 -> 227 us, 320x180 3709 -> 3890 us
-    // for three edits, 1080p 1993 -> 2397 us), and so do the FP64 re-test,
-    // which has a kernel of its own, levels sized by read-backs and batches
-    // past kStepMaxSamples.
-    const bool fused = B && pl.no_sync && !retest && shadows && pl.n_samples <= kStepMaxSamples;
+    // on queues where they waited for one another; past kStepMaxSamples they
+    // run on one stream.  Single frames keep the side streams (with k_step
+    // 64x64 215 -> 227 us, 320x180 3709 -> 3890 us for three edits, 1080p 1993
+    // -> 2397 us), and so do the FP64 re-test, which has a kernel of its own,
+    // and levels sized by read-backs.
+    const bool bounded = B && pl.no_sync && !retest && shadows;
+    const bool long_batch = bounded && pl.n_samples > kStepMaxSamples;
+    const bool fused = bounded && !long_batch;
     const bool chain = !pl.slots() && !view;
     // The shadow rays of level k (k_occlude) depend only on
     // k_shade(k), and level k + 1 does not depend on them: with `overlap`
     // they run on the workspace's side stream, concurrently with the next
     // level, and join the render stream before k_combine (the last level's
     // stay on the render stream, see below).
-    const bool ov = overlap && shadows && !fused;
+    const bool ov = overlap && shadows && !fused && !long_batch;
     if (ov) {
         int st = ws.side_init();
         if (st != RTG_OK) return st;

@@ -1,8 +1,9 @@
 """Batches whose levels do not run as one launch each (k_step): those past its
-longest (2^24 samples), those with an FP64 re-test, and those whose queues are
-sized by read-backs.  Their shadow rays run on the side stream beside the next
-level, or with RTG_FLAG_ONE_STREAM on the batch's own: both must give each
-request's frame rendered alone, launched and replayed from a graph."""
+longest (2^24 samples), which run on one stream, those with an FP64 re-test, and
+those whose queues are sized by read-backs.  The shadow rays of these two run on
+the side stream beside the next level, or with RTG_FLAG_ONE_STREAM on the
+batch's own.  All must give each request's frame rendered alone, launched and
+replayed from a graph."""
 from __future__ import annotations
 
 import numpy as np
