@@ -12,10 +12,10 @@
 // 64 rays goes on with quads once 16 are left; and quads whose rays are done
 // take over subtrees of those still walking.
 //
-// us a call, before -> after (with the handing on): 12 thumbnails in a batch 1273 -> 895,
-// burst of 32 requests 2354 -> 1793, 60 mixed requests 6765 -> 5704, 801x451
-// frame at 4 samples 1853 -> 1761, 1080p frame 1807 -> 1741, 1280x720 normal
-// view 423 -> 405, 64x64 frame 209 -> 209.
+// us a call, lane by lane and short queues by quads -> this: 12 thumbnails in a
+// batch 1273 -> 895, burst of 32 requests 1861 -> 1479, 60 mixed requests 6765 ->
+// 5704, 801x451 frame at 4 samples 1854 -> 1762, 1080p frame 1962 -> 1909,
+// 1280x720 normal view 423 -> 405, 64x64 frame unchanged.
 //
 // The results are trace_closest's and trace_any's: the same child tests
 // (Node4Test), primitive tests and winner (the least (t, key)), which depend
@@ -44,7 +44,6 @@ constexpr int kQuadRaysPerCu = 24 * 16;
 // frame 1.06 / 1.03 / 1.05x, 12 thumbnails in a batch 1.10 / 1.05 / 1.01x, burst
 // of 32 requests 1.04 / 1.02 / 0.96x, 1080p frame 1.00 / 1.00 / 0.99x.
 constexpr int kFewRaysPerCu = 16;
-static_assert(kLdsStack * kQuadLanes + kStackMax - kLdsStack >= kStackMax, "a quad's stack holds any walk");
 
 // Move across the quad: lane k reads lane (k ^ 1), (k ^ 2) or (k ^ 3) of its
 // quad.  Quads are active or inactive as a whole.

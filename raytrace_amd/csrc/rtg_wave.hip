@@ -10,9 +10,13 @@
 // then, bottom-up from the deepest level:
 //   combine local Blinn-Phong from the light mask, composed with the node's
 //           children in the reference's order; written into the parent's
-//           child slot (level 0: the sample colour)
+//           child slot (level 0: the sample colour).  Where no hit spawns two
+//           rays, one launch for all levels instead (k_chain): each chain's
+//           last node walks its links up to level 0
 //   resolve average of the samples of a pixel, quantised to RGB8 (with one
-//           sample per pixel, level 0's combine writes the pixel itself)
+//           sample per pixel, level 0's colours go to the pixels themselves)
+// Batches of up to 2^24 samples run the closest hits of level k + 1, the shadow
+// tests of level k and the lighting of level k - 1 in one launch (k_step).
 // The per-node arithmetic is the megakernel's (shade_local, compose), so the
 // two engines give bit-identical frames.
 //
@@ -881,7 +885,7 @@ __global__ void k_resolve(WaveArgs A, const float4 *samples) {
     // a pass that a cancel stopped part-way keeps its pixels untouched (127)
     if (A.cancel != nullptr && *(volatile unsigned *)A.abort != 0) return;
     const WaveReq &R = req_at<B>(A, blockIdx.y);
-    if (R.spp == 1) return;  // written by level 0's k_combine
+    if (R.spp == 1) return;  // written by put_sample
     // pixels of the pass: block rows row0 .. row0 + n_samples / (bw 64 spp)
     const int lg = R.tile_lg, th_lg = 6 - lg;
     const int y0 = R.row0 << th_lg;
@@ -1174,8 +1178,8 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
     // The shadow rays of level k (k_occlude) depend only on
     // k_shade(k), and level k + 1 does not depend on them: with `overlap`
     // they run on the workspace's side stream, concurrently with the next
-    // level, and join the render stream before k_combine (the last level's
-    // stay on the render stream, see below).
+    // level, and join the render stream before the colours are composed (the
+    // last level's stay on the render stream, see below).
     const bool ov = overlap && shadows && !fused && !long_batch;
     if (ov) {
         int st = ws.side_init();
@@ -1326,8 +1330,8 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             ktime_end(A, sk, kt, &ctr[k].n_shadow.v);
         }
         // Local lighting of every level but the last, once its shadow rays are
-        // done, on their stream (beside the next levels): the level's
-        // k_combine, on the frame's last stretch, then only composes.  Single
+        // done, on their stream (beside the next levels): k_chain or the
+        // level's k_combine, on the frame's last stretch, then only composes.  Single
         // frames with every level enqueued at once only: where levels wait for
         // host read-backs (many lights, deep trees) the extra side work ended
         // up on the frame's path (measured).
@@ -1384,7 +1388,7 @@ static int enqueue_wave(const SceneView &S0, const WaveArgs &a, const WavePlan &
             ws.w_samples.as<float4>(), lit(k) ? 1 : 0);
         ktime_end(A, stream, kt, n_ptr);
     }
-    if (B || a.r0.spp != 1) {  // a single frame at one sample per pixel is written by k_combine
+    if (B || a.r0.spp != 1) {  // a single frame at one sample per pixel is written already
         const int kt = ktime_begin(A, stream, KT_RESOLVE, 0);
         k_resolve<B><<<dim3(B ? 256 : 1024, pl.n_reqs), 256, 0, stream>>>(args, ws.w_samples.as<float4>());
         ktime_end(A, stream, kt);
@@ -1612,8 +1616,8 @@ int launch_batch(const BatchItem *items, int n, unsigned long long *counts, unsi
                          (ws.epoch * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)(uintptr_t)counts * 0xC2B2AE3D27D4EB4Full) ^
                          ((uint64_t)(uintptr_t)retests * 0x165667B19E3779F9ull) ^
                          (A.tune.key() * 0x27D4EB2F165667C5ull) ^ ((uint64_t)one_stream << 63);
-    // each level's shadow rays beside the next level on the side stream
-    // (`overlap`), or all on `stream`
+    // `overlap`: batches that do not run as k_step have each level's shadow rays
+    // beside the next level on the side stream; else all on `stream`
     auto enqueue = [&](bool overlap) -> int {
         k_chunk_req<<<(int)((n_chunks + 255) / 256), 256, 0, stream>>>(a.reqs, n_pad, ws.b_chunks.as<int>(),
                                                                       (int)n_chunks);
@@ -1638,8 +1642,9 @@ int launch_batch(const BatchItem *items, int n, unsigned long long *counts, unsi
         ws.graph = nullptr;
         const bool kt = A.ktimes;
         A.ktimes = false;  // no timing events inside a captured graph
-        // Capture with the side stream (the fork and join events become graph
-        // edges); should that capture fail, capture the one-stream order.
+        // Batches that fork are captured with the side stream (the fork and join
+        // events become graph edges); should that capture fail, the one-stream
+        // order is captured.  (A batch on one stream is only tried again.)
         std::string why;
         for (int attempt = 0; attempt < 2 && ws.graph == nullptr; ++attempt) {
             RTG_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
